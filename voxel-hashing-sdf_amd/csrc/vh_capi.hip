@@ -55,15 +55,10 @@ int fail(int code, const std::string& msg) { return set_last_error(code, msg); }
 constexpr int kIntegrateGrid = 5120;
 // Integration workers of the fused batch launch (k_integrate_alloc), whose allocation
 // workgroups are dispatched after the integration ones: fewer workers leave the allocation
-// more of the GPU. room_medium_5mm, integration-only frames/s by worker count (3,072 /
-// 4,096 / 8,192): FP32 63.8k / 62.6k / 59.6k, FP16 63.9k / 63.8k / 62.2k, F16R 51.1k /
-// 52.2k / 51.8k, FP32 + colour 40.6k / 39.6k / 38.9k, F16R + colour 35.4k / 36.5k / 36.0k;
-// FP32 with 2,048 workers 56.4k. Average fused launch after the depth-window and load-order
-// work (2,048 / 3,072 / 4,096 / 5,120 workers): FP32 115.1 / 100.8 / 101.2 / 102.6 us, FP16
-// 124.8 / 106.9 / 105.1 / 106.2, F16R 142.4 / 126.1 / 121.7 / 123.3, FP32 + colour 195.9 /
-// 167.6 / 164.1 / 171.5. Plain FP32 takes 3,072; every costlier voxel update takes 4,096.
-constexpr int kFusedGrid = 3072;
-constexpr int kFusedGridHeavy = 4096;
+// more of the GPU, more share the blocks more evenly. 500 frames of a room at 5 mm, FP32, 2,048 /
+// 3,072 / 4,096 / 5,120 workers: 6.83 / 5.96 / 5.75 / 5.77 ms; F16R + colour, 64 frames: 1.40 /
+// 1.27 / 1.23 / 1.26 ms.
+constexpr int kFusedGrid = 4096;
 constexpr int kGnGrid = 512;  // most workgroups of a solver or backward reduction
 
 // Solver grid for n points: one point per lane, up to kGnGrid workgroups (a partial per
@@ -88,10 +83,9 @@ int integrate_grid() {
   static const int g = grid_setting("VH_INTEGRATE_GRID", kIntegrateGrid);
   return g;
 }
-int fused_grid(int storage, bool color) {
+int fused_grid() {
   static const int g = grid_setting("VH_FUSED_GRID", kFusedGrid);
-  static const int heavy = grid_setting("VH_FUSED_GRID", kFusedGridHeavy);
-  return storage == VH_STORAGE_F32 && !color ? g : heavy;
+  return g;
 }
 
 }  // namespace
@@ -218,6 +212,10 @@ int set_device(vh_volume* v) {
 
 size_t voxel_bytes(int storage) { return storage == VH_STORAGE_F32 ? 8 : 4; }
 
+// Row pitch (pixels) of the images that the allocation writes for the integration: a multiple
+// of 4, so that a row starts at a 16-byte boundary.
+int image_pitch(const vh_config& c) { return (c.width + 3) & ~3; }
+
 FrameArgs frame_args(vh_volume* v, int which) {
   FrameArgs a{};
   const vh_config& c = v->cfg;
@@ -245,6 +243,7 @@ FrameArgs frame_args(vh_volume* v, int which) {
   }
   a.W = c.width;
   a.H = c.height;
+  a.pitch = image_pitch(c);
   a.K = Intr{c.fx, c.fy, c.cx, c.cy};
   a.max_depth = c.max_depth;
   a.min_depth = c.min_depth;
@@ -369,7 +368,7 @@ int enqueue_frame_kernels(vh_volume* v, int which, float staged_scale, int ki, i
   if (fa < 2 || fa >= 6) a.depth_scale = u16 ? staged_scale : 1.0f;
   const bool carve = v->cfg.carve != 0;
   if (which == 2) {
-    VH_HIP(launch_integrate_alloc(a, v->cfg.storage, u16, fused_grid(v->cfg.storage, v->cfg.color != 0), ki, ka, v->stream));
+    VH_HIP(launch_integrate_alloc(a, v->cfg.storage, u16, fused_grid(), ki, ka, v->stream));
     if (carve) VH_HIP(launch_carve(a, ka, v->stream));  // the batch just allocated
     return VH_OK;
   }
@@ -1115,10 +1114,10 @@ int vh_create(const vh_config* cfg, vh_volume** out) {
   // room for four times an even share of the whole pool
   v->stripe_cap = (uint32_t)(cfg->pool_blocks / (kStripes / 4) + 4096);
   const size_t pool = (size_t)cfg->pool_blocks;
-  const size_t frame_px = (size_t)cfg->width * cfg->height;
+  const size_t frame_px = (size_t)cfg->width * cfg->height, image_px = (size_t)image_pitch(*cfg) * cfg->height;
   if ((rc = dev_alloc(&v->keys, v->n_slots * 8)) || (rc = dev_alloc(&v->vals, v->n_slots * 8)) ||
       (rc = dev_alloc(&v->marks, 2 * v->n_slots * 4)) || (rc = dev_alloc(&v->block_keys, pool * 8)) ||
-      (rc = dev_alloc(&v->block_info, pool * 8)) || (rc = dev_alloc(&v->dm, (size_t)2 * kMaxBatch * frame_px * 4)) ||
+      (rc = dev_alloc(&v->block_info, pool * 8)) || (rc = dev_alloc(&v->dm, (size_t)2 * kMaxBatch * image_px * 4 + 64)) ||
       (cfg->carve && (rc = dev_alloc(&v->tilemax, (size_t)2 * kMaxBatch * ((cfg->width + kTile - 1) / kTile) *
                                                      ((cfg->height + kTile - 1) / kTile) * sizeof(float)))) ||
       (rc = dev_alloc(&v->voxels, pool * kB3 * voxel_bytes(cfg->storage))) ||
@@ -1126,7 +1125,7 @@ int vh_create(const vh_config* cfg, vh_volume** out) {
       (rc = dev_alloc(&v->ctl, sizeof(FrameCtl))) ||
       (rc = dev_alloc(&v->stage_depth, frame_px * 4)) || (rc = dev_alloc(&v->stage_pose, 16 * sizeof(float))) ||
       (cfg->color && ((rc = dev_alloc(&v->colors, pool * kB3 * 4)) || (rc = dev_alloc(&v->stage_rgb, frame_px * 3)) ||
-                      (rc = dev_alloc(&v->rgba, 2 * kMaxBatch * frame_px * 4))))) {
+                      (rc = dev_alloc(&v->rgba, 2 * kMaxBatch * image_px * 4))))) {
     std::string msg = g_last_error;
     free_volume(v);
     return fail(rc, msg);

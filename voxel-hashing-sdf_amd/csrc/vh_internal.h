@@ -14,8 +14,9 @@
 //   touched[2][kStripes * stripe_cap] u32 slot ids of the blocks crossed by a batch's bands
 //                                   (each once), in kStripes sub-lists with separate
 //                                   counters, one list per batch parity;
-//   dm[2][8][W*H]                   per batch parity and frame of the batch, each pixel's depth / mu
+//   dm[2][8][pitch*H]               per batch parity and frame of the batch, each pixel's depth / mu
 //                                   (-inf where not a valid measurement), gathered by the integration;
+//                                   rows of pitch = W rounded up to 4 pixels, 64 bytes after the last;
 //   tilemax[2][8][tiles]            carving volumes: per batch parity and frame of the batch, the
 //                                   largest valid depth of each 16 x 16 pixel tile;
 //   ctl                             counters of the frame pipeline (FrameCtl).
@@ -53,27 +54,6 @@ __device__ __forceinline__ float div_rn(float a, float b) {
   const float q0 = a * y;
   float q = __builtin_fmaf(__builtin_fmaf(-b, q0, a), y, q0);
   const bool tiny = __builtin_fabsf(a) < 0x1p-76f && a != 0.0f;
-  if (__builtin_expect(__builtin_amdgcn_ballot_w64(tiny) != 0, 0)) q = tiny ? a / b : q;
-  return q;
-}
-
-// div_rn for dividends that are exact non-negative integers (0 or >= 1; the colour update's
-// c * w + rgb): the quotient by b <= 2^25 is then 0 or at least 2^-25, never subnormal, so
-// the correction alone is exact and there is no fallback test.
-__device__ __forceinline__ float div_rn_int(float a, float b) {
-  const float y = recip_rn(b);
-  const float q0 = a * y;
-  return __builtin_fmaf(__builtin_fmaf(-b, q0, a), y, q0);
-}
-
-// div_rn for dividends that are rarely exactly +0 and never -0 (the TSDF mean's s*w + dist:
-// dist is never -0, and x + y is -0 only when both are): a = +0 takes the fallback, whose
-// quotient +0 is the one the correction gives, so the zero test can go.
-__device__ __forceinline__ float div_rn_rare0(float a, float b) {
-  const float y = recip_rn(b);
-  const float q0 = a * y;
-  float q = __builtin_fmaf(__builtin_fmaf(-b, q0, a), y, q0);
-  const bool tiny = __builtin_fabsf(a) < 0x1p-76f;
   if (__builtin_expect(__builtin_amdgcn_ballot_w64(tiny) != 0, 0)) q = tiny ? a / b : q;
   return q;
 }
@@ -124,6 +104,7 @@ struct FrameArgs {
   float depth_scale;
   // camera and volume parameters
   int32_t W, H;
+  int32_t pitch;   // row pitch of dm and rgba in pixels: W rounded up to a multiple of 4
   Intr K;
   BandScale band;  // reciprocals for the band setup
   float max_depth, min_depth, vox, bsz, mu, inv_mu;
@@ -144,11 +125,11 @@ struct FrameArgs {
   const uint8_t* rgb;
   uint32_t* colors;
   // colour volumes: the allocation pass packs each pixel of frame j of a batch into one word
-  // {r | g << 8 | b << 16} at rgba + (parity * kMaxBatch + j) * W*H, which the integration
+  // {r | g << 8 | b << 16} at rgba + (parity * kMaxBatch + j) * pitch*H, which the integration
   // of the batch gathers
   uint32_t* rgba;
   // the allocation pass writes each pixel of frame j of a batch as scaled_depth (depth / mu,
-  // -inf where not valid) to dm + (parity * kMaxBatch + j) * W*H; the integration gathers it
+  // -inf where not valid) to dm + (parity * kMaxBatch + j) * pitch*H; the integration gathers it
   float* dm;
   // carving volumes (null otherwise): the allocation pass writes the largest valid depth of each
   // kTile x kTile pixel tile of frame j of a batch to tilemax + (parity * kMaxBatch + j) *

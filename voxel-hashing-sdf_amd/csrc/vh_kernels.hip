@@ -237,7 +237,7 @@ __device__ void alloc_tile(const FrameArgs& a, uint32_t tile, uint32_t frame, ui
   for (int r = 0; r < kRows; ++r) {
     const int v = v0 + 16 * r;
     if (u < a.W && v < a.H) {
-      const size_t staged = ((size_t)parity * kMaxBatch + jb) * a.W * a.H + (size_t)v * a.W + u;
+      const size_t staged = (((size_t)parity * kMaxBatch + jb) * a.H + v) * a.pitch + u;
       // the pixel's colour, packed for the integration's one-word gathers
       if constexpr (kColor) a.rgba[staged] = px3[r][0] | px3[r][1] << 8 | px3[r][2] << 16;
       // the pre-scaled depth the integration of this frame gathers
@@ -337,16 +337,16 @@ __device__ __forceinline__ void mean_update(float& s, float& w, float dist, floa
 }
 
 // Colour update of the reference (src/tsdf.cu:743-745): per channel (c * w_old + rgb) / w_new
-// in FP32 (the product and sum are exact integers below 2^24; the quotient correctly
-// rounded by div_rn), truncated to 8 bits. w_old is the stored weight before this update;
-// c and px are packed {r | g << 8 | b << 16}.
-__device__ __forceinline__ uint32_t color_update(uint32_t c, float w_old, uint32_t px) {
-  const float w_new = w_old + 1.0f;
+// in FP32 (the product and sum are exact integers below 2^24; the quotient correctly rounded
+// as in div_rn), truncated to 8 bits. w_old is the stored weight before this update, w_new
+// = w_old + 1 and y = RN(1/w_new); c and px are packed {r | g << 8 | b << 16}.
+__device__ __forceinline__ uint32_t color_update(uint32_t c, float w_old, float w_new, float y, uint32_t px) {
   uint32_t out = 0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const float num = __builtin_fmaf((float)((c >> (8 * k)) & 255u), w_old, (float)((px >> (8 * k)) & 255u));
-    out |= (uint32_t)(uint8_t)div_rn_int(num, w_new) << (8 * k);
+    const float q0 = num * y;
+    out |= (uint32_t)(uint8_t)__builtin_fmaf(__builtin_fmaf(-w_new, q0, num), y, q0) << (8 * k);
   }
   return out;
 }
@@ -366,76 +366,77 @@ constexpr int kPlaceEdge = 0;    // some voxel may project outside the image: pe
 constexpr int kPlaceInside = 1;  // every voxel inside: no checks, depth gathered from the image
 constexpr int kPlaceWindow = 2;  // every voxel inside, its pixels in a window staged in LDS
 // LDS window per wave (pixels): the pre-scaled depth of the pixel rectangle that a block's
-// voxels project into, rows of a power-of-two pitch <= 64. A 5 mm block at 2 m covers about
+// voxels project into, rows of a power-of-two pitch of 4 to 64. A 5 mm block at 2 m covers about
 // 12 x 12 pixels; at 0.5 m about 50 x 50, which does not fit and is gathered from the image.
 constexpr uint32_t kWin = 512;
 
-// A block's window in a frame: the image rectangle of columns ulo .. ulo + cols - 1 and rows
-// vlo .. vlo + rows - 1 (both inside the image), in LDS at pitch 2^shift.
+// A block's window in a frame: the image rectangle of columns ulo .. ulo + cols - 1 (ulo a
+// multiple of 4) and rows vlo .. vlo + rows - 1, in LDS at pitch 2^shift.
 struct DepthWindow {
-  uint32_t first;  // byte offset 4 (vlo W + ulo) of the rectangle's first pixel in the image
-  uint32_t shift;  // log2 of the LDS row pitch in pixels, <= 6
+  uint32_t first;  // byte offset 4 (vlo pitch + ulo) of the rectangle's first pixel in the image
+  uint32_t shift;  // log2 of the LDS row pitch in pixels, 2 .. 6
   uint32_t rows, cols;
   uint32_t bias;   // LDS byte offset of pixel (u, v) = (bits(M + v) << (shift + 2)) + (bits(M + u) << 2) - bias
 };
 
-// Smallest and largest of x over lanes 0, 7, 56 and 63, the lanes whose columns end at the
-// block's 8 corners: the half-row mirror (DPP) pairs lane 0 with 7 and 56 with 63, then two
-// reads of lanes 0 and 56.
-__device__ __forceinline__ uint32_t half_mirror(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x141, 0xf, 0xf, false);
+// Smallest and largest of x over the 8 lanes of an aligned group (DPP: the quad's pairs, the
+// quad's halves, the half-row mirror).
+template <int kCtrl>
+__device__ __forceinline__ int32_t dpp(int32_t x) { return __builtin_amdgcn_mov_dpp(x, kCtrl, 0xf, 0xf, false); }
+__device__ __forceinline__ int32_t oct_min(int32_t x) {
+  x = min(x, dpp<0xB1>(x));
+  x = min(x, dpp<0x4E>(x));
+  return min(x, dpp<0x141>(x));
 }
-__device__ __forceinline__ int32_t corner_min(int32_t x) {
-  x = min(x, (int32_t)half_mirror((uint32_t)x));
-  return min(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 56));
-}
-__device__ __forceinline__ int32_t corner_max(int32_t x) {
-  x = max(x, (int32_t)half_mirror((uint32_t)x));
-  return max(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 56));
+__device__ __forceinline__ int32_t oct_max(int32_t x) {
+  x = max(x, dpp<0xB1>(x));
+  x = max(x, dpp<0x4E>(x));
+  return max(x, dpp<0x141>(x));
 }
 
-// Placement of a block in a frame (wave-uniform). The lane's column runs from voxel 0 to
-// voxel 7 of cl + q*ax (homogeneous coordinates); the block's lattice box is the convex hull
-// of its 8 corners, the column end points of lanes 0, 7, 56 and 63. For depths > 0 the
-// perspective image of a convex combination is a convex combination of the images, and a
-// voxel's own projection differs from the exact one, as the corners' do, by far less than
-// 1/2 pixel. So if every end point has z in [2^-60, 2^60], every voxel's z lies in
-// [2^-64, 2^64], and with umin, umax the least and largest u = X/z of the corners a voxel's
-// pixel round(u) lies in [round(umin - 1/2), round(umax + 1/2)] (for errors below 1/2 these
-// roundings cannot cross the voxel's); likewise v. That rectangle is the block's window.
-// kPlaceEdge unless the window lies inside the image; then kPlaceWindow when it fits kWin at a
-// pitch of at most 64 pixels, else kPlaceInside. The bounds are the bits of (u -+ 1/2) + M as
+// Placement of a block in up to 8 frames at once: lanes 8 j .. 8 j + 7 hold the block's 8
+// corners in frame j (hb: the frame's homogeneous block origin, off: the corner's homogeneous
+// offset), so one pass over the lanes places the block in every frame of the batch (a pass per
+// frame spent about 75 vector instructions on wave-uniform values in each). The block's lattice
+// box is the convex hull of its corners. For depths > 0 the perspective image of a convex
+// combination is a convex combination of the images, and a voxel's own projection differs from
+// the exact one, as the corners' do, by far less than 1/2 pixel. So if every corner has z in
+// [2^-60, 2^60], every voxel's z lies in [2^-64, 2^64], and with umin, umax the least and
+// largest u = X/z of the corners a voxel's pixel round(u) lies in [round(umin - 1/2),
+// round(umax + 1/2)] (for errors below 1/2 these roundings cannot cross the voxel's); likewise
+// v. That rectangle, its left edge moved down to a multiple of 4 pixels, is the block's window.
+// kPlaceEdge unless the rectangle lies inside the image; then kPlaceWindow when it fits kWin at
+// a pitch of at most 64 pixels, else kPlaceInside. The bounds are the bits of (u -+ 1/2) + M as
 // signed integers: for positive sums below 2^24 they are M's plus the rounded bound, larger
-// sums exceed every image bound and negative ones lie below them.
-__device__ __forceinline__ int block_place(const FrameArgs& a, const float ax[3], const float cl[3], DepthWindow& w) {
-  bool zin = true;
-  float u[2], v[2];
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {  // voxel 0 of the column is cl itself
-    const float z = e ? __builtin_fmaf(7.0f, ax[2], cl[2]) : cl[2];
-    const float iz = recip_rn(z);
-    u[e] = (e ? __builtin_fmaf(7.0f, ax[0], cl[0]) : cl[0]) * iz;
-    v[e] = (e ? __builtin_fmaf(7.0f, ax[1], cl[1]) : cl[1]) * iz;
-    zin = zin & (z >= 0x1p-60f) & (z <= 0x1p60f);
-  }
-  // computed whatever the placement, so that the window stays in scalar registers
-  const int32_t lu = corner_min((int32_t)__float_as_uint((fminf(u[0], u[1]) - 0.5f) + kPixMagic));
-  const int32_t hu = corner_max((int32_t)__float_as_uint((fmaxf(u[0], u[1]) + 0.5f) + kPixMagic));
-  const int32_t lv = corner_min((int32_t)__float_as_uint((fminf(v[0], v[1]) - 0.5f) + kPixMagic));
-  const int32_t hv = corner_max((int32_t)__float_as_uint((fmaxf(v[0], v[1]) + 0.5f) + kPixMagic));
-  const uint32_t cols = (uint32_t)(hu - lu) + 1u, rows = (uint32_t)(hv - lv) + 1u;
-  // pitch: the power of two >= cols (2 for one column), at most 64
-  const uint32_t shift = 32u - (uint32_t)__builtin_clz(min(cols - 1u, 63u) | 1u);
-  w.first = 4u * (((uint32_t)lv - kPixMagicBits) * (uint32_t)a.W + ((uint32_t)lu - kPixMagicBits));
-  w.shift = shift;
-  w.rows = rows;
-  w.cols = cols;
-  w.bias = ((uint32_t)lv << (shift + 2u)) + ((uint32_t)lu << 2);
+// sums (and NaN) exceed every image bound and negative ones lie below them.
+struct Placement {
+  uint32_t first, bias;  // DepthWindow's
+  uint32_t desc;         // placement | shift << 2 | cols << 5 | rows << 12
+};
+__device__ __forceinline__ Placement block_place(const FrameArgs& a, const float hb[3], const float off[3]) {
+  const float z = hb[2] + off[2];
+  const float iz = __builtin_amdgcn_rcpf(z);  // within 1 ulp: the bounds leave 1/2 pixel
+  const float u = (hb[0] + off[0]) * iz, v = (hb[1] + off[1]) * iz;
+  const uint64_t zin = __builtin_amdgcn_ballot_w64((z >= 0x1p-60f) & (z <= 0x1p60f));
+  const int32_t lu = oct_min((int32_t)__float_as_uint((u - 0.5f) + kPixMagic));
+  const int32_t hu = oct_max((int32_t)__float_as_uint((u + 0.5f) + kPixMagic));
+  const int32_t lv = oct_min((int32_t)__float_as_uint((v - 0.5f) + kPixMagic));
+  const int32_t hv = oct_max((int32_t)__float_as_uint((v + 0.5f) + kPixMagic));
   const int32_t mb = (int32_t)kPixMagicBits;
-  const bool inside = __builtin_amdgcn_ballot_w64(!zin) == 0 && lu >= mb && hu <= mb + a.W - 1 && lv >= mb &&
+  const uint32_t lane = threadIdx.x & 63u;
+  const bool inside = ((zin >> (lane & 56u)) & 255u) == 255u && lu >= mb && hu <= mb + a.W - 1 && lv >= mb &&
                       hv <= mb + a.H - 1;
+  const int32_t la = lu & ~3;  // M's bits are a multiple of 4
+  const uint32_t cols = (uint32_t)(hu - la) + 1u, rows = (uint32_t)(hv - lv) + 1u;
+  // pitch: the power of two >= cols, at least 4 and at most 64
+  const uint32_t shift = 32u - (uint32_t)__builtin_clz(min(cols - 1u, 63u) | 3u);
   const bool fits = cols <= 64u && rows <= (kWin >> shift);
-  return inside ? (fits ? kPlaceWindow : kPlaceInside) : kPlaceEdge;
+  Placement p;
+  p.first = 4u * (((uint32_t)lv - kPixMagicBits) * (uint32_t)a.pitch + ((uint32_t)la - kPixMagicBits));
+  p.bias = ((uint32_t)lv << (shift + 2u)) + ((uint32_t)la << 2);
+  p.desc = inside ? (fits ? (uint32_t)kPlaceWindow | shift << 2 | cols << 5 | rows << 12 : (uint32_t)kPlaceInside)
+                  : (uint32_t)kPlaceEdge;
+  return p;
 }
 
 // LDS addresses as integers: the byte address of an LDS location, and a read from one.
@@ -444,55 +445,99 @@ __device__ __forceinline__ uint32_t lds_address(const float* p) { return (uint32
 __device__ __forceinline__ float lds_read(uint32_t byte_address) { return *(const LdsFloat*)(size_t)byte_address; }
 
 // The window's pixels of pre-scaled depth image dmf into the wave's LDS window at byte address
-// win (row r at win + 4 (r << shift)), by loads that write LDS directly: load t covers rows
-// t * 64 >> shift onwards, lane l column l mod 2^shift of row l >> shift, and writes word
-// 64 t + l. The loads use no registers, so the caller computes its pixels while they are in
-// flight and waits for them (window_ready) before its first read.
+// win (row r at win + 4 (r << shift)), by 16-byte loads that write LDS directly: load t covers
+// rows t * 256 >> shift onwards, lane l the four pixels from column 4 (l mod 2^(shift - 2)) of row
+// l >> (shift - 2), and writes words 256 t + 4 l onwards. Image rows and the window's left edge
+// are multiples of 4 pixels, so every access is 16-byte aligned; the last load of a row may read
+// up to 3 pixels past the rectangle (the images are followed by 64 bytes). A typical window of
+// 12 x 12 pixels is one load (three with 4-byte loads). The loads use no registers, so the caller
+// computes its pixels while they are in flight and waits for them (window_ready) before its first
+// read.
 __device__ __forceinline__ void stage_window(const FrameArgs& a, const float* dmf, const DepthWindow& w, uint32_t win) {
-  const uint32_t lane = threadIdx.x & 63u, w4 = 4u * (uint32_t)a.W;
-  const uint32_t row = lane >> w.shift, col = lane & ((1u << w.shift) - 1u), step = 64u >> w.shift;
+  const uint32_t lane = threadIdx.x & 63u, w4 = 4u * (uint32_t)a.pitch, per = w.shift - 2u;
+  const uint32_t row = lane >> per, col = 4u * (lane & ((1u << per) - 1u)), step = 64u >> per;
   const char* src = reinterpret_cast<const char*>(dmf) + w.first;
-  const uint32_t off = row * w4 + 4u * col;
-  const int left = col < w.cols && row < w.rows ? (int)(w.rows - row) : 0;  // rows the lane loads, at most
-  const uint32_t n_it = (w.rows + step - 1u) >> (6u - w.shift);             // loads of the widest lane
+  const uint32_t off = __umul24(row, w4) + 4u * col;  // both below 2^24
+  const int left = col < w.cols ? (int)(w.rows - row) : 0;  // rows from the lane's own to the window's end
+  const uint32_t n_it = (w.rows + step - 1u) >> (6u - per);
   for (uint32_t t = 0; t < n_it; ++t) {
     const char* rows_t = src + t * step * w4;  // uniform
     if ((int)(t * step) < left)
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(rows_t + off),
-                                       (__attribute__((address_space(3))) void*)(size_t)(win + 256u * t), 4, 0, 0);
+                                       (__attribute__((address_space(3))) void*)(size_t)(win + 1024u * t), 16, 0, 0);
   }
 }
 // Wait for the window's loads (vmcnt 0; the compiler does not order a read through an integer
 // LDS address after them by itself).
 __device__ __forceinline__ void window_ready() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 
+// The 8 voxels of a lane between a block's load and its store. kReg (launches of several frames
+// with the reciprocal table, storage FP32 or FP16): the value s as the storage rounds it and the
+// weight as the byte offset t = 4 w of RN(1/w) in the table, so a frame's update reads the
+// table at t + 4 with no conversion, and an unobserved voxel reads the table's entry 0, which is
+// 0: its value is then s + 0 * (-1 - s) = s bit for bit, with no selects (|s| <= 1). The two
+// conversions each way per voxel are paid once per block. Otherwise the storage word itself
+// (F16R's word is not a function of its value: the residual of a tie has two forms).
+template <int kStorage, bool kReg>
+struct LaneVoxels {
+  using IO = VoxelIO<kStorage>;
+  using Word = typename IO::Word;
+  Word w[8];
+  __device__ __forceinline__ void load(int q, Word x) { w[q] = x; }
+  __device__ __forceinline__ Word word(int q) const { return w[q]; }
+};
+template <>
+struct LaneVoxels<VH_STORAGE_F32, true> {
+  using Word = float2;
+  float s[8];
+  uint32_t t[8];
+  __device__ __forceinline__ void load(int q, Word x) { s[q] = x.x; t[q] = (uint32_t)(x.y * 4.0f); }
+  __device__ __forceinline__ Word word(int q) const { return make_float2(s[q], (float)t[q] * 0.25f); }
+  __device__ __forceinline__ void set(int q, float v) { s[q] = v; }
+};
+template <>
+struct LaneVoxels<VH_STORAGE_F16, true> {
+  using Word = uint32_t;
+  float s[8];
+  uint32_t t[8];
+  __device__ __forceinline__ void load(int q, Word x) {
+    s[q] = (float)__builtin_bit_cast(_Float16, (uint16_t)(x & 0xffffu));
+    t[q] = (x >> 16) << 2;
+  }
+  __device__ __forceinline__ Word word(int q) const {
+    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)s[q]) | t[q] << 14;  // s[q] is a binary16 value
+  }
+  __device__ __forceinline__ void set(int q, float v) {
+    s[q] = (float)__builtin_bit_cast(_Float16, f32_to_f16_rn(v));
+  }
+};
+
 // One frame's update of the lane's 8 voxels of a block (homogeneous column cl, step ax): per
 // half, all projections, then all pre-scaled depth (and colour) fetches, then the updates, so
-// the fetches are in flight together. Branch-free: every lane computes, the observation flag
-// selects. dmf: the frame's pre-scaled depth image (scaled_depth of each pixel).
-// kPlace (block_place's result): kPlaceInside and kPlaceWindow leave out the range checks,
-// which are known to pass (the values computed are the same); kPlaceWindow reads the depth
-// from the window that stage_window is loading (pitch 2^wshift; wbase: the LDS byte address of
-// pixel (u, v) is (bits(M + v) << (wshift + 2)) + (bits(M + u) << 2) + wbase modulo 2^32, the
-// window's address minus DepthWindow::bias). (Issuing the next frame's gathers before
-// this frame's updates, with two register sets, was slower: 92 against 86 us per FP32 batch
-// launch.)
-template <int kStorage, bool kColor, int kPlace, bool kTab>
-__device__ __forceinline__ void frame_update(const FrameArgs& a, const float ax[3], const float cl[3],
+// the fetches are in flight together. Branch-free per lane: every lane computes, the observation
+// flag selects. dmf: the frame's pre-scaled depth image (scaled_depth of each pixel).
+// place (block_place's result, wave-uniform) chooses how a half's depths are fetched; the
+// projection and the update around it are common, so the voxels stay in their registers (a
+// variant of the whole update per placement cost 16 register copies per frame where the
+// variants join). kPlaceInside and kPlaceWindow leave out the range checks, which are known to
+// pass; kPlaceWindow reads the depth from the window that stage_window is loading (pitch
+// 2^wshift; wbase: the LDS byte address of pixel (u, v) is (bits(M + v) << (wshift + 2)) +
+// (bits(M + u) << 2) + wbase modulo 2^32, the window's address minus DepthWindow::bias). A voxel
+// outside the image gets depth -inf, which no update follows. (Issuing the next frame's gathers
+// before this frame's updates, with two register sets, was slower: 92 against 86 us per FP32
+// batch launch.)
+template <int kStorage, bool kColor, bool kTab, bool kReg>
+__device__ __forceinline__ void frame_update(const FrameArgs& a, uint32_t place, const float ax[3], const float cl[3],
                                              const float* dmf, const uint32_t* rgba, uint32_t wshift,
-                                             uint32_t wbase, typename VoxelIO<kStorage>::Word old[8],
+                                             uint32_t wbase, uint32_t t_cap, LaneVoxels<kStorage, kReg>& vx,
                                              uint32_t cold[8], uint32_t& upd, const float* rcp_tab) {
   using IO = VoxelIO<kStorage>;
   using Word = typename IO::Word;
-  constexpr bool kInside = kPlace != kPlaceEdge, kWindow = kPlace == kPlaceWindow;
-  const uint32_t w4 = (4u * (uint32_t)a.W) & 0xffffffu, bias = pix_bias(a.W);
+  const uint32_t w4 = (4u * (uint32_t)a.pitch) & 0xffffffu, bias = pix_bias(a.pitch);
   // two halves of 4 voxels: fewer values live at once (occupancy) for 4 fetches in flight
 #pragma unroll
   for (int h = 0; h < 8; h += 4) {
-    float zc[4];
-    int pix[4];
-    uint32_t off[4];   // kInside: byte offset of the pixel in the depth (and RGB) image, off a scalar base
-    uint32_t loff[4];  // kWindow: byte offset of the pixel in the LDS window
+    float zc[4], uf[4], vf[4];  // camera depth; M + column, M + row of the pixel
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float fq = (float)(h + r);  // voxel 0 is the column itself (fma(0, a, c) = c but for -0)
@@ -500,90 +545,119 @@ __device__ __forceinline__ void frame_update(const FrameArgs& a, const float ax[
       const float Y = h + r ? __builtin_fmaf(fq, ax[1], cl[1]) : cl[1];
       zc[r] = h + r ? __builtin_fmaf(fq, ax[2], cl[2]) : cl[2];
       const float iz = recip_rn(zc[r]);
-      if constexpr (kInside) {
-        const uint32_t ub = __float_as_uint(__builtin_fmaf(X, iz, kPixMagic));
-        const uint32_t vb = __float_as_uint(__builtin_fmaf(Y, iz, kPixMagic));
-        if constexpr (kWindow) {
-          loff[r] = (((vb << wshift) + ub) << 2) + wbase;
-          if constexpr (kColor) off[r] = (vb & 0xffffffu) * w4 + ((ub << 2) - bias);
-        } else {
-          off[r] = (vb & 0xffffffu) * w4 + ((ub << 2) - bias);
-        }
-      } else {
-        pix[r] = pixel_of(X, Y, zc[r], iz, a.W, a.H);
-      }
+      uf[r] = __builtin_fmaf(X, iz, kPixMagic);
+      vf[r] = __builtin_fmaf(Y, iz, kPixMagic);
     }
     float dv[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      if constexpr (kWindow) {
-        if (h == 0 && r == 0) window_ready();  // the pixels are computed: now wait for the window
-        dv[r] = lds_read(loff[r]);
-      }
-      else if constexpr (kInside) dv[r] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(dmf) + off[r]);
-      else dv[r] = dmf[max(pix[r], 0)];
-    }
     uint32_t px[4];
-    if constexpr (kColor) {
+    if (place == (uint32_t)kPlaceWindow) {
+      uint32_t loff[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        if constexpr (kInside) px[r] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(rgba) + off[r]);
-        else px[r] = rgba[max(pix[r], 0)];
+        const uint32_t ub = __float_as_uint(uf[r]), vb = __float_as_uint(vf[r]);
+        loff[r] = (((vb << wshift) + ub) << 2) + wbase;
+        if constexpr (kColor)
+          px[r] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(rgba) +
+                                                     ((vb & 0xffffffu) * w4 + ((ub << 2) - bias)));
       }
+      if (h == 0) window_ready();  // the pixels are computed: now wait for the window
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dv[r] = lds_read(loff[r]);
+    } else if (place == (uint32_t)kPlaceInside) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t ub = __float_as_uint(uf[r]), vb = __float_as_uint(vf[r]);
+        const uint32_t off = (vb & 0xffffffu) * w4 + ((ub << 2) - bias);
+        dv[r] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(dmf) + off);
+        if constexpr (kColor) px[r] = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(rgba) + off);
+      }
+    } else {
+      int pix[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        pix[r] = pixel_of(uf[r], vf[r], zc[r], a.W, a.H, a.pitch);
+        dv[r] = dmf[max(pix[r], 0)];
+        if constexpr (kColor) px[r] = rgba[max(pix[r], 0)];
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) dv[r] = pix[r] >= 0 ? dv[r] : -INFINITY;
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int q = h + r;
       const float t = __builtin_fmaf(-zc[r], a.inv_mu, dv[r]);
-      const bool ok = (kInside || pix[r] >= 0) & (t > -1.0f);
-      const float dist = fminf(1.0f, t);
-      float sv, wv;
-      IO::unpack(old[q], sv, wv);
-      if constexpr (kColor) {
-        const uint32_t c = color_update(cold[q], wv, px[r]);
-        cold[q] = ok ? c : cold[q];
+      const bool ok = t > -1.0f;
+      if constexpr (kReg) {
+        const float dist = __builtin_amdgcn_fmed3f(t, -1.0f, 1.0f);  // min(1, t) where observed, -1 elsewhere
+        const uint32_t tn = ok ? vx.t[q] + 4u : 0u;
+        const float y = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(rcp_tab) + tn);
+        if constexpr (kColor) {
+          const float w_old = (float)vx.t[q] * 0.25f;
+          const uint32_t c = color_update(cold[q], w_old, w_old + 1.0f, y, px[r]);
+          cold[q] = ok ? c : cold[q];
+          upd |= (uint32_t)ok << q;
+        }
+        vx.set(q, __builtin_fmaf(dist - vx.s[q], y, vx.s[q]));
+        vx.t[q] = min(max(vx.t[q], tn), t_cap);
+      } else {
+        const float dist = fminf(1.0f, t);
+        float sv, wv;
+        IO::unpack(vx.w[q], sv, wv);
+        if constexpr (kColor) {
+          const uint32_t c = color_update(cold[q], wv, wv + 1.0f, recip_rn(wv + 1.0f), px[r]);
+          cold[q] = ok ? c : cold[q];
+          upd |= (uint32_t)ok << q;
+        }
+        mean_update<kTab>(sv, wv, dist, a.cap, rcp_tab);
+        const Word nw = IO::pack(sv, wv);
+        vx.w[q] = ok ? nw : vx.w[q];
       }
-      mean_update<kTab>(sv, wv, dist, a.cap, rcp_tab);
-      const Word nw = IO::pack(sv, wv);
-      old[q] = ok ? nw : old[q];
-      if constexpr (kColor) upd |= (uint32_t)ok << q;
     }
     __builtin_amdgcn_sched_barrier(0);  // keep the halves apart: the scheduler would merge them
   }
 }
 
 // Per frame of a batch, staged in LDS by stage_frames: the pose (row-major 3x4) and the
-// frame's homogeneous voxel steps (block_frame_h).
-struct FrameLds {
+// frame's homogeneous voxel steps (block_frame_h), each padded to 16 bytes.
+struct __align__(16) FrameLds {
   float T[12];
-  BlockFrame h;
+  float ax[4], ay[4], az[4];
+};
+// Per frame and lane: the column's homogeneous offset from the block origin, the
+// same for every block.
+struct __align__(16) ColumnLds {
+  float off[64][4];
 };
 
-// s_frm: the batch's k frames; rcp_tab: RN(1/w) for w < kRcpTab (read when kTab); s_win: the
-// LDS byte address of the wave's depth window (kWin pixels). kShared: the block origin of
-// each frame is computed once per block (launches of several frames), else in the frame loop.
-template <int kStorage, bool kColor, bool kTab, bool kShared>
-__device__ void integrate_worker(const FrameArgs& a, uint32_t worker, uint32_t workers, uint32_t f0, uint32_t k,
-                                 uint32_t parity, unsigned long long* s_val, unsigned long long* s_key,
-                                 uint32_t* s_mark, const FrameLds* s_frm, const float* rcp_tab, uint32_t s_win) {
+// my_off, n: lane s holds the exclusive offset of the list's stripe s; the list's length. s_frm,
+// s_col: the batch's k frames; rcp_tab: RN(1/w) for w < kRcpTab with 0 at w = 0 (read when
+// kTab); s_win: the LDS byte address of the wave's depth window (kWin pixels). kBatch: a launch of
+// several frames (k > 1).
+template <int kStorage, bool kColor, bool kTab, bool kBatch>
+__device__ void integrate_worker(const FrameArgs& a, uint32_t worker, uint32_t workers, uint32_t my_off, uint32_t n,
+                                 uint32_t f0, uint32_t k, uint32_t parity, unsigned long long* s_val,
+                                 unsigned long long* s_key, uint32_t* s_mark, const FrameLds* s_frm,
+                                 const ColumnLds* s_col, const float* rcp_tab, uint32_t s_win) {
   using IO = VoxelIO<kStorage>;
   using Word = typename IO::Word;
+  constexpr bool kReg = kTab && kBatch && kStorage != VH_STORAGE_F16R;
   FrameCtl* ctl = a.ctl;
   const int lane = threadIdx.x & 63;
-  const uint32_t* lcount = list_count_of(ctl, parity);
   const uint32_t* list = list_of(a, parity);
   uint32_t* marks = marks_of(a, parity);
-  // lane s holds stripe s's length and exclusive offset
-  const uint32_t my_len = min(lcount[lane * kLine], a.stripe_cap);
-  uint32_t incl = my_len;
+  const size_t frame_px = (size_t)a.pitch * a.H;
+  const uint32_t t_cap = a.cap < (float)kRcpTab ? 4u * (uint32_t)a.cap : ~0u;
+
+  // lanes 8 j .. 8 j + 7: the 8 corners of a block in frame j of the batch (a single frame: all
+  // groups the same), as homogeneous offsets from its origin
+  const uint32_t jl = kBatch ? min((uint32_t)lane >> 3, k - 1u) : 0u;
+  float corner[3];
+  {
+    const float c0 = (lane & 1) ? 7.0f : 0.0f, c1 = (lane & 2) ? 7.0f : 0.0f, c2 = (lane & 4) ? 7.0f : 0.0f;
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t y = (uint32_t)__shfl_up((int)incl, off);
-    if (lane >= off) incl += y;
+    for (int r = 0; r < 3; ++r)
+      corner[r] = __builtin_fmaf(c0, s_frm[jl].ax[r], __builtin_fmaf(c1, s_frm[jl].ay[r], c2 * s_frm[jl].az[r]));
   }
-  const uint32_t my_off = incl - my_len;
-  const uint32_t n = read_lane_u32(incl, 63);
-  const size_t frame_px = (size_t)a.W * a.H;
 
   // Lane j fetches the list entry, slot value, key and mark of this worker's j-th block
   // (clearing the mark for the next batch of this parity) and parks them in LDS, so the
@@ -618,9 +692,9 @@ __device__ void integrate_worker(const FrameArgs& a, uint32_t worker, uint32_t w
     __builtin_amdgcn_wave_barrier();  // one wave owns this slice: it only needs its own writes
     const uint32_t nj = min(64u, (n - t0 + workers - 1) / workers);
     for (uint32_t j = 0; j < nj; ++j) {
-      const unsigned long long val = s_val[j];
-      const unsigned long long keyj = s_key[j];
-      const uint32_t mark = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_mark[j]) & ((1u << k) - 1u);
+      const unsigned long long val = uniform64(s_val[j]);
+      const unsigned long long keyj = uniform64(s_key[j]);
+      const uint32_t mark = uniform(s_mark[j]) & ((1u << k) - 1u);
       const uint32_t idx = (uint32_t)val;
       if (idx >= a.pool_cap) {
         if (lane == 0) raise_flag(ctl, kFlagPoolFull);
@@ -629,75 +703,77 @@ __device__ void integrate_worker(const FrameArgs& a, uint32_t worker, uint32_t w
       const bool fresh = (uint32_t)(val >> 32) - f0 < k;  // born in this batch: starts at zero
       int bx, by, bz;
       unpack_key(keyj, bx, by, bz);
-      Word* vp = reinterpret_cast<Word*>(a.voxels) + (size_t)idx * kB3 + lane;
-      Word old[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) old[q] = fresh ? IO::zero() : vp[64 * q];
-      uint32_t* cp = kColor ? a.colors + (size_t)idx * kB3 + lane : nullptr;
+      Word* vp = reinterpret_cast<Word*>(a.voxels) + (size_t)idx * kB3;
+      uint32_t* cp = kColor ? a.colors + (size_t)idx * kB3 : nullptr;
+      LaneVoxels<kStorage, kReg> vx;
       uint32_t cold[8];
-      if constexpr (kColor) {
+      {
+        Word old[8];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) cold[q] = fresh ? 0u : cp[64 * q];
-      }
-      uint32_t upd = 0u;  // colour volumes: bit q set when voxel q was observed in the batch
-      // the block origin in homogeneous pixel coordinates per frame of the batch: with kShared
-      // lane j < k computes frame j's and the frame loop takes it with readlane, so these
-      // wave-uniform values are computed once per block rather than by every lane in every
-      // frame (a single-frame launch would only add the readlanes, and computes it inline)
-      float hbl[3] = {0.0f, 0.0f, 0.0f};
-      if (kShared && (uint32_t)lane < k) {
-        float T[12], cb[3];
+        for (int q = 0; q < 8; ++q) old[q] = fresh ? IO::zero() : vp[lane + 64 * q];
+        if constexpr (kColor) {
 #pragma unroll
-        for (int q = 0; q < 12; ++q) T[q] = s_frm[lane].T[q];
-        block_origin_cam(T, a.vox, bx, by, bz, cb);
-        to_pixel_h(a.K, cb, hbl);
-      }
-      for (uint32_t m = mark; m != 0u; m &= m - 1u) {
-        const uint32_t jf = (uint32_t)__builtin_ctz(m);
-        const FrameLds& F = s_frm[jf];
-        const BlockFrame hf = F.h;
-        float hb[3], cl[3];
-        if constexpr (kShared) {
-#pragma unroll
-          for (int r = 0; r < 3; ++r)
-            hb[r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hbl[r]), (int)jf));
-        } else {
+          for (int q = 0; q < 8; ++q) cold[q] = fresh ? 0u : cp[lane + 64 * q];
+        }
+        // the block's placement in every frame of the batch, while its voxels are on their way
+        // (lane group j holds frame j's; the frame loop takes it with readlane)
+        float hb[3];
+        Placement pl;
+        {
           float T[12], cb[3];
 #pragma unroll
-          for (int q = 0; q < 12; ++q) T[q] = F.T[q];
+          for (int q = 0; q < 12; ++q) T[q] = s_frm[jl].T[q];
           block_origin_cam(T, a.vox, bx, by, bz, cb);
           to_pixel_h(a.K, cb, hb);
+          pl = block_place(a, hb, corner);
         }
-        column_h(hf, hb, lane >> 3, lane & 7, cl);
-        const size_t fo = ((size_t)parity * kMaxBatch + jf) * frame_px;
-        const uint32_t* rgba = kColor ? a.rgba + fo : nullptr;
-        const float* dmf = a.dm + fo;
-        DepthWindow win;
-        const int place = block_place(a, hf.ax, cl, win);
-        if (place == kPlaceWindow) {
-          stage_window(a, dmf, win, s_win);
-          frame_update<kStorage, kColor, kPlaceWindow, kTab>(a, hf.ax, cl, dmf, rgba, win.shift, s_win - win.bias,
-                                                             old, cold, upd, rcp_tab);
-        } else if (place == kPlaceInside) {
-          frame_update<kStorage, kColor, kPlaceInside, kTab>(a, hf.ax, cl, dmf, rgba, 0u, 0u, old, cold, upd,
-                                                             rcp_tab);
-        } else {
-          frame_update<kStorage, kColor, kPlaceEdge, kTab>(a, hf.ax, cl, dmf, rgba, 0u, 0u, old, cold, upd, rcp_tab);
-        }
-      }
-      // Depth-only volumes write the block whole (unobserved voxels keep the words read,
-      // fresh blocks zero there; the wave owns the block in this launch), which saves the
-      // per-voxel mask; colour volumes (12 B per voxel) write fresh blocks whole and other
-      // blocks where observed.
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        if constexpr (kColor) {
-          if (fresh || ((upd >> q) & 1u)) {
-            vp[64 * q] = old[q];
-            cp[64 * q] = cold[q];
+        for (int q = 0; q < 8; ++q) vx.load(q, old[q]);
+        uint32_t upd = 0u;  // colour volumes: bit q set when voxel q was observed in the batch
+        for (uint32_t m = mark; m != 0u; m &= m - 1u) {
+          const uint32_t jf = (uint32_t)__builtin_ctz(m);
+          const int src = kBatch ? 8 * (int)jf : 0;
+          float ax[3], cl[3];
+#pragma unroll
+          for (int r = 0; r < 3; ++r) {
+            ax[r] = s_frm[jf].ax[r];
+            // the block origin plus the column's offset
+            cl[r] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hb[r]), src)) + s_col[jf].off[lane][r];
           }
-        } else {
-          vp[64 * q] = old[q];
+          const size_t fo = ((size_t)parity * kMaxBatch + jf) * frame_px;
+          const uint32_t* rgba = kColor ? a.rgba + fo : nullptr;
+          const float* dmf = a.dm + fo;
+          const uint32_t desc = read_lane_u32(pl.desc, src);
+          const uint32_t place = desc & 3u;
+          uint32_t wshift = 0u, wbase = 0u;
+          if (place == (uint32_t)kPlaceWindow) {
+            DepthWindow win;
+            win.first = read_lane_u32(pl.first, src);
+            win.bias = read_lane_u32(pl.bias, src);
+            win.shift = (desc >> 2) & 7u;
+            win.cols = (desc >> 5) & 127u;
+            win.rows = desc >> 12;
+            stage_window(a, dmf, win, s_win);
+            wshift = win.shift;
+            wbase = s_win - win.bias;
+          }
+          frame_update<kStorage, kColor, kTab, kReg>(a, place, ax, cl, dmf, rgba, wshift, wbase, t_cap, vx, cold, upd,
+                                                     rcp_tab);
+        }
+        // Depth-only volumes write the block whole (unobserved voxels keep the words read,
+        // fresh blocks zero there; the wave owns the block in this launch), which saves the
+        // per-voxel mask; colour volumes (12 B per voxel) write fresh blocks whole and other
+        // blocks where observed.
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          if constexpr (kColor) {
+            if (fresh || ((upd >> q) & 1u)) {
+              vp[lane + 64 * q] = vx.word(q);
+              cp[lane + 64 * q] = cold[q];
+            }
+          } else {
+            vp[lane + 64 * q] = vx.word(q);
+          }
         }
       }
     }
@@ -768,11 +844,12 @@ __device__ void batch_done(const FrameArgs& a, uint32_t groups, uint32_t f0, uin
 }
 
 constexpr int kIntegrateWaves = 4;  // independent workers per workgroup
-// Register budget of the integration kernels (measured on room_medium_5mm): depth only, 5
-// waves per SIMD (96 VGPRs; uncapped the two frame_update variants take 106 and leave 4
-// waves; capped, at most 7 values spill and every voxel format runs faster); colour, 4 waves
-// (128 VGPRs: at 96 about 50 values spill into the frame loop, 13 % slower).
-#define VH_INTEGRATE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(kColor ? 4 : 5)))
+// Register budget of the integration kernels: depth only, 6 waves per SIMD (80 VGPRs, at most one
+// value spills; 500 frames of a room at 5 mm in batches of 8, FP32: 6.22 ms at 5 waves, 5.94 at 6,
+// with the fused launch's 4,096 workers; before the values and weights of a block stayed in
+// registers in the form the update takes them, 6 waves spilled into the frame loop); colour, 4
+// waves (128 VGPRs: at 96 about 50 values spill into the frame loop, 13 % slower).
+#define VH_INTEGRATE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(kColor ? 4 : 6)))
 
 // The k poses of a batch (inputs cur .. cur+k-1) into LDS, read by every block of the
 // workgroup's workers (a global load per block and frame would put a memory round trip in
@@ -785,22 +862,36 @@ __device__ __forceinline__ void stage_poses(const FrameArgs& a, uint32_t cur, ui
   }
   __syncthreads();
 }
-// The poses and the homogeneous steps of a batch's frames into LDS. All 256 lanes call it.
-__device__ __forceinline__ void stage_frames(const FrameArgs& a, uint32_t cur, uint32_t k, FrameLds* s_frm,
-                                             float* rcp_tab, bool tab) {
+// The poses, homogeneous steps and column offsets of a batch's frames into LDS, and the
+// reciprocal table. pose: the t-th of the batch's 12 k pose entries in lane t. All 256 lanes call
+// it. Each wave forms the steps of the frames whose columns it fills (the same values in every
+// lane), so that one barrier separates the poses from everything made of them.
+__device__ __forceinline__ void stage_frames(const FrameArgs& a, float pose, uint32_t k, FrameLds* s_frm,
+                                             ColumnLds* s_col, float* rcp_tab, bool tab) {
   const uint32_t t = threadIdx.x;
   if (t < 12u * k) {
     const uint32_t j = t / 12u, q = t - 12u * j;
-    s_frm[j].T[q] = a.poses[16 * (size_t)input_slot(cur, j, a.n_seq) + q];
+    s_frm[j].T[q] = pose;
   }
   if (tab)
-    for (uint32_t i = t; i < kRcpTab; i += blockDim.x) rcp_tab[i] = recip_rn((float)i);
+    for (uint32_t i = t; i < kRcpTab; i += blockDim.x) rcp_tab[i] = i ? recip_rn((float)i) : 0.0f;
   __syncthreads();
-  if (t < k) {
+  const uint32_t lane = t & 63u;
+  for (uint32_t j = t >> 6; j < k; j += kIntegrateWaves) {
     float T[12];
+    BlockFrame h;
 #pragma unroll
-    for (int q = 0; q < 12; ++q) T[q] = s_frm[t].T[q];
-    block_frame_h(T, a.vox, a.K, s_frm[t].h);
+    for (int q = 0; q < 12; ++q) T[q] = s_frm[j].T[q];
+    block_frame_h(T, a.vox, a.K, h);
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      if (lane == 0) {
+        s_frm[j].ax[r] = h.ax[r];
+        s_frm[j].ay[r] = h.ay[r];
+        s_frm[j].az[r] = h.az[r];
+      }
+      s_col[j].off[lane][r] = __builtin_fmaf((float)(lane >> 3), h.ay[r], (float)(lane & 7u) * h.az[r]);
+    }
   }
   __syncthreads();
 }
@@ -813,42 +904,66 @@ __device__ __forceinline__ bool rcp_table_covers(const FrameArgs& a, const Frame
 }
 
 // The integration's LDS: per wave the staged list entries, slot values, keys and marks and
-// the depth window; per workgroup the batch's frames and the reciprocal table.
+// the depth window; per workgroup the batch's frames and the reciprocal table. kFrames: 1 or
+// kMaxBatch (27 KB, 5 workgroups per CU).
+template <int kFrames>
 struct IntegrateLds {
-  FrameLds frm[kMaxBatch];  // first: a frame's words are then within one read's offset range
+  float rcp[kRcpTab];
+  FrameLds frm[kFrames];
+  ColumnLds col[kFrames];
+  float win[kIntegrateWaves][kWin];
   unsigned long long val[kIntegrateWaves][64], key[kIntegrateWaves][64];
   uint32_t mark[kIntegrateWaves][64];
-  float rcp[kRcpTab];
-  float win[kIntegrateWaves][kWin];
 };
+template <bool kBatch>
+using IntegrateLdsOf = IntegrateLds<kBatch ? kMaxBatch : 1>;
+static_assert(offsetof(IntegrateLds<1>, win) % 16 == 0 && offsetof(IntegrateLds<kMaxBatch>, win) % 16 == 0,
+              "stage_window writes 16 bytes per lane");
 
 // The workgroup's share of the batch of k frames (first frame f0, list parity, first input
 // cur). All 256 lanes call it.
-template <int kStorage, bool kColor, bool kShared>
+template <int kStorage, bool kColor, bool kBatch>
 __device__ __forceinline__ void integrate_group(const FrameArgs& a, uint32_t group, uint32_t groups, uint32_t f0,
-                                                uint32_t k, uint32_t parity, uint32_t cur, IntegrateLds& L) {
-  const int wave = threadIdx.x >> 6;
+                                                uint32_t k, uint32_t parity, uint32_t cur, IntegrateLdsOf<kBatch>& L) {
+  const uint32_t t = threadIdx.x, lane = t & 63u;
+  const int wave = t >> 6;
+  // the pose entries and the list's lengths, in flight together
+  float pose = 0.0f;
+  if (t < 12u * k) {
+    const uint32_t j = t / 12u, q = t - 12u * j;
+    pose = a.poses[16 * (size_t)input_slot(cur, j, a.n_seq) + q];
+  }
+  const uint32_t my_len = min(list_count_of(a.ctl, parity)[lane * kLine], a.stripe_cap);
   const bool tab = rcp_table_covers(a, a.ctl, k);
-  stage_frames(a, cur, k, L.frm, L.rcp, tab);
+  // lane s holds stripe s's length and exclusive offset
+  uint32_t incl = my_len;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t y = (uint32_t)__shfl_up((int)incl, off);
+    if ((int)lane >= off) incl += y;
+  }
+  const uint32_t my_off = incl - my_len, n = read_lane_u32(incl, 63);
   const uint32_t worker = group * kIntegrateWaves + wave, workers = groups * kIntegrateWaves;
+  if (group * kIntegrateWaves >= n) return;  // a short list: no block for this workgroup
+  stage_frames(a, pose, k, L.frm, L.col, L.rcp, tab);
   const uint32_t win = uniform(lds_address(L.win[wave]));
   if (tab)
-    integrate_worker<kStorage, kColor, true, kShared>(a, worker, workers, f0, k, parity, L.val[wave], L.key[wave],
-                                                      L.mark[wave], L.frm, L.rcp, win);
+    integrate_worker<kStorage, kColor, true, kBatch>(a, worker, workers, my_off, n, f0, k, parity, L.val[wave],
+                                                     L.key[wave], L.mark[wave], L.frm, L.col, L.rcp, win);
   else
-    integrate_worker<kStorage, kColor, false, kShared>(a, worker, workers, f0, k, parity, L.val[wave], L.key[wave],
-                                                       L.mark[wave], L.frm, L.rcp, win);
+    integrate_worker<kStorage, kColor, false, kBatch>(a, worker, workers, my_off, n, f0, k, parity, L.val[wave],
+                                                      L.key[wave], L.mark[wave], L.frm, L.col, L.rcp, win);
 }
 
-// Integration of the batch of k frames that the last allocation launch prepared (kShared: k > 1).
-template <int kStorage, bool kColor, bool kShared>
+// Integration of the batch of k frames that the last allocation launch prepared (kBatch: k > 1).
+template <int kStorage, bool kColor, bool kBatch>
 __global__ __launch_bounds__(64 * kIntegrateWaves) VH_INTEGRATE_OCCUPANCY void k_integrate(FrameArgs a, uint32_t k) {
-  __shared__ IntegrateLds L;
+  __shared__ IntegrateLdsOf<kBatch> L;
   const FrameCtl* ctl = a.ctl;
   // control values are uniform: keep them (and what derives from them) in scalar registers
   const uint32_t f0 = uniform(ctl->frame_id), parity = uniform(ctl->batch_id) & 1u,
                  cur = uniform(ctl->cursor[a.cursor_id]);
-  integrate_group<kStorage, kColor, kShared>(a, blockIdx.x, gridDim.x, f0, k, parity, cur, L);
+  integrate_group<kStorage, kColor, kBatch>(a, blockIdx.x, gridDim.x, f0, k, parity, cur, L);
   batch_done(a, gridDim.x, f0, k, parity);
 }
 
@@ -865,7 +980,7 @@ __global__ __launch_bounds__(64 * kIntegrateWaves) VH_INTEGRATE_OCCUPANCY void k
   // a workgroup either allocates or integrates: the two share the LDS
   __shared__ union {
     AllocLds<kAllocRows> alloc;
-    IntegrateLds integ;
+    IntegrateLdsOf<true> integ;
   } L;
   const uint32_t b = blockIdx.x;
   const bool alloc = b >= int_groups;

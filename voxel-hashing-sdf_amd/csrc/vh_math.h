@@ -130,12 +130,8 @@ VH_HD void block_frame_h(const float* T, float vox, const Intr& K, BlockFrame& f
   to_pixel_h(K, c.ay, f.ay);
   to_pixel_h(K, c.az, f.az);
 }
-// Homogeneous coordinates of the column (j, i) of a block whose origin is at cb (homogeneous):
-// cb + fma(j, b, i*c); voxel k of the column is then fma(k, a, column).
-VH_HD void column_h(const BlockFrame& f, const float cb[3], int j, int i, float out[3]) {
-  const float fj = (float)j, fi = (float)i;
-  for (int r = 0; r < 3; ++r) out[r] = cb[r] + fmaf(fj, f.ay[r], fi * f.az[r]);
-}
+// The column (j, i) of a block whose origin is at cb (homogeneous) lies at cb + fma(j, b, i c) with
+// the frame's homogeneous steps b, c along y and z; voxel k of it at fma(k, a, column).
 
 // Observation of the voxel at homogeneous point (X, Y, z) (reference IntegrateHashKernel skip
 // rules, src/tsdf.cu:706-738), in two steps so that a caller can issue all depth fetches of a
@@ -146,7 +142,7 @@ VH_HD void column_h(const BlockFrame& f, const float cb[3], int j, int i, float 
 //     (the reference divides per coordinate and rounds ties away from zero, cam2frame,
 //     src/tsdf.cu:75-79). Within the image the sum lies in [2^23, 2^24), where the float
 //     spacing is 1, so the sum is M plus the rounded coordinate, and its bits give the pixel
-//     index without a conversion. -1 when z is outside 2^-64 <= z <= 2^64 or the pixel outside
+//     index (in an image of row pitch `pitch`) without a conversion. -1 when z is outside 2^-64 <= z <= 2^64 or the pixel outside
 //     the image. The range bound keeps z and 1/z normal, where the kernels' three-instruction
 //     reciprocal equals the IEEE quotient.
 //   truncation: the pixel's pre-scaled depth m = d * (1/mu) for a depth 0 < d <= max_depth
@@ -156,14 +152,12 @@ VH_HD void column_h(const BlockFrame& f, const float cb[3], int j, int i, float 
 constexpr float kMinZ = 0x1p-64f, kMaxZ = 0x1p64f;
 constexpr float kPixMagic = 0x1.8p23f;  // M = 1.5 * 2^23, bits 0x4B400000
 constexpr uint32_t kPixMagicBits = 0x4B400000u;
-VH_HD int pixel_of(float X, float Y, float z, float iz, int W, int H) {
-  const float uf = fmaf(X, iz, kPixMagic);
-  const float vf = fmaf(Y, iz, kPixMagic);
+VH_HD int pixel_of(float uf, float vf, float z, int W, int H, int pitch) {
   const bool inside = (z >= kMinZ) & (z <= kMaxZ) & (uf >= kPixMagic) & (uf <= kPixMagic + (float)(W - 1)) &
                       (vf >= kPixMagic) & (vf <= kPixMagic + (float)(H - 1));
   // both factors are below 2^24 (W, H <= 16384): the masks let the compiler use a 24-bit
   // multiply-add instead of a 64-bit one
-  return inside ? (int)(((uint32_t)(vf - kPixMagic) & 0xffffffu) * ((uint32_t)W & 0xffffffu) + (uint32_t)(uf - kPixMagic))
+  return inside ? (int)(((uint32_t)(vf - kPixMagic) & 0xffffffu) * ((uint32_t)pitch & 0xffffffu) + (uint32_t)(uf - kPixMagic))
                 : -1;
 }
 // Byte offset 4 (v W + u) of pixel (u, v) from the sums uf = M + u, vf = M + v of pixel_of
