@@ -77,29 +77,37 @@ __device__ __forceinline__ float depth_at(const void* base, float scale, int pix
 }
 
 // ============================================================================ allocation
-// Workgroup = a tile of 16 x 64 pixels, 256 lanes, each lane one pixel in each of the tile's
-// four 16 x 16 bands. Phase 1: every lane walks its pixels' truncation bands in turn and
-// inserts the block keys into an LDS hash set, so each distinct block of the tile is kept
-// once. Phase 2: the distinct keys go to the
-// global hash (find or insert), take a pool index if new, and mark the block for this frame
-// of the batch (an atomic OR of the frame's bit into the slot's mark); the lanes that found
-// the mark empty append the slot to the workgroup's stripe of the batch's block list, and
-// the lanes that found their frame's bit clear count the block for that frame.
+// Workgroup = a tile of 64 x 16 pixels (16 x 16 in a single frame's launch), 256 lanes, each lane
+// one pixel in each of the tile's 16 x 16 bands, so a workgroup reads and writes whole cache lines
+// of the image rows. Phase 1: the blocks that the pixels' truncation bands cross go into an LDS hash
+// set, so each distinct block of the tile is kept once. Phase 2: the distinct keys go to the global
+// hash (find or insert), take a pool index if new, and mark the block for this frame of the batch
+// (an atomic OR of the frame's bit into the slot's mark); the lanes that found the mark empty append
+// the slot to the workgroup's stripe of the batch's block list, and the lanes that found their
+// frame's bit clear count the block for that frame.
+// What bounds it: vector issue (about 270 instructions per wave and band) with the latency of the
+// set and of phase 2's four dependent round trips between. 8 frames of 640 x 480 launched alone:
+// 5 mm 43.3 -> 31.5 us, 1 cm 38.2 -> 28.0 us against a walk per lane with a compare-and-swap per key
+// (a launch without the bands takes 7.7 us, without the set 22.6).
 constexpr int kSetSlots = 1024;  // LDS key set (8 KB)
-constexpr int kUniqCap = 1024;   // distinct keys kept per tile (8 KB)
-// 16-row bands per tile of a batched launch. One workgroup per four bands pays the LDS clear,
+// 16 x 16 bands per tile of a batched launch. One workgroup per four bands pays the LDS clear,
 // the barriers and the chain of dependent global atomics of phase 2 once for all four, and
-// merges the bands' keys: the fused batch launch ran 3.8 % faster than with one band
-// (room_medium_5mm), 2, 6 and 8 bands gained less or lost. A single frame's launch keeps one
-// band per workgroup, which fills the GPU with 4x as many workgroups.
-constexpr int kAllocRows = 4;
-__host__ __device__ constexpr uint32_t alloc_tiles(int W, int H, int rows) {
-  return (uint32_t)(((W + 15) >> 4) * ((H + 16 * rows - 1) / (16 * rows)));
+// merges the bands' keys: 500 frames at 5 mm take 6.41 ms with 2 bands, 6.00 with 4, 6.01 with 5. A
+// single frame's launch keeps one band per workgroup, which fills the GPU with 4x as many
+// workgroups.
+constexpr int kAllocBands = 4;
+__host__ __device__ constexpr uint32_t alloc_tiles(int W, int H, int bands) {
+  return (uint32_t)(((W + 16 * bands - 1) / (16 * bands)) * ((H + 15) >> 4));
 }
 
+// Home slot of a packed key in a tile's set. pack_key is linear in the block coordinates, so a step
+// along an axis adds a constant (key_step).
 static_assert(kSetSlots == 1 << 10, "set_hash gives 10 bits");
 __device__ __forceinline__ uint32_t set_hash(uint64_t key) {
   return (((uint32_t)key ^ (uint32_t)(key >> 32)) * 0x9e3779b1u) >> 22;
+}
+__device__ __forceinline__ uint64_t key_step(int dx, int dy, int dz) {
+  return ((uint64_t)(int64_t)dx << (2 * kKeyBits)) + ((uint64_t)(int64_t)dy << kKeyBits) + (uint64_t)(int64_t)dz;
 }
 
 // The block list, its stripe lengths and the slot marks are double-buffered by batch
@@ -184,32 +192,173 @@ __device__ void claim_keys(const FrameArgs& a, uint64_t key, bool act, uint32_t 
   }
 }
 
-// Allocation of one tile of frame `frame` (index jb of its batch, input slot fs): 16 pixel
-// columns by 16 * kRows rows, 256 lanes, each lane one pixel of every 16-row band.
 // The allocation's LDS: the key set, the tile's distinct keys and, for carving volumes, the
 // bands' largest depths.
-template <int kRows>
+template <int kBands>
 struct AllocLds {
   unsigned long long set[kSetSlots];
-  unsigned long long uniq[kUniqCap];
+  unsigned long long uniq[kSetSlots];
   uint32_t nuniq;
-  float tmax[4][kRows];
+  float tmax[4][kBands];
 };
 
+// Puts the active lanes' keys into the tile's set; a key new to the set joins the list of distinct
+// keys (at most one entry per slot). True for lanes whose key found no room within 32 probes. A
+// probe reads before it swaps: a key that is there is found by a read, which serves equal keys of
+// the wave at once.
+template <int kBands>
+__device__ __forceinline__ bool set_insert(AllocLds<kBands>& L, unsigned long long key, bool act) {
+  bool spill = act;
+  if (act) {
+    uint32_t h = set_hash(key);
+#pragma unroll 1
+    for (int p = 0; p < 32; ++p) {
+      unsigned long long old = __hip_atomic_load(&L.set[h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (old == kEmptyKey) {
+        old = atomicCAS(&L.set[h], (unsigned long long)kEmptyKey, key);
+        if (old == kEmptyKey) L.uniq[atomicAdd(&L.nuniq, 1u)] = key;
+      }
+      if (old == key || old == kEmptyKey) { spill = false; break; }
+      h = (h + 1) & (kSetSlots - 1);
+    }
+  }
+  return spill;
+}
+
+// x of another lane of the row of 16 (DPP control kCtrl).
+template <int kCtrl>
+__device__ __forceinline__ int32_t dpp(int32_t x) { return __builtin_amdgcn_mov_dpp(x, kCtrl, 0xf, 0xf, false); }
+// Windows of a wave's pixels in a single frame's launch; the lanes left then walk. A frame of
+// 47,000 blocks at 4 mm, far and noisy: 16.6 us with no limit, 15.3 with 2; one of 15,000 at 5 mm:
+// 9.8 and 10.7. A batch's launch, with four bands per workgroup, is 1 to 3 % slower with a limit.
+constexpr int kMaxWindows = 3;
+
+// OR of x over the wave's lanes (in every lane's result; DPP within rows of 16, then the rows').
+__device__ __forceinline__ uint32_t wave_or(uint32_t x) {
+  x |= (uint32_t)dpp<0xB1>((int32_t)x);
+  x |= (uint32_t)dpp<0x4E>((int32_t)x);
+  x |= (uint32_t)dpp<0x141>((int32_t)x);
+  x |= (uint32_t)dpp<0x140>((int32_t)x);
+  return read_lane_u32(x, 0) | read_lane_u32(x, 16) | read_lane_u32(x, 32) | read_lane_u32(x, 48);
+}
+
+// The distinct blocks of a tile's bands, claimed. A wave's 8 x 8 pixels cross a handful of
+// blocks near one another, so they are gathered as bits: the window is the 4 x 4 x 4 blocks
+// around one lane's band, every lane whose band lies in it sets the bits of its blocks in a
+// 64-bit word, the words are ORed over the wave, and lane i then holds block i of the window
+// where its bit is set: at most one key per lane, all distinct, go to the tile's set in one round
+// (each lane's keys in turn took a round trip and its mask arithmetic per key: 12 of 36 us of a
+// batch of 8 frames launched alone). Lanes outside take the next window.
+// The blocks of a band that moves at most one block per axis are known without a walk: the
+// first; the first after one step along the axis crossed first; the last before the step along
+// the axis crossed last; the last (band_next's order: smallest crossing parameter first, ties to
+// the lower axis). Bands of two blocks along an axis walk within the window, longer ones
+// (truncations of more than four voxels) insert block by block.
+template <int kBands>
+__device__ __forceinline__ void tile_bands(const FrameArgs& a, const float* T, const float* dr, int u0, int v,
+                                           uint32_t frame, uint32_t jb, uint32_t parity, uint32_t stripe,
+                                           AllocLds<kBands>& L) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // lane i's block of a window: (i >> 4, (i >> 2) & 3, i & 3) from its corner
+  const uint64_t lane_off = key_step(lane >> 4, (lane >> 2) & 3, lane & 3);
+#pragma unroll 1
+  for (int r = 0; r < kBands; ++r) {
+    const int u = u0 + 16 * r;
+    bool active = u < a.W && v < a.H && depth_valid(dr[r], a.max_depth);
+    if (!__ballot(active)) continue;
+    float A[3], B[3];
+    const bool in_range = band_segment(T, a.K, a.band, a.mu, a.min_depth, u, v, dr[r], A, B);
+    if (active && !in_range) raise_flag(a.ctl, kFlagRange);
+    active = active && in_range;
+    BandDDA s;
+    band_start(A, B, s, [](float x) { return recip_rn(x); });
+    const int sx = s.ex - s.ix, sy = s.ey - s.iy, sz = s.ez - s.iz;
+    const int reach = max(max(abs(sx), abs(sy)), abs(sz)), moves = abs(sx) + abs(sy) + abs(sz);
+    // one-block moves: the faces' crossing parameters (band_t), infinite along an axis that stays
+    const float tx = sx ? ((float)max(s.ix, s.ex) - s.ax) * s.rx : INFINITY;
+    const float ty = sy ? ((float)max(s.iy, s.ey) - s.ay) * s.ry : INFINITY;
+    const float tz = sz ? ((float)max(s.iz, s.ez) - s.az) * s.rz : INFINITY;
+    const int bx = 16 * sx, by = 4 * sy, bz = sz;  // steps in window bits
+    const int b_first = tx <= ty && tx <= tz ? bx : (ty <= tz ? by : bz);
+    const int b_last = tz >= tx && tz >= ty ? bz : (ty >= tx ? by : bx);  // used where all three move
+    uint64_t left = __ballot(active && reach <= 2);
+    bool walking = active && reach > 2;
+    for (int windows = 0;; ++windows) {
+      uint64_t key;
+      bool want;
+      if (left && (kBands > 1 || windows < kMaxWindows)) {
+        const int lead = (left >> 27) & 1u ? 27 : first_lane(left);  // a lane in the middle if it can be
+        const int wx = __builtin_amdgcn_readlane(min(s.ix, s.ex), lead) - 1,
+                  wy = __builtin_amdgcn_readlane(min(s.iy, s.ey), lead) - 1,
+                  wz = __builtin_amdgcn_readlane(min(s.iz, s.ez), lead) - 1;
+        const int x0 = s.ix - wx, y0 = s.iy - wy, z0 = s.iz - wz;
+        const bool in = __builtin_amdgcn_inverse_ballot_w64(left) &&
+                        (uint32_t)((x0 | y0 | z0) | ((x0 + sx) | (y0 + sy) | (z0 + sz))) < 4u;
+        const int i0 = 16 * x0 + 4 * y0 + z0, i3 = i0 + ((bx + by) + bz);
+        uint64_t bits = 0u;
+        if (in) {
+          bits = (1ull << (i0 & 63)) | (1ull << (i3 & 63));
+          if (moves > 1) bits |= 1ull << ((i0 + b_first) & 63);
+          if (moves > 2) bits |= 1ull << ((i3 - b_last) & 63);
+        }
+        const bool two = in && reach > 1;
+        if (__ballot(two)) {
+          BandDDA w = s;
+          bool more = two;
+          if (two) bits = 0u;
+          while (__ballot(more)) {
+            if (more) {
+              bits |= 1ull << ((16 * (w.ix - wx) + 4 * (w.iy - wy) + (w.iz - wz)) & 63);
+              more = band_next(w);
+            }
+          }
+        }
+        want = __builtin_amdgcn_inverse_ballot_w64((uint64_t)wave_or((uint32_t)bits) |
+                                                   (uint64_t)wave_or((uint32_t)(bits >> 32)) << 32);
+        key = pack_key(wx, wy, wz) + lane_off;
+        left &= ~__ballot(in);
+      } else {
+        walking = walking || __builtin_amdgcn_inverse_ballot_w64(left);
+        left = 0u;
+        if (!__ballot(walking)) break;
+        key = pack_key(s.ix, s.iy, s.iz);
+        want = walking;
+        if (walking) walking = band_next(s);
+      }
+      const uint64_t home = __hip_atomic_load(&L.set[set_hash(key)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const bool need = want && home != key;
+      if (__ballot(need)) {
+        const bool spill = set_insert(L, key, need);
+        if (__ballot(spill)) claim_keys(a, key, spill, frame, jb, parity, lane, stripe);
+      }
+    }
+  }
+  __syncthreads();
+  // the tile's distinct keys
+  const uint32_t n = L.nuniq;
+  for (uint32_t b0 = 0; b0 < n; b0 += 256) {
+    const uint32_t i = b0 + tid;
+    const bool act = i < n;
+    const uint32_t wave_first = b0 + (uint32_t)(wave << 6);
+    if (wave_first >= n) break;  // whole wave idle (uniform per wave)
+    claim_keys(a, act ? L.uniq[i] : kEmptyKey, act, frame, jb, parity, lane, stripe);
+  }
+}
+
+// Allocation of one tile of frame `frame` (index jb of its batch, input slot fs): 16 pixel
+// rows by 16 * kBands columns, 256 lanes, each lane one pixel of every 16 x 16 band (a wave 8 x 8
+// of them).
 // kColor: the volume keeps colour (a.rgba is set), known at compile time so that no branch
 // separates the tile's loads.
-template <bool kU16, int kRows, bool kColor>
+template <bool kU16, int kBands, bool kColor>
 __device__ void alloc_tile(const FrameArgs& a, uint32_t tile, uint32_t frame, uint32_t jb, uint32_t parity,
-                           uint32_t fs, AllocLds<kRows>& L) {
-  unsigned long long* s_set = L.set;
-  unsigned long long* s_uniq = L.uniq;
-  uint32_t& s_nuniq = L.nuniq;
+                           uint32_t fs, AllocLds<kBands>& L) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int tiles_x = (a.W + 15) >> 4;
-  const int u = ((int)(tile % tiles_x) << 4) + ((wave & 1) << 3) + (lane & 7);
-  const int v0 = (int)(tile / tiles_x) * (16 * kRows) + ((wave >> 1) << 3) + (lane >> 3);
+  const int tiles_x = (a.W + 16 * kBands - 1) / (16 * kBands);
+  const int tx = (int)(tile % tiles_x), ty = (int)(tile / tiles_x);
+  const int u0 = tx * (16 * kBands) + ((wave & 1) << 3) + (lane & 7);
+  const int v = ty * 16 + ((wave >> 1) << 3) + (lane >> 3);
   const uint32_t stripe = tile & (kStripes - 1);
-  FrameCtl* ctl = a.ctl;
   const float* Tp = a.poses + 16 * (size_t)fs;
   float T[12];
 #pragma unroll
@@ -220,12 +369,12 @@ __device__ void alloc_tile(const FrameArgs& a, uint32_t tile, uint32_t frame, ui
   // the lane's depths (and colours) of all bands: every load is issued before the first use
   // (a pixel outside the image loads a pixel inside it, whose value is not used), so the loads
   // are in flight together
-  float dr[kRows];
-  uint32_t px3[kRows][3];
-  const int uc = min(u, a.W - 1);
+  float dr[kBands];
+  uint32_t px3[kBands][3];
+  const int vc = min(v, a.H - 1);
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const int vc = min(v0 + 16 * r, a.H - 1);
+  for (int r = 0; r < kBands; ++r) {
+    const int uc = min(u0 + 16 * r, a.W - 1);
     dr[r] = depth_at<kU16>(base, a.depth_scale, vc * a.W + uc);
     if constexpr (kColor) {
       const uint8_t* px = a.rgb + ((size_t)fs * a.W * a.H + (size_t)vc * a.W + uc) * 3;
@@ -234,8 +383,8 @@ __device__ void alloc_tile(const FrameArgs& a, uint32_t tile, uint32_t frame, ui
     }
   }
 #pragma unroll
-  for (int r = 0; r < kRows; ++r) {
-    const int v = v0 + 16 * r;
+  for (int r = 0; r < kBands; ++r) {
+    const int u = u0 + 16 * r;
     if (u < a.W && v < a.H) {
       const size_t staged = (((size_t)parity * kMaxBatch + jb) * a.H + v) * a.pitch + u;
       // the pixel's colour, packed for the integration's one-word gathers
@@ -248,77 +397,35 @@ __device__ void alloc_tile(const FrameArgs& a, uint32_t tile, uint32_t frame, ui
   }
 
   // carving volumes: the largest valid depth of each 16 x 16 band (a max-depth tile)
-  float (*s_tmax)[kRows] = L.tmax;
+  float (*s_tmax)[kBands] = L.tmax;
   if (a.tilemax) {
 #pragma unroll
-    for (int r = 0; r < kRows; ++r) {
+    for (int r = 0; r < kBands; ++r) {
       float m = depth_valid(dr[r], a.max_depth) ? dr[r] : 0.0f;
 #pragma unroll
       for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
       if (lane == 0) s_tmax[wave][r] = m;
     }
   }
-  for (int i = tid; i < kSetSlots; i += 256) s_set[i] = kEmptyKey;
-  if (tid == 0) s_nuniq = 0;
+  for (int i = tid; i < kSetSlots; i += 256) L.set[i] = kEmptyKey;
+  if (tid == 0) L.nuniq = 0;
   __syncthreads();
-  if (a.tilemax && tid < kRows) {
-    const int ty = (int)(tile / tiles_x) * kRows + tid;
-    if (ty < a.tiles_y)
-      a.tilemax[((size_t)parity * kMaxBatch + jb) * a.tiles_x * a.tiles_y + (size_t)ty * a.tiles_x + tile % tiles_x] =
+  if (a.tilemax && tid < kBands) {
+    const int mx = tx * kBands + tid;
+    if (mx < a.tiles_x)
+      a.tilemax[(((size_t)parity * kMaxBatch + jb) * a.tiles_y + ty) * a.tiles_x + mx] =
           fmaxf(fmaxf(s_tmax[0][tid], s_tmax[1][tid]), fmaxf(s_tmax[2][tid], s_tmax[3][tid]));
   }
-
-#pragma unroll 1
-  for (int r = 0; r < kRows; ++r) {
-    const int v = v0 + 16 * r;
-    BandDDA s;
-    bool active = false;
-    if (u < a.W && v < a.H && depth_valid(dr[r], a.max_depth)) {
-      active = band_setup(T, a.K, a.band, a.mu, a.min_depth, u, v, dr[r], s, [](float x) { return recip_rn(x); });
-      if (!active) raise_flag(ctl, kFlagRange);
-    }
-    // phase 1: distinct keys of the tile into LDS; keys that do not fit are claimed directly
-    while (__ballot(active)) {
-      bool spill = false;
-      uint64_t key = kEmptyKey;
-      if (active) {
-        key = pack_key(s.ix, s.iy, s.iz);
-        uint32_t h = set_hash(key);
-        spill = true;
-        for (int p = 0; p < 32; ++p) {
-          const unsigned long long old = atomicCAS(&s_set[h], (unsigned long long)kEmptyKey, (unsigned long long)key);
-          if (old == key) { spill = false; break; }
-          if (old == kEmptyKey) {
-            const uint32_t n = atomicAdd(&s_nuniq, 1u);
-            if (n < kUniqCap) { s_uniq[n] = key; spill = false; }
-            break;
-          }
-          h = (h + 1) & (kSetSlots - 1);
-        }
-      }
-      if (__ballot(spill)) claim_keys(a, key, spill, frame, jb, parity, lane, stripe);
-      if (active) active = band_next(s);
-    }
-  }
-  __syncthreads();
-  // phase 2: the tile's distinct keys
-  const uint32_t n = min(s_nuniq, (uint32_t)kUniqCap);
-  for (uint32_t b0 = 0; b0 < n; b0 += 256) {
-    const uint32_t i = b0 + tid;
-    const bool act = i < n;
-    const uint32_t wave_first = b0 + (uint32_t)(wave << 6);
-    if (wave_first >= n) break;  // whole wave idle (uniform per wave)
-    claim_keys(a, act ? s_uniq[i] : kEmptyKey, act, frame, jb, parity, lane, stripe);
-  }
+  tile_bands(a, T, dr, u0, v, frame, jb, parity, stripe, L);
 }
 
 // Allocation of the batch about to be integrated: `tiles` workgroups per frame.
-template <bool kU16, int kRows, bool kColor>
-__global__ __launch_bounds__(256) void k_alloc(FrameArgs a, uint32_t tiles) {
-  __shared__ AllocLds<kRows> L;
+template <bool kU16, int kBands, bool kColor>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_alloc(FrameArgs a, uint32_t tiles) {
+  __shared__ AllocLds<kBands> L;
   const uint32_t jb = blockIdx.x / tiles;
   const FrameCtl* ctl = a.ctl;
-  alloc_tile<kU16, kRows, kColor>(a, blockIdx.x - jb * tiles, ctl->frame_id + jb, jb, ctl->batch_id & 1u,
+  alloc_tile<kU16, kBands, kColor>(a, blockIdx.x - jb * tiles, ctl->frame_id + jb, jb, ctl->batch_id & 1u,
                           input_slot(ctl->cursor[a.cursor_id], jb, a.n_seq), L);
 }
 
@@ -381,8 +488,6 @@ struct DepthWindow {
 
 // Smallest and largest of x over the 8 lanes of an aligned group (DPP: the quad's pairs, the
 // quad's halves, the half-row mirror).
-template <int kCtrl>
-__device__ __forceinline__ int32_t dpp(int32_t x) { return __builtin_amdgcn_mov_dpp(x, kCtrl, 0xf, 0xf, false); }
 __device__ __forceinline__ int32_t oct_min(int32_t x) {
   x = min(x, dpp<0xB1>(x));
   x = min(x, dpp<0x4E>(x));
@@ -979,7 +1084,7 @@ __global__ __launch_bounds__(64 * kIntegrateWaves) VH_INTEGRATE_OCCUPANCY void k
                                                                          uint32_t k_int) {
   // a workgroup either allocates or integrates: the two share the LDS
   __shared__ union {
-    AllocLds<kAllocRows> alloc;
+    AllocLds<kAllocBands> alloc;
     IntegrateLdsOf<true> integ;
   } L;
   const uint32_t b = blockIdx.x;
@@ -989,7 +1094,7 @@ __global__ __launch_bounds__(64 * kIntegrateWaves) VH_INTEGRATE_OCCUPANCY void k
   const uint32_t f0 = uniform(ctl->frame_id), batch = uniform(ctl->batch_id), cur = uniform(ctl->cursor[a.cursor_id]);
   if (alloc) {
     const uint32_t jb = idx / tiles;
-    alloc_tile<kU16, kAllocRows, kColor>(a, idx - jb * tiles, f0 + k_int + jb, jb, (batch + 1u) & 1u,
+    alloc_tile<kU16, kAllocBands, kColor>(a, idx - jb * tiles, f0 + k_int + jb, jb, (batch + 1u) & 1u,
                                  input_slot(cur, k_int + jb, a.n_seq), L.alloc);
   } else {  // uniform branch: the whole workgroup integrates
     integrate_group<kStorage, kColor, true>(a, idx, int_groups, f0, k_int, batch & 1u, cur, L.integ);
@@ -1089,7 +1194,10 @@ __global__ __launch_bounds__(256) void k_carve(FrameArgs a, uint32_t k) {
     if (b < n) {
       const unsigned long long info = a.block_info[b];
       slot = (uint32_t)info;
-      const int32_t born = (int32_t)((uint32_t)(info >> 32) - f0);  // birth frame relative to f0
+      // birth frame relative to f0; for a block born in this batch the first frame whose bands
+      // cross it (the recorded frame is that of the lane that inserted the key, in no fixed order)
+      int32_t born = (int32_t)((uint32_t)(info >> 32) - f0);
+      if (born >= 0) born = (int32_t)__builtin_ctz(marks[slot] | 1u << (k - 1u));
       int bx, by, bz;
       unpack_key(a.block_keys[b], bx, by, bz);
       for (uint32_t j = 0; j < k; ++j)
@@ -2730,12 +2838,12 @@ static void with_input(bool u16, bool color, F f) {
 }
 
 hipError_t launch_alloc(const FrameArgs& a, int depth_u16, int k, hipStream_t st) {
-  const int rows = k > 1 ? kAllocRows : 1;
-  const uint32_t tiles = alloc_tiles(a.W, a.H, rows);
+  const int bands = k > 1 ? kAllocBands : 1;
+  const uint32_t tiles = alloc_tiles(a.W, a.H, bands);
   const dim3 g(tiles * k), b(256);
   with_input(depth_u16 != 0, a.rgba != nullptr, [&](auto U, auto C) {
     constexpr bool u16 = decltype(U)::value, col = decltype(C)::value;
-    if (rows > 1) hipLaunchKernelGGL((k_alloc<u16, kAllocRows, col>), g, b, 0, st, a, tiles);
+    if (bands > 1) hipLaunchKernelGGL((k_alloc<u16, kAllocBands, col>), g, b, 0, st, a, tiles);
     else hipLaunchKernelGGL((k_alloc<u16, 1, col>), g, b, 0, st, a, tiles);
   });
   return hipGetLastError();
@@ -2773,7 +2881,7 @@ hipError_t launch_carve(const FrameArgs& a, int k, hipStream_t st) {
 hipError_t launch_integrate_alloc(const FrameArgs& a, int storage, int depth_u16, int grid, int k_int, int k_alloc,
                                   hipStream_t st) {
   const uint32_t ig = (uint32_t)(grid / kIntegrateWaves);
-  const uint32_t tiles = alloc_tiles(a.W, a.H, kAllocRows);
+  const uint32_t tiles = alloc_tiles(a.W, a.H, kAllocBands);
   const uint32_t ag = tiles * (uint32_t)k_alloc;
   with_storage(storage, [&](auto S) {
     with_input(depth_u16 != 0, a.colors != nullptr, [&](auto U, auto C) {

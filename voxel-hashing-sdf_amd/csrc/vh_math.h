@@ -281,8 +281,7 @@ VH_HD float f16r_inv_scale_of(float hf) {
 // This replaces the reference's whole-ray DDA over every 10th pixel (src/tsdf.cu:2088-2238),
 // which ignores the truncation band. Steps are chosen among the axes that still have to
 // move, smallest crossing parameter first, ties to the lower axis; the walk therefore ends
-// exactly at the end block after |e - i|_1 steps. band_setup returns false if the band
-// leaves the key range.
+// exactly at the end block after |e - i|_1 steps.
 struct BandDDA {
   float ax, ay, az;  // start point, block units
   float rx, ry, rz;  // band_recip of the direction (end - start)
@@ -311,10 +310,9 @@ VH_HD BandScale band_scale(const Intr& K, float bsz) { return BandScale{1.0f / K
 // Segment of pixel (u, v) between camera depths t0 = max(d - mu, min_depth) and t1 = d + mu,
 // in block units: the pixel's ray per unit depth r = ((u - cx) * RN(1/fx), (v - cy) * RN(1/fy)),
 // camera points (r t, t), world points R p + t (cam_to_world), block coordinates
-// world * RN(1/bsz).
-template <class Rn>
-VH_HD bool band_setup(const float* T, const Intr& K, const BandScale& sc, float mu, float min_depth, int u,
-                      int v, float d, BandDDA& s, Rn rn) {
+// world * RN(1/bsz). False when an end point leaves the key range.
+VH_HD bool band_segment(const float* T, const Intr& K, const BandScale& sc, float mu, float min_depth, int u, int v,
+                        float d, float a[3], float b[3]) {
   float t0 = d - mu;
   if (t0 < min_depth) t0 = min_depth;
   const float t1 = d + mu;
@@ -322,16 +320,20 @@ VH_HD bool band_setup(const float* T, const Intr& K, const BandScale& sc, float 
   float wax, way, waz, wbx, wby, wbz;
   cam_to_world(T, rx * t0, ry * t0, t0, wax, way, waz);
   cam_to_world(T, rx * t1, ry * t1, t1, wbx, wby, wbz);
-  s.ax = wax * sc.ibsz; s.ay = way * sc.ibsz; s.az = waz * sc.ibsz;
-  const float bx = wbx * sc.ibsz, by = wby * sc.ibsz, bz = wbz * sc.ibsz;
+  a[0] = wax * sc.ibsz; a[1] = way * sc.ibsz; a[2] = waz * sc.ibsz;
+  b[0] = wbx * sc.ibsz; b[1] = wby * sc.ibsz; b[2] = wbz * sc.ibsz;
   const float lim = 1048000.0f;  // keeps every block inside the 21-bit key range (NaN fails)
-  const int in_range = (int)(fabsf(s.ax) < lim) & (int)(fabsf(s.ay) < lim) & (int)(fabsf(s.az) < lim) &
-                       (int)(fabsf(bx) < lim) & (int)(fabsf(by) < lim) & (int)(fabsf(bz) < lim);
-  if (!in_range) return false;
-  s.rx = band_recip(bx - s.ax, rn); s.ry = band_recip(by - s.ay, rn); s.rz = band_recip(bz - s.az, rn);
-  s.ix = (int)floorf(s.ax); s.iy = (int)floorf(s.ay); s.iz = (int)floorf(s.az);
-  s.ex = (int)floorf(bx); s.ey = (int)floorf(by); s.ez = (int)floorf(bz);
-  return true;
+  const int in_range = (int)(fabsf(a[0]) < lim) & (int)(fabsf(a[1]) < lim) & (int)(fabsf(a[2]) < lim) &
+                       (int)(fabsf(b[0]) < lim) & (int)(fabsf(b[1]) < lim) & (int)(fabsf(b[2]) < lim);
+  return in_range != 0;
+}
+// The walk from a to b (band_segment).
+template <class Rn>
+VH_HD void band_start(const float a[3], const float b[3], BandDDA& s, Rn rn) {
+  s.ax = a[0]; s.ay = a[1]; s.az = a[2];
+  s.rx = band_recip(b[0] - a[0], rn); s.ry = band_recip(b[1] - a[1], rn); s.rz = band_recip(b[2] - a[2], rn);
+  s.ix = (int)floorf(a[0]); s.iy = (int)floorf(a[1]); s.iz = (int)floorf(a[2]);
+  s.ex = (int)floorf(b[0]); s.ey = (int)floorf(b[1]); s.ez = (int)floorf(b[2]);
 }
 // Crossing parameter of the next block face along one axis (only for axes still moving):
 // (face - a) * band_recip(direction).
