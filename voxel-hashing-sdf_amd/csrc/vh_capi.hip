@@ -59,10 +59,12 @@ constexpr int kIntegrateGrid = 5120;
 // 3,072 / 4,096 / 5,120 workers: 6.83 / 5.96 / 5.75 / 5.77 ms; F16R + colour, 64 frames: 1.40 /
 // 1.27 / 1.23 / 1.26 ms.
 constexpr int kFusedGrid = 4096;
-constexpr int kGnGrid = 512;  // most workgroups of a solver or backward reduction
+constexpr int kGnGrid = 512;  // most partial sums of a solver reduction
+constexpr int kBackwardGrid = 2048;  // most workgroups of a backward reduction
+static_assert(kBackwardGrid * 6 <= 2 * kGnGrid * kGnAcc, "the solver's partial sums hold the backward's");
 
-// Solver grid for n points: one point per lane, up to kGnGrid workgroups (a partial per
-// workgroup is summed by the solve step). The accumulation is latency-bound, so the shorter
+// Partial sums of a solver evaluation over n points: one per 256 points, up to kGnGrid (they
+// are summed by the solve step). The accumulation is latency-bound, so the shorter
 // chain per lane wins over the extra partials: tracked floor_large_4mm (19,200 points per
 // evaluation) 4,532 frames/s with two points per lane, 4,783 with one, 3,766 with four.
 int gn_grid(int64_t n) {
@@ -279,6 +281,7 @@ QueryArgs query_args(vh_volume* v) {
   q.voxels = v->voxels;
   q.pool_cap = (uint32_t)v->cfg.pool_blocks;
   q.vox = v->cfg.vox_size;
+  q.inv_vox = 1.0 / (double)v->cfg.vox_size;
   return q;
 }
 
@@ -316,39 +319,43 @@ TrackArgs track_args(vh_volume* v) {
 // evaluations, each one launch that first takes the step from the previous evaluation (the
 // partial sums and states alternate between two buffers by evaluation parity), then the final
 // step, which leaves the best accepted pose in cand. partials: 2 x kGnGrid x kGnAcc doubles,
-// state: 2, stats: (iters + 1) rows.
+// state: 2, stats: (iters + 1) rows. With track, the points and the starting pose are the tracked
+// frame's, taken up by the first evaluation, and the final step writes the frame's pose and rows out.
 hipError_t enqueue_gn_evaluations(vh_volume* v, GnArgs g, int iters, double* partials, GnState* state, double* cand,
-                                  double* stats) {
+                                  double* stats, const TrackArgs* track = nullptr) {
   const int grid = gn_grid(g.n);
+  g.grid = grid;
   const size_t pstride = (size_t)kGnGrid * kGnAcc;
   g.pose = cand;
   for (int it = 0; it <= iters; ++it) {
     g.partials = partials + (it & 1) * pstride;
     g.prev_grid = it > 0 ? grid : 0;
+    g.track = track && it == 0;
+    if (g.track) g.t = *track;
     g.prev_partials = partials + ((it + 1) & 1) * pstride;
     g.st_in = state + ((it + 1) & 1);
     g.st_out = state + (it & 1);
     g.cand_out = nullptr;
     g.stats_row = it > 0 ? stats + kGnStats * (it - 1) : nullptr;
-    hipError_t e = launch_gn_accum(g, v->cfg.storage, grid, v->stream);
+    hipError_t e = launch_gn_accum(g, v->cfg.storage, v->stream);
     if (e != hipSuccess) return e;
   }
-  return launch_gn_solve(partials + (iters & 1) * pstride, grid, state + (iters & 1), state + ((iters + 1) & 1), cand,
-                         1, stats + kGnStats * iters, v->stream);
+  const double* last = partials + (iters & 1) * pstride;
+  GnState *in = state + (iters & 1), *out = state + ((iters + 1) & 1);
+  if (track) return launch_track_solve(last, grid, in, out, cand, *track, v->stream);
+  return launch_gn_solve(last, grid, in, out, cand, stats + kGnStats * iters, v->stream);
 }
 
 // Tracking part of a frame of the tracked sequence: back-projection, iters + 1 solver
 // evaluations and the final step, the pose write-out.
 int enqueue_track_kernels(vh_volume* v) {
   const TrackArgs t = track_args(v);
-  VH_HIP(launch_track_begin(t, v->stream));
   GnArgs g{};
   g.q = query_args(v);
   g.mu = v->cfg.trunc;
   g.pts = t.pts;
   g.n = (int64_t)t.pw * t.ph;
-  VH_HIP(enqueue_gn_evaluations(v, g, t.iters, v->gn_partials, v->gn_state, v->gn_pose, v->gn_stats));
-  VH_HIP(launch_track_end(t, v->stream));
+  VH_HIP(enqueue_gn_evaluations(v, g, t.iters, v->gn_partials, v->gn_state, v->gn_pose, v->gn_stats, &t));
   return VH_OK;
 }
 
@@ -1724,9 +1731,11 @@ int vh_query_sdf_backward_device(vh_volume* v, const float* d_pts, int64_t n, co
   if ((rc = ensure_gn_scratch(v))) return rc;
   float* d_T = v->bw_pose;
   VH_HIP(hipMemcpyAsync(d_T, c2w, 12 * sizeof(float), hipMemcpyHostToDevice, v->stream));
+  // one point per lane, up to kBackwardGrid workgroups (6 partial sums each)
+  const int grid = (int)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, kBackwardGrid));
   VH_HIP(launch_backward(query_args(v), v->cfg.storage, d_pts, n, d_T, d_grad_r, d_r, d_valid, d_J,
-                         d_pose_grad ? v->gn_partials : nullptr, kGnGrid, d_voxel_grad, v->stream));
-  if (d_pose_grad) VH_HIP(launch_reduce6(v->gn_partials, kGnGrid, d_pose_grad, v->stream));
+                         d_pose_grad ? v->gn_partials : nullptr, grid, d_voxel_grad, v->stream));
+  if (d_pose_grad) VH_HIP(launch_reduce6(v->gn_partials, grid, d_pose_grad, v->stream));
   // the scratch pose must outlive the kernels before the next call reuses it
   VH_HIP(hipStreamSynchronize(v->stream));
   return VH_OK;

@@ -272,6 +272,7 @@ struct QueryArgs {
   const void* voxels;
   uint32_t pool_cap;
   float vox;
+  double inv_vox;  // RN(1 / vox)
 };
 
 // Gauss-Newton accumulators: 21 (J^T W J upper) + 6 (J^T W r) + 1 (r^2) + 1 (valid samples) +
@@ -307,22 +308,6 @@ struct GnStart {
   double lambda;
 };
 
-struct GnArgs {
-  QueryArgs q;
-  float mu;           // truncation (metres): residual scale of the noise model
-  const float* pts;   // camera-frame points (a non-finite coordinate marks a point to skip)
-  int64_t n;
-  const double* pose; // without a previous evaluation: the pose to evaluate (12 doubles, 3x4)
-  double* partials;   // gridDim.x * kGnAcc
-  // the previous evaluation, stepped from at the start of the launch (prev_grid = 0: none)
-  const double* prev_partials;
-  int prev_grid;
-  const GnState* st_in;  // solver state before that step
-  GnState* st_out;       // after it (written by workgroup 0)
-  double* cand_out;      // the new candidate (workgroup 0), or null
-  double* stats_row;     // the previous evaluation's stats row (workgroup 0)
-};
-
 // Tracking over a bound sequence: frame f (the sequence cursor) starts Gauss-Newton from
 // prior[f] (or, with `increment` and f > 0, from out[f-1] * prior[f]), back-projects its
 // depth on a stride grid, and writes the accepted pose to out[f], which the frame's
@@ -347,6 +332,28 @@ struct TrackArgs {
   GnState* state;
   int32_t iters;
 };
+
+struct GnArgs {
+  QueryArgs q;
+  float mu;           // truncation (metres): residual scale of the noise model
+  const float* pts;   // camera-frame points (a non-finite coordinate marks a point to skip)
+  int64_t n;
+  const double* pose; // without a previous evaluation: the pose to evaluate (12 doubles, 3x4)
+  double* partials;   // grid * kGnAcc
+  int grid;           // partial sums of this evaluation
+  // the previous evaluation, stepped from at the start of the launch (prev_grid = 0: none)
+  const double* prev_partials;
+  int prev_grid;
+  const GnState* st_in;  // solver state before that step
+  GnState* st_out;       // after it (written by workgroup 0)
+  double* cand_out;      // the new candidate (workgroup 0), or null
+  double* stats_row;     // the previous evaluation's stats row (workgroup 0)
+  // the first evaluation of a tracked frame (track != 0): its points come from the frame's depth
+  // image and are stored to t.pts for the others, its pose is the frame's starting pose
+  int track;
+  TrackArgs t;
+};
+
 
 // launchers (vh_kernels.hip); all asynchronous on `st`
 // Allocation of the next k frames (one batch, 1 <= k <= kMaxBatch), then their integration.
@@ -383,15 +390,15 @@ hipError_t launch_backward(const QueryArgs& q, int storage, const float* pts, in
                            float* J, double* partials, int grid, float* voxel_grad,
                            hipStream_t st);
 hipError_t launch_reduce6(const double* partials, int grid, double* out6, hipStream_t st);
-hipError_t launch_gn_accum(const GnArgs& a, int storage, int grid, hipStream_t st);
+hipError_t launch_gn_accum(const GnArgs& a, int storage, hipStream_t st);
 hipError_t launch_gn_solve(const double* partials, int grid, const GnState* st_in, GnState* st_out, double* cand,
-                           int final_step, double* stats_row, hipStream_t st);
+                           double* stats_row, hipStream_t st);
+hipError_t launch_track_solve(const double* partials, int grid, const GnState* st_in, GnState* st_out, double* cand,
+                              const TrackArgs& t, hipStream_t st);
 // cand = s.pose, solver state cleared with damping s.lambda.
 hipError_t launch_gn_start(const GnStart& s, GnState* state, double* cand, hipStream_t st);
 // Gauss-Newton state reset + prior pose of the current frame, and the depth back-projection,
 // in one launch.
-hipError_t launch_track_begin(const TrackArgs& t, hipStream_t st);
 // Accepted pose (and the frame's solver stats) to the per-frame outputs.
-hipError_t launch_track_end(const TrackArgs& t, hipStream_t st);
 
 }  // namespace vh

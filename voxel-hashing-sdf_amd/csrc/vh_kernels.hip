@@ -2199,48 +2199,140 @@ __global__ __launch_bounds__(256) void k_st_place(StreamArgs a) {
 }
 
 // ============================================================================ queries
+// q = a / b, correctly rounded, from y = RN(1 / b): q0 = RN(a y) is within an ulp, a - q0 b is exact
+// under FMA, and RN(q0 + (a - q0 b) y) is the quotient (Markstein): 3
+// operations instead of the division's 11.
+__device__ __forceinline__ double quotient(double a, double b, double y) {
+  const double q0 = a * y;
+  return __builtin_fma(__builtin_fma(-q0, b, a), y, q0);
+}
+
+// The four keys of a bucket, as one pair of 16-byte loads.
+struct BucketKeys {
+  ulonglong2 k01, k23;
+};
+__device__ __forceinline__ BucketKeys load_bucket(const HashView& h, uint64_t b) {
+  const ulonglong2* bp = reinterpret_cast<const ulonglong2*>(h.keys + b * kSlotsPerBucket);
+  return {bp[0], bp[1]};
+}
+constexpr int kAbsent = -1, kElsewhere = -2;
+// Slot of the key in its home bucket; kAbsent when an empty slot ends the search there,
+// kElsewhere when the bucket is full of other keys (the search goes on in the next).
+__device__ __forceinline__ int match_bucket(const BucketKeys& k, uint64_t key) {
+  const uint64_t ks[4] = {k.k01.x, k.k01.y, k.k23.x, k.k23.y};
+  int slot = kElsewhere;
+#pragma unroll
+  for (int s = 3; s >= 0; --s) {
+    slot = ks[s] == kEmptyKey ? kAbsent : slot;
+    slot = ks[s] == key ? s : slot;
+  }
+  return slot;
+}
+
 // Trilinear sample of the normalised TSDF at world point q; false unless all 8 lattice
 // corners are allocated and observed. The lattice position q/vox and its cell fraction are
 // formed in FP64 (an FP32 q/vox at |q| ~ 3 m is off by ~2e-5 of a voxel), the blend runs in
 // FP32. vid/w receive the pool voxel ids and weights; g the gradient w.r.t. q.
+//
+// What bounds it: dependent memory round trips, and the L1's one cache line a cycle. The cell's
+// corners lie in one block, or in 2, 4 or 8 where it crosses block faces (a third of all cells, some
+// lane of nearly every wave). The lookups are made together in two stages, the cell's own block and
+// its neighbours across one face, then those across edges and the corner, each stage loading every
+// bucket before the first is looked at: with the voxels five round trips, where one lookup after
+// another took up to 18. The 8 corners come as 4 pairs. Solver evaluation of 300,000 points (FP32): 30.6
+// us with 8 voxel loads, 26.6 with pairs.
 template <int kStorage>
 __device__ __forceinline__ bool sample_sdf(const QueryArgs& q, double px, double py, double pz,
                                            float& sdf, float g[3], uint32_t vid[8], float w[8]) {
   using IO = VoxelIO<kStorage>;
   using Word = typename IO::Word;
   const double vox = (double)q.vox;
-  const double gxd = px / vox, gyd = py / vox, gzd = pz / vox;
+  const double gxd = quotient(px, vox, q.inv_vox), gyd = quotient(py, vox, q.inv_vox), gzd = quotient(pz, vox, q.inv_vox);
   if (!(fabs(gxd) < 8.0e6 && fabs(gyd) < 8.0e6 && fabs(gzd) < 8.0e6)) return false;
   const double flx = floor(gxd), fly = floor(gyd), flz = floor(gzd);
   const int ix = (int)flx, iy = (int)fly, iz = (int)flz;
   const float fx = (float)(gxd - flx), fy = (float)(gyd - fly), fz = (float)(gzd - flz);
   const Word* voxw = reinterpret_cast<const Word*>(q.voxels);
-  // the corners' blocks first (one lookup per distinct block), then all 8 voxel loads at
-  // once, then the weight tests: a test after each load would make every load wait for the
-  // one before it
-  uint64_t last_key = kEmptyKey;
-  uint32_t blk = kNoBlock;
+  // blocks by the faces crossed to reach them: bit 2 x, bit 1 y, bit 0 z
+  const int cross = (((ix & 7) == 7) << 2) | (((iy & 7) == 7) << 1) | ((iz & 7) == 7);
+  const uint64_t key0 = pack_key(ix >> 3, iy >> 3, iz >> 3);
+  const auto key_of = [&](int c) {
+    return key0 + ((uint64_t)((c >> 2) & 1) << (2 * kKeyBits)) + ((uint64_t)((c >> 1) & 1) << kKeyBits) + (uint64_t)(c & 1);
+  };
+  const auto needs = [&](int c) { return (cross & c) == c; };
+  uint32_t blk[8];
+  int elsewhere = 0;
+  constexpr int kStage[2][4] = {{0, 1, 2, 4}, {3, 5, 6, 7}};
+#pragma unroll
+  for (int st = 0; st < 2; ++st) {
+    BucketKeys bk[4];
+    uint64_t home[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = kStage[st][i];
+      blk[c] = kNoBlock;
+      if (needs(c)) {
+        home[i] = bucket_of(key_of(c), q.hash.log2_buckets);
+        bk[i] = load_bucket(q.hash, home[i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int c = kStage[st][i];
+      if (needs(c)) {
+        const int slot = match_bucket(bk[i], key_of(c));
+        if (slot >= 0) blk[c] = (uint32_t)q.hash.vals[home[i] * kSlotsPerBucket + slot];
+        elsewhere |= slot == kElsewhere ? 1 << c : 0;
+      }
+    }
+  }
+  while (elsewhere) {  // a home bucket full of other keys: the whole search
+    const int c = __ffs(elsewhere) - 1;
+    elsewhere &= elsewhere - 1;
+    const uint32_t found = find_block(q.hash, key_of(c));
+#pragma unroll
+    for (int k = 0; k < 8; ++k) blk[k] = k == c ? found : blk[k];
+  }
+  // a corner across no further face lies in the block without it
+  if (!(cross & 1)) { blk[1] = blk[0]; blk[3] = blk[2]; blk[5] = blk[4]; blk[7] = blk[6]; }
+  if (!(cross & 2)) { blk[2] = blk[0]; blk[3] = blk[1]; blk[6] = blk[4]; blk[7] = blk[5]; }
+  if (!(cross & 4)) { blk[4] = blk[0]; blk[5] = blk[1]; blk[6] = blk[2]; blk[7] = blk[3]; }
+  bool seen = true;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) seen = seen & (blk[k] < q.pool_cap);
+  if (!seen) return false;
 #pragma unroll
   for (int k = 0; k < 8; ++k) {
     const int cx = ix + (k >> 2), cy = iy + ((k >> 1) & 1), cz = iz + (k & 1);
-    const uint64_t key = pack_key(cx >> 3, cy >> 3, cz >> 3);
-    if (key != last_key) {
-      last_key = key;
-      blk = find_block(q.hash, key);
-      if (blk >= q.pool_cap) return false;
-    }
-    vid[k] = blk * kB3 + (uint32_t)((((cx & 7) * 8) + (cy & 7)) * 8 + (cz & 7));
+    vid[k] = blk[k] * kB3 + (uint32_t)((((cx & 7) * 8) + (cy & 7)) * 8 + (cz & 7));
   }
-  Word wd[8];
+  // z neighbours in one load (z is the fastest index of a block); where the cell crosses a z
+  // face the pair is the last of its row, and the neighbour's first voxel a load of its own
+  struct __attribute__((packed, aligned(sizeof(Word)))) Pair {
+    Word a, b;
+  };
+  const bool cross_z = (cross & 1) != 0;
+  Pair pair[4];
+  Word next[4];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) wd[k] = voxw[vid[k]];
+  for (int k = 0; k < 4; ++k) {
+    pair[k] = *reinterpret_cast<const Pair*>(voxw + (vid[2 * k] - (cross_z ? 1u : 0u)));
+    next[k] = IO::zero();
+  }
+  if (cross_z) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) next[k] = voxw[vid[2 * k + 1]];
+  }
   float s[8];
-  bool seen = true;
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    float wv;
-    IO::unpack(wd[k], s[k], wv);
-    seen = seen & (wv > 0.0f);
+  for (int k = 0; k < 4; ++k) {
+    float sa, wa, sb, wb, sn, wn;
+    IO::unpack(pair[k].a, sa, wa);
+    IO::unpack(pair[k].b, sb, wb);
+    IO::unpack(next[k], sn, wn);
+    s[2 * k] = cross_z ? sb : sa;
+    s[2 * k + 1] = cross_z ? sn : sb;
+    seen = seen & ((cross_z ? wb : wa) > 0.0f) & ((cross_z ? wn : wb) > 0.0f);
   }
   if (!seen) return false;
   trilinear_weights(fx, fy, fz, w);
@@ -2284,6 +2376,13 @@ __device__ __forceinline__ double shfl_xor_d(double v, int m) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
+__device__ __forceinline__ double shfl_d(double v, int src) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __shfl((int)(b & 0xffffffffll), src);
+  const int hi = __shfl((int)(b >> 32), src);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
 // Sums acc[0..N) over the workgroup (256 lanes) into out[0..N); fixed tree, deterministic.
 template <int N>
 __device__ __forceinline__ void wg_reduce_store(double (&acc)[N], double* out) {
@@ -2308,22 +2407,43 @@ __device__ __forceinline__ void wg_reduce_store(double (&acc)[N], double* out) {
   __syncthreads();
 }
 
-// Sums acc[0..N) (N <= 32) over the workgroup (256 lanes) into out[0..N) by recursive halving
+// Sums acc[0..N) (N <= 32) over each four waves of the workgroup by recursive halving
 // within each wave: at lane distance m = 32, 16, 8, 4, 2 every lane sends the half of its
 // values its partner (lane ^ m) keeps and adds the partner's half of its own, so the values
 // per lane halve each step (31 double exchanges instead of 6 per value); a last exchange at
-// distance 1 completes the wave's sums, which lane 2 i + 1 ... hold for value i; the four waves
-// are added in order. Fixed tree, deterministic.
+// distance 1 completes the wave's sums, which wave_sums stores in s_part; sum_of_four then adds
+// four waves' in order. Fixed tree, deterministic.
+//
+// The first two steps' exchanges are one instruction per word (v_permlane32_swap and
+// v_permlane16_swap hand one half of a register for the other half of another), no LDS permute and no
+// selects.
+template <int kDistance>
+__device__ __forceinline__ double exchange_add(double lower, double upper) {  // each lane's half, with its partner's part
+  const long long a = __double_as_longlong(lower), b = __double_as_longlong(upper);
+  const uint32_t w[2][2] = {{(uint32_t)a, (uint32_t)b}, {(uint32_t)(a >> 32), (uint32_t)(b >> 32)}};
+  uint32_t x[2], y[2];
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const auto r = kDistance == 32 ? __builtin_amdgcn_permlane32_swap(w[k][0], w[k][1], false, false)
+                                   : __builtin_amdgcn_permlane16_swap(w[k][0], w[k][1], false, false);
+    x[k] = r[0];
+    y[k] = r[1];
+  }
+  return __longlong_as_double((long long)((uint64_t)x[1] << 32 | x[0])) + __longlong_as_double((long long)((uint64_t)y[1] << 32 | y[0]));
+}
 template <int N>
-__device__ __forceinline__ void wg_reduce_store_rs(const double (&acc)[N], double* out) {
+__device__ __forceinline__ void wave_sums(const double (&acc)[N], double (&s_part)[32]) {
   static_assert(N <= 32, "at most 32 values");
-  __shared__ double s_part[4][32];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
   double v[32];
 #pragma unroll
   for (int k = 0; k < 32; ++k) v[k] = k < N ? acc[k] : 0.0;
 #pragma unroll
-  for (int h = 16; h >= 1; h >>= 1) {  // h values per lane after this step; distance 2h
+  for (int i = 0; i < 16; ++i) v[i] = exchange_add<32>(v[i], v[i + 16]);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = exchange_add<16>(v[i], v[i + 8]);
+#pragma unroll
+  for (int h = 4; h >= 1; h >>= 1) {  // h values per lane after this step; distance 2h
     const bool upper = (lane & (2 * h)) != 0;  // this lane keeps the upper half
 #pragma unroll
     for (int i = 0; i < h; ++i) {
@@ -2336,61 +2456,162 @@ __device__ __forceinline__ void wg_reduce_store_rs(const double (&acc)[N], doubl
   // value index of this lane: the halves it kept, from bit 5 (most significant) to bit 1
   const int idx = ((lane >> 5) & 1) * 16 + ((lane >> 4) & 1) * 8 + ((lane >> 3) & 1) * 4 + ((lane >> 2) & 1) * 2 +
                   ((lane >> 1) & 1);
-  if ((lane & 1) == 0) s_part[wave][idx] = total;
-  __syncthreads();
-  if (threadIdx.x < N) {
-    const int k = threadIdx.x;
-    out[k] = ((s_part[0][k] + s_part[1][k]) + s_part[2][k]) + s_part[3][k];
-  }
-  __syncthreads();
+  if ((lane & 1) == 0) s_part[idx] = total;
+}
+__device__ __forceinline__ double sum_of_four(const double (*s_part)[32], int k) {
+  return ((s_part[0][k] + s_part[1][k]) + s_part[2][k]) + s_part[3][k];
+}
+
+// The chunk of a list that a workgroup takes, so that the workgroups of one XCD (dispatched round
+// robin over 8) take neighbouring chunks and their blocks are fetched into one L2 instead of eight.
+__device__ __forceinline__ uint32_t xcd_chunk(uint32_t wg, uint32_t grid) {
+  const uint32_t xcd = wg & 7u, rest = grid & 7u;
+  return xcd * (grid >> 3) + (xcd < rest ? xcd : rest) + (wg >> 3);
 }
 
 // Residuals r_i = sdf(R p_i + t) and their derivatives with respect to a left se(3)
-// perturbation (rho, phi): dr/drho = grad, dr/dphi = q x grad.
+// perturbation (rho, phi): dr/drho = grad, dr/dphi = q x grad. Workgroup chunk c takes the points
+// [c per, (c + 1) per), per a multiple of 256.
+//
+// What bounds it: the voxel gradients' float atomics, which leave the XCD (a gradient row may be
+// written from any of them) as one request per cache line and instruction. A lane's own eight corners,
+// one instruction each, made 64 points' lines per instruction; the wave turns its 64 x 8
+// additions over in LDS, so that an instruction holds all eight corners of 8 neighbouring points,
+// which lie in two lines per point and mostly in their neighbours' too. 300,000 points of a frame
+// (FP16): 123 us with a lane's corners and points dealt out grid-wide, 59 so (2.19e6 atomic
+// requests, 9.8e5); adding up in an LDS hash set of the workgroup's lines first (7.8e5) took 65.
 template <int kStorage>
-__global__ __launch_bounds__(256) void k_backward(QueryArgs q, const float* pts, int64_t n, const float* T12,
+__global__ __launch_bounds__(256) void k_backward(QueryArgs q, const float* pts, int64_t n, int64_t per, const float* T12,
                                                   const float* grad_r, float* r_out, uint8_t* valid, float* J,
                                                   double* partials, float* voxel_grad) {
+  __shared__ float4 s_add[4][128];
+  __shared__ uint4 s_vid[4][128];
+  constexpr uint32_t kNoVoxel = 0xffffffffu;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t first = per * (int64_t)xcd_chunk(blockIdx.x, gridDim.x);
+  const int64_t end = first + per < n ? first + per : n;
   double acc[6] = {0, 0, 0, 0, 0, 0};
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    double qx, qy, qz;
-    pose_apply_d(T12, pts[3 * i], pts[3 * i + 1], pts[3 * i + 2], qx, qy, qz);
-    float r = 0.0f, g[3] = {0, 0, 0}, w[8];
+  for (int64_t base = first + 64 * wave; base < end; base += 256) {  // base: the wave's first point
+    const int64_t i = base + lane;
     uint32_t vid[8];
-    const bool ok = sample_sdf<kStorage>(q, qx, qy, qz, r, g, vid, w);
-    float j[6] = {0, 0, 0, 0, 0, 0};
-    if (ok) {
-      const double gx = g[0], gy = g[1], gz = g[2];
-      j[0] = g[0]; j[1] = g[1]; j[2] = g[2];
-      j[3] = (float)(qy * gz - qz * gy);
-      j[4] = (float)(qz * gx - qx * gz);
-      j[5] = (float)(qx * gy - qy * gx);
+    float add[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) vid[k] = kNoVoxel, add[k] = 0.0f;
+    if (i < end) {
+      double qx, qy, qz;
+      pose_apply_d(T12, pts[3 * i], pts[3 * i + 1], pts[3 * i + 2], qx, qy, qz);
+      float r = 0.0f, g[3] = {0, 0, 0}, w[8];
+      const bool ok = sample_sdf<kStorage>(q, qx, qy, qz, r, g, vid, w);
+      float j[6] = {0, 0, 0, 0, 0, 0};
+      if (ok) {
+        const double gx = g[0], gy = g[1], gz = g[2];
+        j[0] = g[0]; j[1] = g[1]; j[2] = g[2];
+        j[3] = (float)(qy * gz - qz * gy);
+        j[4] = (float)(qz * gx - qx * gz);
+        j[5] = (float)(qx * gy - qy * gx);
+      }
+      if (r_out) r_out[i] = ok ? r : 0.0f;
+      if (valid) valid[i] = ok ? 1 : 0;
+      if (J) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) J[6 * i + k] = j[k];
+      }
+      const float up = grad_r ? grad_r[i] : 0.0f;
+      if (ok) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) acc[k] += (double)up * (double)j[k];
+      }
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        if (ok) add[k] = up * w[k];
+        else vid[k] = kNoVoxel;
+      }
     }
-    if (r_out) r_out[i] = ok ? r : 0.0f;
-    if (valid) valid[i] = ok ? 1 : 0;
-    if (J) {
+    if (voxel_grad) {
+      wave_sync();  // the previous round's reads are issued
+      s_add[wave][2 * lane] = make_float4(add[0], add[1], add[2], add[3]);
+      s_add[wave][2 * lane + 1] = make_float4(add[4], add[5], add[6], add[7]);
+      s_vid[wave][2 * lane] = make_uint4(vid[0], vid[1], vid[2], vid[3]);
+      s_vid[wave][2 * lane + 1] = make_uint4(vid[4], vid[5], vid[6], vid[7]);
+      wave_sync();
 #pragma unroll
-      for (int k = 0; k < 6; ++k) J[6 * i + k] = j[k];
-    }
-    const float up = grad_r ? grad_r[i] : 0.0f;
-    if (ok && grad_r) {
-#pragma unroll
-      for (int k = 0; k < 6; ++k) acc[k] += (double)up * (double)j[k];
-      if (voxel_grad) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) atomicAdd(voxel_grad + vid[k], up * w[k]);
+      for (int k = 0; k < 8; ++k) {
+        const uint32_t v = reinterpret_cast<const uint32_t*>(s_vid[wave])[64 * k + lane];
+        const float a = reinterpret_cast<const float*>(s_add[wave])[64 * k + lane];
+        if (v != kNoVoxel) atomicAdd(voxel_grad + v, a);
       }
     }
   }
   if (partials) wg_reduce_store<6>(acc, partials + 6 * (size_t)blockIdx.x);
 }
 
-__global__ __launch_bounds__(64) void k_reduce6(const double* partials, int grid, double* out6) {
-  if (threadIdx.x < 6) {
-    double s = 0.0;
-    for (int g = 0; g < grid; ++g) s += partials[6 * (size_t)g + threadIdx.x];
-    out6[threadIdx.x] = s;
+// Sums the workgroups' partials, one wave per accumulator: each lane every 64th in order, then a
+// fixed tree (one lane per accumulator took 66 us over 512 partials).
+__global__ __launch_bounds__(384) void k_reduce6(const double* partials, int grid, double* out6) {
+  const int lane = threadIdx.x & 63, k = threadIdx.x >> 6;
+  double s = 0.0;
+#pragma unroll 8
+  for (int g = lane; g < grid; g += 64) s += partials[6 * (size_t)g + k];
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) s += shfl_xor_d(s, m);
+  if (lane == 0) out6[k] = s;
+}
+
+// ============================================================================ tracking
+__device__ __forceinline__ uint32_t track_slot(const TrackArgs& t) { return t.ctl->cursor[1] % t.n_seq; }
+
+// A tracked frame's starting pose, into s_pose (lanes 0..11 of every workgroup): with increments,
+// out[f-1] * prior[f] in FP64, each entry summed in column order ((a0 b0 + a1 b1) + a2 b2) +
+// a3 b3. Workgroup 0 makes it the candidate and clears the solver state (the first evaluation, not a
+// memset node, so the captured graph replays it exactly).
+__device__ __forceinline__ void track_start(const TrackArgs& t, uint32_t fs, double* s_pose) {
+  const int k = threadIdx.x;
+  const bool w0 = blockIdx.x == 0;
+  const float* P = t.prior + 16 * (size_t)fs;
+  if (k < 12) {
+    double p;
+    if (t.increment && fs > 0) {
+      const float* A = t.out + 16 * (size_t)(fs - 1);
+      const int r = k >> 2, c = k & 3;
+      p = (((double)A[4 * r] * (double)P[c] + (double)A[4 * r + 1] * (double)P[4 + c]) +
+           (double)A[4 * r + 2] * (double)P[8 + c]) + (double)A[4 * r + 3] * (double)P[12 + c];
+    } else {
+      p = (double)P[k];
+    }
+    s_pose[k] = p;
+    if (w0) {
+      t.pose[k] = p;
+      t.state->cand[k] = p;   // the first evaluation's pose
+      t.state->start[k] = p;  // the motion prior's centre
+    }
   }
+  if (w0 && k == 0) {  // no accepted pose yet (the other fields are set by the first acceptance)
+    t.state->has = 0;
+    t.state->lambda = 1e-4;
+    const double st = t.prior_sigma_t, sr = t.prior_sigma_r;
+    t.state->lam_t = st > 0.0 ? 1.0 / (st * st) : 0.0;
+    t.state->lam_r = sr > 0.0 ? 1.0 / (sr * sr) : 0.0;
+    t.state->n_eff = t.n_eff;
+  }
+}
+
+// Point i of a tracked frame: one stride-th pixel back-projected to the camera frame ((u - cx) d / fx,
+// (v - cy) d / fy, d) in FP32 with this operation order; a pixel without a valid depth gives
+// NaN (skipped by the solver). Stored for the frame's further evaluations.
+__device__ __forceinline__ void track_point(const TrackArgs& t, uint32_t fs, int i, float& x, float& y, float& z) {
+  const int u = (i % t.pw) * t.stride, v = (i / t.pw) * t.stride;
+  const size_t first = (size_t)fs * t.W * t.H;
+  const float d = t.depth_u16 ? depth_at<true>(reinterpret_cast<const uint16_t*>(t.depth) + first, t.depth_scale, v * t.W + u)
+                              : depth_at<false>(reinterpret_cast<const float*>(t.depth) + first, t.depth_scale, v * t.W + u);
+  x = y = z = __builtin_nanf("");
+  if (depth_valid(d, t.max_depth)) {
+    x = (((float)u - t.K.cx) * d) / t.K.fx;
+    y = (((float)v - t.K.cy) * d) / t.K.fy;
+    z = d;
+  }
+  t.pts[3 * i] = x;
+  t.pts[3 * i + 1] = y;
+  t.pts[3 * i + 2] = z;
 }
 
 // ============================================================================ Gauss-Newton
@@ -2409,66 +2630,178 @@ __device__ __forceinline__ double huber_weight(double e) {
 // q = R p + t and e = s r, the point adds W J J^T and W r J with W = huber_weight(e) s^2 (one
 // Gauss-Newton step of the iteratively reweighted problem), r^2, and rho(e) to the cost; a
 // point without a valid sample adds rho(s), the cost of a saturated residual r = 1.
-__device__ __forceinline__ void gn_solve_wg(const double* partials, int grid, const GnState* st_in, GnState* st_out, double* s_cand,
-                            double* cand_out, int final_step, double* stats_row);
-__device__ __forceinline__ void gn_step(const double* tot, GnState& S, double* s_cand, double* cand_out, int final_step,
-                                        double* stats_row);
+struct GnPoint {
+  float x, y, z;  // camera frame
+  float r, g[3];  // the sample at q
+};
+__device__ __forceinline__ GnPoint gn_load(const GnArgs& a, uint32_t fs, int64_t i) {
+  GnPoint p{};
+  if (a.track) {
+    track_point(a.t, fs, (int)i, p.x, p.y, p.z);
+  } else {
+    p.x = a.pts[3 * i];
+    p.y = a.pts[3 * i + 1];
+    p.z = a.pts[3 * i + 2];
+  }
+  return p;
+}
+// A non-finite coordinate (no depth at this pixel) leaves the point out.
+__device__ __forceinline__ bool gn_considered(const GnPoint& p) { return isfinite(p.x) && isfinite(p.y) && isfinite(p.z); }
+template <int kStorage>
+__device__ __forceinline__ bool gn_sample(const GnArgs& a, const double* pose, GnPoint& p) {
+  double qx, qy, qz;
+  pose_apply_d(pose, p.x, p.y, p.z, qx, qy, qz);
+  float w[8];
+  uint32_t vid[8];
+  return sample_sdf<kStorage>(a.q, qx, qy, qz, p.r, p.g, vid, w);
+}
+// acc: kGnAcc sums; counts [28] and [29] are whole numbers and exact.
+__device__ __forceinline__ void gn_add(const GnArgs& a, const double* pose, const GnPoint& p, bool ok, double (&acc)[kGnAcc]) {
+  acc[29] += 1.0;
+  const double zt = (double)p.z - 0.4;
+  const double sc = (double)a.mu / (0.0012 + 0.0019 * (zt * zt));
+  if (!ok) {
+    acc[30] += huber_rho(sc);
+    return;
+  }
+  double qx, qy, qz;
+  pose_apply_d(pose, p.x, p.y, p.z, qx, qy, qz);
+  const double rd = (double)p.r, e = sc * rd;
+  const double W = huber_weight(e) * sc * sc;
+  const double gx = p.g[0], gy = p.g[1], gz = p.g[2];
+  const double j[6] = {gx, gy, gz, qy * gz - qz * gy, qz * gx - qx * gz, qx * gy - qy * gx};
+  double wj[6];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) wj[c] = W * j[c];
+  int m = 0;
+#pragma unroll
+  for (int r = 0; r < 6; ++r)
+#pragma unroll
+    for (int c = r; c < 6; ++c) acc[m++] += wj[r] * j[c];
+#pragma unroll
+  for (int c = 0; c < 6; ++c) acc[21 + c] += wj[c] * rd;
+  acc[27] += rd * rd;
+  acc[28] += 1.0;
+  acc[30] += huber_rho(e);
+}
 
 // One evaluation. With a previous evaluation (prev_grid > 0) every workgroup first takes its
 // Levenberg-Marquardt step itself (gn_solve_wg over the previous partials: the same sums in
 // the same order, so every workgroup gets the same candidate; workgroup 0 stores the state,
 // the candidate and the stats row), which saves a launch per evaluation and needs no ordering
 // between workgroups; otherwise the candidate is a.pose.
-// Register budget: 3 waves per SIMD (154 VGPRs, no spills; the 31 FP64 sums and the robust
-// weighting of a point need more than the 128 of 4 waves, which spilled into the point loop).
-// The grid is at most 512 workgroups of 4 waves, so every wave of a launch is resident at once.
-template <int kStorage>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_gn_accum(GnArgs a) {
-  __shared__ double s_pose[12];
+//
+// Partial sum b of the a.grid is over the points b 256 + t (t < 256), and every a.grid 256th
+// after them, added in order per t. What bounds an evaluation is latency: of the step's serial FP64
+// chain and of the points' lookups. Two launch shapes (gn_shape):
+// - k_gn_accum, while each point has a lane of its own: a workgroup of 256 per partial sum, one point
+//   to a lane, loaded before the step; a fifth wave takes the motion prior's part of the step.
+// - k_gn_accum_wide above: 16 waves, two partial sums a workgroup, a workgroup per CU. All waves
+//   sample, 1,536 points at a time, into LDS, and 8 of them add those up in order; a sampling wave
+//   doesn't hold the 31 FP64 sums (62 registers), so twice as many lookups are in flight
+//   as with both in one loop.
+// Workgroups take neighbouring points by XCD (xcd_chunk): 300,000 points fetched 48 MB, now 19.
+// Measured, per evaluation: 19,200 points (F16) 12.4 -> 8.9 us, 300,000 (FP32) 35.0 -> 23.3 us;
+// 3.5 and 3.3 us of that by the step's shorter chain (gn_step) and the prior's own wave.
+struct GnStepOut {
+  GnState* st;
+  double *cand, *row;
+};
+__device__ __forceinline__ GnStepOut gn_step_out(const GnArgs& a) {
+  const bool w0 = blockIdx.x == 0;
+  return {w0 ? a.st_out : nullptr, w0 ? a.cand_out : nullptr, w0 ? a.stats_row : nullptr};
+}
+template <int kThreads>
+__device__ __forceinline__ void gn_solve_wg(const double* partials, int grid, const GnState* st_in, const GnStepOut& out,
+                                            double* s_cand, int final_step);
+template <int kThreads>
+__device__ __forceinline__ void gn_pose(const GnArgs& a, uint32_t fs, double* s_pose) {
   if (a.prev_grid > 0) {
-    const bool w0 = blockIdx.x == 0;
-    gn_solve_wg(a.prev_partials, a.prev_grid, a.st_in, w0 ? a.st_out : nullptr, s_pose, w0 ? a.cand_out : nullptr, 0,
-                w0 ? a.stats_row : nullptr);
-  } else {
-    if (threadIdx.x < 12) s_pose[threadIdx.x] = a.pose[threadIdx.x];
-    __syncthreads();
+    gn_solve_wg<kThreads>(a.prev_partials, a.prev_grid, a.st_in, gn_step_out(a), s_pose, 0);
+    return;
   }
-  double acc[kGnAcc];
+  if (a.track) track_start(a.t, fs, s_pose);
+  else if (threadIdx.x < 12) s_pose[threadIdx.x] = a.pose[threadIdx.x];
+  __syncthreads();
+}
+
+constexpr int kGnThreads = 320, kGnWideThreads = 1024;
+template <int kStorage>
+__global__ __launch_bounds__(kGnThreads) __attribute__((amdgpu_waves_per_eu(3))) void k_gn_accum(GnArgs a) {
+  __shared__ double s_pose[12];
+  __shared__ double s_part[4][32];
+  const int b = (int)xcd_chunk(blockIdx.x, gridDim.x), t = threadIdx.x;
+  const uint32_t fs = a.track ? track_slot(a.t) : 0u;
+  const int64_t i = b * (int64_t)256 + t;
+  const bool mine = t < 256 && i < a.n;
+  GnPoint p{};
+  if (mine) p = gn_load(a, fs, i);
+  gn_pose<kGnThreads>(a, fs, s_pose);
+  if (t < 256) {
+    double acc[kGnAcc];
 #pragma unroll
-  for (int k = 0; k < kGnAcc; ++k) acc[k] = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < a.n; i += (int64_t)gridDim.x * blockDim.x) {
-    const float px = a.pts[3 * i], py = a.pts[3 * i + 1], pz = a.pts[3 * i + 2];
-    if (!(isfinite(px) && isfinite(py) && isfinite(pz))) continue;  // no depth at this pixel
-    acc[29] += 1.0;
-    const double zt = (double)pz - 0.4;
-    const double sc = (double)a.mu / (0.0012 + 0.0019 * (zt * zt));
-    double qx, qy, qz;
-    pose_apply_d(s_pose, px, py, pz, qx, qy, qz);
-    float r, g[3], w[8];
-    uint32_t vid[8];
-    if (!sample_sdf<kStorage>(a.q, qx, qy, qz, r, g, vid, w)) {
-      acc[30] += huber_rho(sc);
-      continue;
+    for (int k = 0; k < kGnAcc; ++k) acc[k] = 0.0;
+    if (mine && gn_considered(p)) {
+      const bool ok = gn_sample<kStorage>(a, s_pose, p);
+      gn_add(a, s_pose, p, ok, acc);
     }
-    const double rd = (double)r, e = sc * rd;
-    const double W = huber_weight(e) * sc * sc;
-    const double gx = g[0], gy = g[1], gz = g[2];
-    const double j[6] = {gx, gy, gz, qy * gz - qz * gy, qz * gx - qx * gz, qx * gy - qy * gx};
-    double wj[6];
-#pragma unroll
-    for (int p = 0; p < 6; ++p) wj[p] = W * j[p];
-    int m = 0;
-#pragma unroll
-    for (int p = 0; p < 6; ++p)
-#pragma unroll
-      for (int c = p; c < 6; ++c) acc[m++] += wj[p] * j[c];
-#pragma unroll
-    for (int p = 0; p < 6; ++p) acc[21 + p] += wj[p] * rd;
-    acc[27] += rd * rd;
-    acc[28] += 1.0;
-    acc[30] += huber_rho(e);
+    wave_sums<kGnAcc>(acc, s_part[t >> 6]);
   }
-  wg_reduce_store_rs<kGnAcc>(acc, a.partials + kGnAcc * (size_t)blockIdx.x);
+  __syncthreads();
+  if (t < kGnAcc) a.partials[kGnAcc * (size_t)b + t] = sum_of_four(s_part, t);
+}
+
+template <int kStorage>
+__global__ __launch_bounds__(kGnWideThreads) void k_gn_accum_wide(GnArgs a) {
+  constexpr int kRounds = 3;  // points of a lane (of the 512 that add) sampled before they are added
+  enum : uint32_t { kSkip, kMiss, kHit };
+  __shared__ double s_pose[12];
+  __shared__ double s_part[8][32];
+  __shared__ float4 s_smp[kRounds * 512];  // r, g
+  __shared__ float4 s_pt[kRounds * 512];   // the point, and whether it was sampled
+  const int c = (int)xcd_chunk(blockIdx.x, gridDim.x), t = threadIdx.x;
+  const uint32_t fs = a.track ? track_slot(a.t) : 0u;
+  gn_pose<kGnWideThreads>(a, fs, s_pose);
+  // the sums between two turns: in memory by intent, or they'd take registers while sampling
+  volatile double held[kGnAcc];
+  const int64_t stride = a.grid * (int64_t)256;  // a.grid is even
+  for (int64_t first = c * (int64_t)512, turn = 0; turn == 0 || first < a.n; first += kRounds * stride, ++turn) {
+    for (int k = t; k < kRounds * 512; k += kGnWideThreads) {
+      const int64_t i = first + (k >> 9) * stride + (k & 511);
+      if (i >= a.n) break;
+      GnPoint p = gn_load(a, fs, i);
+      uint32_t hit = kSkip;
+      if (gn_considered(p)) hit = gn_sample<kStorage>(a, s_pose, p) ? kHit : kMiss;
+      s_smp[k] = make_float4(p.r, p.g[0], p.g[1], p.g[2]);
+      s_pt[k] = make_float4(p.x, p.y, p.z, __uint_as_float(hit));
+    }
+    __syncthreads();
+    if (t < 512) {
+      double acc[kGnAcc];
+#pragma unroll
+      for (int k = 0; k < kGnAcc; ++k) acc[k] = 0.0;
+      if (turn > 0) {
+#pragma unroll
+        for (int k = 0; k < kGnAcc; ++k) acc[k] = held[k];
+      }
+      for (int r = 0; r < kRounds; ++r) {
+        const int64_t i = first + r * stride + t;
+        if (i >= a.n) break;
+        const float4 m = s_pt[512 * r + t], s = s_smp[512 * r + t];
+        if (__float_as_uint(m.w) == kSkip) continue;
+        gn_add(a, s_pose, GnPoint{m.x, m.y, m.z, s.x, {s.y, s.z, s.w}}, __float_as_uint(m.w) == kHit, acc);
+      }
+      if (first + kRounds * stride >= a.n) {
+        wave_sums<kGnAcc>(acc, s_part[t >> 6]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < kGnAcc; ++k) held[k] = acc[k];
+      }
+    }
+    __syncthreads();  // the next points overwrite the samples
+  }
+  if (t < 512 && (t & 255) < kGnAcc)
+    a.partials[kGnAcc * (size_t)(2 * c + (t >> 8)) + (t & 255)] = sum_of_four(s_part + 4 * (t >> 8), t & 255);
 }
 
 // One workgroup, FP64: deterministic sum of the partials at the candidate pose, then a
@@ -2482,7 +2815,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 //   next candidate is exp(delta^) T_acc with (A + lambda diag(A)) delta = -b, A = J^T W J and
 //   b = J^T W r at the accepted pose, delta = (rho, phi), T <- exp(delta^) T.
 //   stats_row: [n_valid, rms, |delta|, lambda, accepted, accepted pose (12)].
-__device__ __forceinline__ void se3_left_update(const double* x, const double* pose, double* out) {
+// Entry k (< 12, row-major 3x4) of exp((rho, phi)^) pose, x = (rho, phi): one lane per entry.
+__device__ __forceinline__ double se3_left_update(const double* x, const double* pose, int k) {
   const double rho[3] = {x[0], x[1], x[2]}, ph[3] = {x[3], x[4], x[5]};
   const double th2 = ph[0] * ph[0] + ph[1] * ph[1] + ph[2] * ph[2];
   const double th = sqrt(th2);
@@ -2492,29 +2826,29 @@ __device__ __forceinline__ void se3_left_update(const double* x, const double* p
     B1 = 0.5 - th2 / 24.0;
     C1 = 1.0 / 6.0 - th2 / 120.0;
   } else {
-    A1 = sin(th) / th;
-    B1 = (1.0 - cos(th)) / th2;
-    C1 = (th - sin(th)) / (th2 * th);
+    double sn, cs;
+    sincos(th, &sn, &cs);
+    A1 = sn / th;
+    B1 = (1.0 - cs) / th2;
+    C1 = (th - sn) / (th2 * th);
   }
   const double K[3][3] = {{0.0, -ph[2], ph[1]}, {ph[2], 0.0, -ph[0]}, {-ph[1], ph[0], 0.0}};
-  double K2[3][3], R[3][3], V[3][3];
-  for (int p = 0; p < 3; ++p)
-    for (int c = 0; c < 3; ++c) {
-      double acc = 0.0;
-      for (int k = 0; k < 3; ++k) acc += K[p][k] * K[k][c];
-      K2[p][c] = acc;
-    }
-  for (int p = 0; p < 3; ++p)
-    for (int c = 0; c < 3; ++c) {
-      const double I = p == c ? 1.0 : 0.0;
-      R[p][c] = I + A1 * K[p][c] + B1 * K2[p][c];
-      V[p][c] = I + B1 * K[p][c] + C1 * K2[p][c];
-    }
-  for (int p = 0; p < 3; ++p) {
-    for (int c = 0; c < 3; ++c) out[4 * p + c] = R[p][0] * pose[c] + R[p][1] * pose[4 + c] + R[p][2] * pose[8 + c];
-    out[4 * p + 3] = R[p][0] * pose[3] + R[p][1] * pose[7] + R[p][2] * pose[11] +
-                     (V[p][0] * rho[0] + V[p][1] * rho[1] + V[p][2] * rho[2]);
+  const int p = k >> 2, c = k & 3;
+  double Kp[3];  // row p
+#pragma unroll
+  for (int q = 0; q < 3; ++q) Kp[q] = p == 0 ? K[0][q] : p == 1 ? K[1][q] : K[2][q];
+  double R[3], V[3];  // row p of both
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    double k2 = 0.0;
+#pragma unroll
+    for (int m = 0; m < 3; ++m) k2 += Kp[m] * K[m][q];
+    const double I = p == q ? 1.0 : 0.0;
+    R[q] = I + A1 * Kp[q] + B1 * k2;
+    V[q] = I + B1 * Kp[q] + C1 * k2;
   }
+  const double turned = R[0] * pose[c] + R[1] * pose[4 + c] + R[2] * pose[8 + c];
+  return c < 3 ? turned : turned + (V[0] * rho[0] + V[1] * rho[1] + V[2] * rho[2]);
 }
 
 // Motion prior of a tracked frame at pose T (row-major 3x4): xi = log(S^-1 T) with S the
@@ -2590,149 +2924,187 @@ __device__ __forceinline__ void motion_prior(const GnState& S, double* Ab, doubl
   Ab[26] += (tv[0] * g[1] - tv[1] * g[0]) + gr[2];
 }
 
-// The partials are summed by 248 lanes at once: lane (v, j) (v < kGnAcc, j < 8) sums
-// accumulator v over the workgroups g = j, j + 8, ... in order, then lanes v < kGnAcc add the 8
-// sums in a fixed tree, so every workgroup gets the same sums in the same order. Meanwhile
-// lanes below the state's size stage the solver state in LDS, so the step (one lane) reads it
-// from there. All 256 lanes call it; the new candidate is in s_cand on return. st_out,
-// cand_out and stats_row (global, each may be null) receive the new state, the candidate and
-// the evaluation's row.
-__device__ __forceinline__ void gn_solve_wg(const double* partials, int grid, const GnState* st_in, GnState* st_out, double* s_cand,
-                            double* cand_out, int final_step, double* stats_row) {
-  constexpr int kWays = 8, kStateWords = (int)(sizeof(GnState) / sizeof(double));
-  static_assert(kWays * kGnAcc <= 256 && kStateWords <= 256 && sizeof(GnState) % sizeof(double) == 0, "layout");
-  __shared__ double s_sum[kWays][kGnAcc];
-  __shared__ double tot[kGnAcc];
-  __shared__ double s_st[kStateWords];
-  const int t = threadIdx.x;
-  if (t < kStateWords) s_st[t] = reinterpret_cast<const double*>(st_in)[t];
-  if (t < kWays * kGnAcc) {
-    const int v = t % kGnAcc, j = t / kGnAcc;
-    // in order g = j, j + 8, ...; the loads of 8 terms in flight together, then their sum
-    double acc = 0.0;
-    int g = j;
-    for (; g + 7 * kWays < grid; g += 8 * kWays) {
-      double p[8];
-#pragma unroll
-      for (int r = 0; r < 8; ++r) p[r] = partials[kGnAcc * (size_t)(g + r * kWays) + v];
-#pragma unroll
-      for (int r = 0; r < 8; ++r) acc += p[r];
-    }
-    for (; g < grid; g += kWays) acc += partials[kGnAcc * (size_t)g + v];
-    s_sum[j][v] = acc;
-  }
-  __syncthreads();
-  if (t < kGnAcc)
-    tot[t] = ((s_sum[0][t] + s_sum[1][t]) + (s_sum[2][t] + s_sum[3][t])) +
-             ((s_sum[4][t] + s_sum[5][t]) + (s_sum[6][t] + s_sum[7][t]));
-  __syncthreads();
-  if (t == 0) gn_step(tot, *reinterpret_cast<GnState*>(s_st), s_cand, cand_out, final_step, stats_row);
-  __syncthreads();
-  if (st_out && t < kStateWords) reinterpret_cast<double*>(st_out)[t] = s_st[t];
-}
+struct GnPrior {
+  double Ab[27], cost;  // what the motion prior adds to A, b and the cost
+};
 
-// The Levenberg-Marquardt decision and step of one evaluation (one lane), on the solver state
-// staged in LDS (updated in place; the workgroup writes it out afterwards).
-__device__ __forceinline__ void gn_step(const double* tot, GnState& S, double* s_cand, double* cand_out, int final_step,
-                                        double* stats_row) {
-  double c[12], row[kGnStats];
+// The Levenberg-Marquardt decision and step of one evaluation by one wave, on the solver state
+// staged in LDS (updated in place; the workgroup writes it out afterwards). One lane's serial chain
+// set its time (of an evaluation of 19,200 points, 4.3 us of 9.6), at an instruction every few cycles: so what is per entry (the matrix and
+// pose kept, the update of the pose, the outputs) goes one lane per entry, the rest is computed by all
+// lanes alike, and the triangular solves divide by a pivot through its reciprocal, taken once (quotient).
+__device__ __forceinline__ void gn_step(const double* tot, const GnPrior& prior, GnState& S, double* s_cand,
+                                        const GnStepOut& out, int final_step) {
+  const int lane = threadIdx.x & 63;
   const double cnt = tot[28];
   // tracking: depth term scaled to n_eff points, plus the motion prior
   const double al = S.n_eff > 0.0 && tot[29] > 0.0 ? S.n_eff / tot[29] : 1.0;
-  double cost = al * tot[30], Ab[27];
-#pragma unroll
-  for (int k = 0; k < 27; ++k) Ab[k] = al * tot[k];
-  if (S.lam_t > 0.0 || S.lam_r > 0.0) motion_prior(S, Ab, cost);
-  row[0] = cnt;
-  row[1] = cnt > 0.0 ? sqrt(tot[27] / cnt) : 0.0;
-  row[2] = 0.0;
-  const bool accept = !S.has || cost <= S.cost;
+  const double cost = al * tot[30] + prior.cost;
+  const bool had = S.has != 0;
+  const bool accept = !had || cost <= S.cost;
+  const double lambda = !accept ? fmin(S.lambda * 4.0, 1e9) : had ? fmax(S.lambda / 3.0, 1e-9) : S.lambda;
+  wave_sync();  // every lane has the state it decides on
   if (accept) {
-#pragma unroll
-    for (int k = 0; k < 12; ++k) S.pose[k] = S.cand[k];  // the pose this evaluation was made at
-#pragma unroll
-    for (int k = 0; k < 27; ++k) S.Ab[k] = Ab[k];
-    S.cost = cost;
-    S.lambda = S.has ? fmax(S.lambda / 3.0, 1e-9) : S.lambda;
-    S.has = 1;
-  } else {
-    S.lambda = fmin(S.lambda * 4.0, 1e9);
+    if (lane < 12) S.pose[lane] = S.cand[lane];  // the pose this evaluation was made at
+    if (lane < 27) S.Ab[lane] = al * tot[lane] + prior.Ab[lane];
+    if (lane == 0) {
+      S.cost = cost;
+      S.has = 1;
+    }
   }
-  row[3] = S.lambda;
-  row[4] = accept ? 1.0 : 0.0;
-#pragma unroll
-  for (int k = 0; k < 12; ++k) row[5 + k] = S.pose[k];
-  // damped normal equations, Cholesky, the two triangular solves (all loops unrolled: the
-  // matrices stay in registers); a matrix that is not positive definite proposes the
-  // accepted pose again
-  double A[6][6], b[6], L[6][6], x[6], y[6];
+  if (lane == 0) S.lambda = lambda;
+  wave_sync();
+  // damped normal equations, Cholesky (in the lower triangle of A, with the forward
+  // substitution), back substitution (all loops unrolled: the matrix stays in registers); a
+  // matrix that is not positive definite proposes the accepted pose again
+  double A[6][6], inv[6], x[6], y[6];
 #pragma unroll
   for (int p = 0, m = 0; p < 6; ++p)
 #pragma unroll
-    for (int q = p; q < 6; ++q, ++m) { A[p][q] = S.Ab[m]; A[q][p] = S.Ab[m]; }
+    for (int q = p; q < 6; ++q, ++m) A[q][p] = S.Ab[m];
 #pragma unroll
-  for (int p = 0; p < 6; ++p) {
-    b[p] = -S.Ab[21 + p];
-    A[p][p] += S.lambda * A[p][p] + 1e-12;
-  }
+  for (int p = 0; p < 6; ++p) A[p][p] += lambda * A[p][p] + 1e-12;
   bool pd = true;
 #pragma unroll
   for (int q = 0; q < 6; ++q) {
     double d = A[q][q];
 #pragma unroll
-    for (int k = 0; k < q; ++k) d -= L[q][k] * L[q][k];
+    for (int k = 0; k < q; ++k) d -= A[q][k] * A[q][k];
     pd = pd && d > 0.0;
-    L[q][q] = sqrt(d);
+    A[q][q] = sqrt(d);
+    inv[q] = 1.0 / A[q][q];
 #pragma unroll
     for (int p = q + 1; p < 6; ++p) {
       double a = A[p][q];
 #pragma unroll
-      for (int k = 0; k < q; ++k) a -= L[p][k] * L[q][k];
-      L[p][q] = a / L[q][q];
+      for (int k = 0; k < q; ++k) a -= A[p][k] * A[q][k];
+      A[p][q] = quotient(a, A[q][q], inv[q]);
     }
-  }
+    double a = -S.Ab[21 + q];
 #pragma unroll
-  for (int p = 0; p < 6; ++p) {
-    double a = b[p];
-#pragma unroll
-    for (int k = 0; k < p; ++k) a -= L[p][k] * y[k];
-    y[p] = a / L[p][p];
+    for (int k = 0; k < q; ++k) a -= A[q][k] * y[k];
+    y[q] = quotient(a, A[q][q], inv[q]);
   }
 #pragma unroll
   for (int p = 5; p >= 0; --p) {
     double a = y[p];
 #pragma unroll
-    for (int k = p + 1; k < 6; ++k) a -= L[k][p] * x[k];
-    x[p] = a / L[p][p];
+    for (int k = p + 1; k < 6; ++k) a -= A[k][p] * x[k];
+    x[p] = quotient(a, A[p][p], inv[p]);
   }
-  if (!final_step && pd) {
-    se3_left_update(x, S.pose, c);
-    row[2] = sqrt(x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3] + x[4] * x[4] + x[5] * x[5]);
-  } else {
-#pragma unroll
-    for (int k = 0; k < 12; ++k) c[k] = S.pose[k];
+  const bool step = !final_step && pd;
+  if (lane < 12) {
+    const double c = step ? se3_left_update(x, S.pose, lane) : S.pose[lane];
+    s_cand[lane] = c;
+    if (out.cand) out.cand[lane] = c;
   }
-#pragma unroll
-  for (int k = 0; k < 12; ++k) {
-    S.cand[k] = c[k];
-    s_cand[k] = c[k];
+  if (out.row && lane < kGnStats) {
+    const double sq = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3] + x[4] * x[4] + x[5] * x[5];
+    const double root = sqrt(lane == 1 ? tot[27] / cnt : sq);
+    const double head = lane == 0 ? cnt : lane == 1 ? (cnt > 0.0 ? root : 0.0) : lane == 2 ? (step ? root : 0.0)
+                        : lane == 3 ? lambda : accept ? 1.0 : 0.0;
+    out.row[lane] = lane < 5 ? head : S.pose[lane < 5 ? 0 : lane - 5];
   }
-  if (cand_out) {
-#pragma unroll
-    for (int k = 0; k < 12; ++k) cand_out[k] = c[k];
-  }
-  if (stats_row) {
-#pragma unroll
-    for (int k = 0; k < kGnStats; ++k) stats_row[k] = row[k];
-  }
+  wave_sync();  // the accepted pose is read
+  if (lane < 12) S.cand[lane] = s_cand[lane];
 }
 
-// The last evaluation's step alone (one workgroup): with final_step the accepted pose is the
-// candidate written to cand.
-__global__ __launch_bounds__(256) void k_gn_solve(const double* partials, int grid, const GnState* st_in,
-                                                  GnState* st_out, double* cand, int final_step, double* stats_row) {
+// All kThreads lanes call it. Accumulator v's sum over the partials g = j, j + 8, ... in order is a
+// term (v, j), v < kGnAcc, j < 8; then one lane per v adds its 8 terms in a fixed tree, so every
+// workgroup gets the same sums in the same order. kThreads = 320: a lane per term, 16 loads in
+// flight; 1,024: four lanes (16 apart) per term, each with a quarter of its partials in flight
+// at once, their sums continued from quarter to quarter. Lanes below the state's size stage the
+// solver state in LDS, the last wave computes the motion prior's terms, which need only the
+// candidate, and the first wave takes the step (gn_step). The new candidate is in s_cand on return;
+// out's pointers (global, each may be null) receive the new state, the candidate and the evaluation's row.
+template <int kThreads>
+__device__ __forceinline__ void gn_solve_wg(const double* partials, int grid, const GnState* st_in, const GnStepOut& out,
+                                            double* s_cand, int final_step) {
+  constexpr int kWays = 8, kTerms = kWays * kGnAcc, kStateWords = (int)(sizeof(GnState) / sizeof(double));
+  static_assert(kTerms <= 256 && kStateWords <= 256 && sizeof(GnState) % sizeof(double) == 0, "layout");
+  static_assert(kThreads == kGnThreads || kThreads == kGnWideThreads, "one lane per term, or four");
+  constexpr int kFlight = 16;
+  __shared__ double s_sum[kTerms];
+  __shared__ double tot[kGnAcc];
+  __shared__ double s_st[kStateWords];
+  __shared__ GnPrior s_prior;
+  const int t = threadIdx.x, lane = t & 63;
+  if (t < kStateWords) s_st[t] = reinterpret_cast<const double*>(st_in)[t];
+  const auto load = [&](double (&p)[kFlight], int term, int r0) {  // the term's partials r0, r0 + 1, ...
+#pragma unroll
+    for (int r = 0; r < kFlight; ++r) {
+      const int g = (r0 + r) * kWays + term / kGnAcc;
+      p[r] = 0.0;
+      if (g < grid) p[r] = partials[kGnAcc * (size_t)g + term % kGnAcc];
+    }
+  };
+  const auto add = [&](double s, const double (&p)[kFlight]) {  // 0.0 beyond the grid leaves a sum as it is
+#pragma unroll
+    for (int r = 0; r < kFlight; ++r) s += p[r];
+    return s;
+  };
+  double p[kFlight];
+  if constexpr (kThreads == kGnThreads) {
+    if (t < kTerms) {
+      double s = 0.0;
+      for (int r0 = 0; r0 * kWays < grid; r0 += kFlight) {
+        load(p, t, r0);
+        s = add(s, p);
+      }
+      s_sum[t] = s;
+    }
+  } else {
+    const int term = 16 * (t >> 6) + (lane & 15), quarter = lane >> 4;
+    if (term < kTerms) {
+      load(p, term, kFlight * quarter);
+      double s = add(0.0, p);
+#pragma unroll
+      for (int k = 1; k < 4; ++k) {
+        const double before = shfl_d(s, (lane & 15) + 16 * (k - 1));
+        const double next = add(before, p);
+        s = quarter == k ? next : s;
+      }
+      if (quarter == 3) s_sum[term] = s;
+    }
+  }
+  if (t == kThreads - 1) {
+    GnPrior pr{};
+    if (st_in->lam_t > 0.0 || st_in->lam_r > 0.0) motion_prior(*st_in, pr.Ab, pr.cost);
+    s_prior = pr;
+  }
+  __syncthreads();
+  if (t < kGnAcc) {
+    const double* s = s_sum + t;
+    tot[t] = ((s[0] + s[kGnAcc]) + (s[2 * kGnAcc] + s[3 * kGnAcc])) +
+             ((s[4 * kGnAcc] + s[5 * kGnAcc]) + (s[6 * kGnAcc] + s[7 * kGnAcc]));
+  }
+  __syncthreads();
+  if (t < 64) gn_step(tot, s_prior, *reinterpret_cast<GnState*>(s_st), s_cand, out, final_step);
+  __syncthreads();
+  if (out.st && t < kStateWords) reinterpret_cast<double*>(out.st)[t] = s_st[t];
+}
+
+// The last evaluation's step alone (one workgroup): the accepted pose is the candidate written to cand.
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void k_gn_solve(const double* partials, int grid, const GnState* st_in,
+                                                       GnState* st_out, double* cand, double* stats_row) {
   __shared__ double s_cand[12];
-  gn_solve_wg(partials, grid, st_in, st_out, s_cand, cand, final_step, stats_row);
+  gn_solve_wg<kThreads>(partials, grid, st_in, GnStepOut{st_out, cand, stats_row}, s_cand, 1);
+}
+
+// A tracked frame's: the accepted pose, rounded to FP32, is the frame's pose; the solver's rows of
+// this frame go to the per-frame stats.
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void k_track_solve(const double* partials, int grid, const GnState* st_in,
+                                                          GnState* st_out, double* cand, TrackArgs t) {
+  __shared__ double s_cand[12];
+  const uint32_t fs = track_slot(t);
+  const int k = threadIdx.x, before = t.iters * kGnStats;  // the earlier evaluations' rows are there
+  double* rows = t.stats ? t.stats + (size_t)fs * (before + kGnStats) : nullptr;
+  if (rows)
+    for (int j = k; j < before; j += kThreads) rows[j] = t.eval_stats[j];
+  gn_solve_wg<kThreads>(partials, grid, st_in, GnStepOut{st_out, cand, rows ? rows + before : nullptr}, s_cand, 1);
+  if (k < 16) t.out[16 * (size_t)fs + k] = k < 12 ? (float)s_cand[k] : (k == 15 ? 1.0f : 0.0f);
 }
 
 // Start of a refinement: the candidate is the starting pose and the solver state is cleared
@@ -2748,77 +3120,6 @@ __global__ __launch_bounds__(64) void k_gn_start(GnStart s, GnState* st, double*
     *st = z;
   }
   if (k < 12) cand[k] = s.pose[k];
-}
-
-// ============================================================================ tracking
-__device__ __forceinline__ uint32_t track_slot(const TrackArgs& t) { return t.ctl->cursor[1] % t.n_seq; }
-
-// The frame's starting pose becomes the candidate; the solver state is cleared (a kernel,
-// not a memset node, so the captured graph replays it exactly). With increments, start =
-// out[f-1] * prior[f] in FP64, each entry summed in column order ((a0 b0 + a1 b1) + a2 b2) +
-// a3 b3. Lanes 0..11 of workgroup 0 of k_track_begin.
-__device__ void track_start(const TrackArgs& t, uint32_t fs) {
-  const int k = threadIdx.x;
-  const float* P = t.prior + 16 * (size_t)fs;
-  if (k < 12) {
-    double p;
-    if (t.increment && fs > 0) {
-      const float* A = t.out + 16 * (size_t)(fs - 1);
-      const int r = k >> 2, c = k & 3;
-      p = (((double)A[4 * r] * (double)P[c] + (double)A[4 * r + 1] * (double)P[4 + c]) +
-           (double)A[4 * r + 2] * (double)P[8 + c]) + (double)A[4 * r + 3] * (double)P[12 + c];
-    } else {
-      p = (double)P[k];
-    }
-    t.pose[k] = p;
-    t.state->cand[k] = p;   // the first evaluation's pose
-    t.state->start[k] = p;  // the motion prior's centre
-  }
-  if (k == 0) {  // no accepted pose yet (the other fields are set by the first acceptance)
-    t.state->has = 0;
-    t.state->lambda = 1e-4;
-    const double st = t.prior_sigma_t, sr = t.prior_sigma_r;
-    t.state->lam_t = st > 0.0 ? 1.0 / (st * st) : 0.0;
-    t.state->lam_r = sr > 0.0 ? 1.0 / (sr * sr) : 0.0;
-    t.state->n_eff = t.n_eff;
-  }
-}
-
-// Start of a tracked frame: workgroup 0 sets the starting pose (track_start), and every lane
-// back-projects one stride-th pixel to its camera-frame point ((u - cx) d / fx,
-// (v - cy) d / fy, d) in FP32 with this operation order; pixels without a valid depth give
-// NaN (skipped by the solver).
-template <bool kU16>
-__global__ __launch_bounds__(256) void k_track_begin(TrackArgs t) {
-  const uint32_t fs = track_slot(t);
-  if (blockIdx.x == 0) track_start(t, fs);
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= t.pw * t.ph) return;
-  const int u = (i % t.pw) * t.stride, v = (i / t.pw) * t.stride;
-  const size_t elem = kU16 ? 2 : 4;
-  const void* base = reinterpret_cast<const char*>(t.depth) + (size_t)fs * t.W * t.H * elem;
-  const float d = depth_at<kU16>(base, t.depth_scale, v * t.W + u);
-  float x = __builtin_nanf(""), y = x, z = x;
-  if (depth_valid(d, t.max_depth)) {
-    x = (((float)u - t.K.cx) * d) / t.K.fx;
-    y = (((float)v - t.K.cy) * d) / t.K.fy;
-    z = d;
-  }
-  t.pts[3 * i] = x;
-  t.pts[3 * i + 1] = y;
-  t.pts[3 * i + 2] = z;
-}
-
-// One workgroup: the accepted pose (the candidate after the final step), rounded to FP32, is
-// the frame's pose; the solver's rows of this frame go to the per-frame stats.
-__global__ __launch_bounds__(64) void k_track_end(TrackArgs t) {
-  const uint32_t fs = track_slot(t);
-  const int k = threadIdx.x;
-  if (k < 16) t.out[16 * (size_t)fs + k] = k < 12 ? (float)t.pose[k] : (k == 15 ? 1.0f : 0.0f);
-  if (t.stats) {
-    const int rows = (t.iters + 1) * kGnStats;
-    for (int j = k; j < rows; j += 64) t.stats[(size_t)fs * rows + j] = t.eval_stats[j];
-  }
 }
 
 }  // namespace
@@ -2993,46 +3294,45 @@ hipError_t launch_query(const QueryArgs& q, int storage, const float* pts, int64
 hipError_t launch_backward(const QueryArgs& q, int storage, const float* pts, int64_t n, const float* T12,
                            const float* grad_r, float* r, uint8_t* valid, float* J, double* partials, int grid,
                            float* voxel_grad, hipStream_t st) {
+  const int64_t per = ((n + grid - 1) / grid + 255) / 256 * 256;
   with_storage(storage, [&](auto S) {
-    hipLaunchKernelGGL(k_backward<decltype(S)::value>, dim3(grid), dim3(256), 0, st, q, pts, n, T12, grad_r, r,
+    hipLaunchKernelGGL(k_backward<decltype(S)::value>, dim3(grid), dim3(256), 0, st, q, pts, n, per, T12, grad_r, r,
                        valid, J, partials, voxel_grad);
   });
   return hipGetLastError();
 }
 
 hipError_t launch_reduce6(const double* partials, int grid, double* out6, hipStream_t st) {
-  hipLaunchKernelGGL(k_reduce6, dim3(1), dim3(64), 0, st, partials, grid, out6);
+  hipLaunchKernelGGL(k_reduce6, dim3(1), dim3(384), 0, st, partials, grid, out6);
   return hipGetLastError();
 }
 
-hipError_t launch_gn_accum(const GnArgs& a, int storage, int grid, hipStream_t st) {
+hipError_t launch_gn_accum(const GnArgs& a, int storage, hipStream_t st) {
   with_storage(storage, [&](auto S) {
-    hipLaunchKernelGGL(k_gn_accum<decltype(S)::value>, dim3(grid), dim3(256), 0, st, a);
+    constexpr int kS = decltype(S)::value;
+    if (a.n <= 256 * (int64_t)a.grid) hipLaunchKernelGGL(k_gn_accum<kS>, dim3(a.grid), dim3(kGnThreads), 0, st, a);
+    else hipLaunchKernelGGL(k_gn_accum_wide<kS>, dim3(a.grid / 2), dim3(kGnWideThreads), 0, st, a);
   });
   return hipGetLastError();
 }
 
+// 128 partials: one round of loads for a lane per term.
 hipError_t launch_gn_solve(const double* partials, int grid, const GnState* st_in, GnState* st_out, double* cand,
-                           int final_step, double* stats_row, hipStream_t st) {
-  hipLaunchKernelGGL(k_gn_solve, dim3(1), dim3(256), 0, st, partials, grid, st_in, st_out, cand, final_step, stats_row);
+                           double* stats_row, hipStream_t st) {
+  if (grid <= 128) hipLaunchKernelGGL(k_gn_solve<kGnThreads>, dim3(1), dim3(kGnThreads), 0, st, partials, grid, st_in, st_out, cand, stats_row);
+  else hipLaunchKernelGGL(k_gn_solve<kGnWideThreads>, dim3(1), dim3(kGnWideThreads), 0, st, partials, grid, st_in, st_out, cand, stats_row);
+  return hipGetLastError();
+}
+
+hipError_t launch_track_solve(const double* partials, int grid, const GnState* st_in, GnState* st_out, double* cand,
+                              const TrackArgs& t, hipStream_t st) {
+  if (grid <= 128) hipLaunchKernelGGL(k_track_solve<kGnThreads>, dim3(1), dim3(kGnThreads), 0, st, partials, grid, st_in, st_out, cand, t);
+  else hipLaunchKernelGGL(k_track_solve<kGnWideThreads>, dim3(1), dim3(kGnWideThreads), 0, st, partials, grid, st_in, st_out, cand, t);
   return hipGetLastError();
 }
 
 hipError_t launch_gn_start(const GnStart& s, GnState* state, double* cand, hipStream_t st) {
   hipLaunchKernelGGL(k_gn_start, dim3(1), dim3(64), 0, st, s, state, cand);
-  return hipGetLastError();
-}
-
-hipError_t launch_track_begin(const TrackArgs& t, hipStream_t st) {
-  const int n = t.pw * t.ph;
-  const dim3 g((n + 255) / 256), b(256);
-  if (t.depth_u16) hipLaunchKernelGGL(k_track_begin<true>, g, b, 0, st, t);
-  else hipLaunchKernelGGL(k_track_begin<false>, g, b, 0, st, t);
-  return hipGetLastError();
-}
-
-hipError_t launch_track_end(const TrackArgs& t, hipStream_t st) {
-  hipLaunchKernelGGL(k_track_end, dim3(1), dim3(64), 0, st, t);
   return hipGetLastError();
 }
 
