@@ -113,7 +113,11 @@ struct vh_volume {
   FrameCtl* ctl = nullptr;
   // staged host input (one frame, both formats) and its pose
   void* stage_depth = nullptr;
-  float* stage_pose = nullptr;
+  float* stage_pose = nullptr;   // 16, directly before stage_depth (one allocation)
+  // page-locked copies of callers' pageable images (host_image), allocated when the first one comes:
+  // vh_integrate's pose, depth and colours; per ring slot the depth and colours
+  char* stage_host = nullptr;
+  char* ring_host = nullptr;
   uint8_t* stage_rgb = nullptr;  // colour volumes: W*H*3
   const uint8_t* seq_rgb = nullptr;  // RGB of the bound sequence (vh_bind_sequence_rgb)
   // bound device sequence
@@ -600,12 +604,14 @@ void free_volume(vh_volume* v) {
     if (v->ring_done[k]) (void)hipEventDestroy(v->ring_done[k]);
   }
   if (v->ring_pose_host) (void)hipHostFree(v->ring_pose_host);
+  if (v->stage_host) (void)hipHostFree(v->stage_host);
+  if (v->ring_host) (void)hipHostFree(v->ring_host);
   if (v->pin) (void)hipHostFree(v->pin);
   if (v->copy_stream) (void)hipStreamDestroy(v->copy_stream);
   for (hipEvent_t e : v->ev_pending) (void)hipEventDestroy(e);
   free_index_buffers(v);
   void* ptrs[] = {v->keys, v->vals, v->marks, v->block_keys, v->block_info, v->tilemax, v->dm, v->voxels, v->touched, v->ctl,
-                  v->stage_depth, v->stage_pose, v->mc_tris, v->mc_cubes, v->mc_counts, v->mc_chunks, v->mc_total, v->mc_nbrs,
+                  v->stage_pose, v->mc_tris, v->mc_cubes, v->mc_counts, v->mc_chunks, v->mc_total, v->mc_nbrs,
                   v->gn_partials, v->gn_pose, v->gn_stats, v->bw_pose, v->gn_state, v->trk_pts,
                   v->ring_depth, v->ring_pose, v->colors, v->stage_rgb, v->ring_rgb, v->mc_rgb, v->rgba,
                   v->st_idx, v->st_keys, v->d_slab_w, v->d_slab_c};
@@ -1063,6 +1069,65 @@ int scratch_for_device(int device, double** out) {
   return VH_OK;
 }
 
+constexpr size_t kPoseBytes = 16 * sizeof(float);
+
+// Where a caller's image lies: page-locked memory is copied from where it is; pageable memory is
+// first copied, rows together, into page-locked memory of the volume; anything else the runtime knows
+// (device or managed memory) is left to its own 2D copy. The runtime's 2D copy goes row by row from
+// pageable memory, and from page-locked memory where rows aren't whole words: a 640 x 480 frame of
+// uint16 took 4.5 ms (and 20 to 97 ms at odd widths), through page-locked memory 0.1.
+enum class HostMemory { kLocked, kPageable, kOther };
+HostMemory memory_of(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();  // an address the runtime doesn't know
+    return HostMemory::kPageable;
+  }
+  if (a.type == hipMemoryTypeUnregistered) return HostMemory::kPageable;
+  return a.type == hipMemoryTypeHost ? HostMemory::kLocked : HostMemory::kOther;
+}
+
+// *buf: `bytes` of page-locked memory, allocated once; null if there is none left (the caller then copies as
+// the runtime does).
+char* locked_buffer(char** buf, size_t bytes) {
+  if (!*buf && hipHostMalloc((void**)buf, bytes, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    *buf = nullptr;
+  }
+  return *buf;
+}
+
+void copy_rows(char* dst, const void* src, size_t row, size_t pitch, size_t rows) {
+  const char* s = static_cast<const char*>(src);
+  if (pitch == row) {
+    std::memcpy(dst, s, row * rows);
+    return;
+  }
+  for (size_t r = 0; r < rows; ++r) std::memcpy(dst + r * row, s + r * pitch, row);
+}
+
+// An image on its way to the device: from `from`, or from the caller's rows where that is null.
+struct HostImage {
+  const void* from = nullptr;  // contiguous page-locked bytes
+  bool gathered = false;       // they are the volume's own
+};
+HostImage host_image(const void* src, size_t row, size_t pitch, size_t rows, char** buf, size_t bytes, size_t offset) {
+  const HostMemory m = memory_of(src);
+  if (m == HostMemory::kOther) return {};
+  if (m == HostMemory::kLocked) {
+    if (pitch == row) return {src, false};
+    if (((row | pitch | reinterpret_cast<uintptr_t>(src)) & 3) == 0) return {};
+  }
+  char* b = locked_buffer(buf, bytes);
+  if (!b) return {};
+  copy_rows(b + offset, src, row, pitch, rows);
+  return {b + offset, true};
+}
+hipError_t copy_image(void* dst, const HostImage& h, const void* src, size_t row, size_t pitch, size_t rows, hipStream_t st) {
+  if (h.from) return hipMemcpyAsync(dst, h.from, row * rows, hipMemcpyHostToDevice, st);
+  return hipMemcpy2DAsync(dst, row, src, pitch, row, rows, hipMemcpyHostToDevice, st);
+}
+
 }  // namespace
 
 extern "C" {
@@ -1130,13 +1195,14 @@ int vh_create(const vh_config* cfg, vh_volume** out) {
       (rc = dev_alloc(&v->voxels, pool * kB3 * voxel_bytes(cfg->storage))) ||
       (rc = dev_alloc(&v->touched, (size_t)2 * kStripes * v->stripe_cap * 4)) ||
       (rc = dev_alloc(&v->ctl, sizeof(FrameCtl))) ||
-      (rc = dev_alloc(&v->stage_depth, frame_px * 4)) || (rc = dev_alloc(&v->stage_pose, 16 * sizeof(float))) ||
+      (rc = dev_alloc(&v->stage_pose, kPoseBytes + frame_px * 4)) ||
       (cfg->color && ((rc = dev_alloc(&v->colors, pool * kB3 * 4)) || (rc = dev_alloc(&v->stage_rgb, frame_px * 3)) ||
                       (rc = dev_alloc(&v->rgba, 2 * kMaxBatch * image_px * 4))))) {
     std::string msg = g_last_error;
     free_volume(v);
     return fail(rc, msg);
   }
+  v->stage_depth = reinterpret_cast<char*>(v->stage_pose) + kPoseBytes;
   hipError_t e = hipMemsetAsync(v->marks, 0, 2 * v->n_slots * 4, v->stream);
   if (e == hipSuccess) e = hipMemsetAsync(v->ctl, 0, sizeof(FrameCtl), v->stream);
   if (e != hipSuccess) {
@@ -1183,12 +1249,21 @@ int vh_integrate(vh_volume* v, const vh_frame* f) {
   const size_t pitch = f->pitch ? (size_t)f->pitch : row;
   if (pitch < row) return fail(VH_ERR_INVALID_ARG, "pitch smaller than a row");
   if (v->colors && !f->rgb) return fail(VH_ERR_INVALID_ARG, "a colour volume needs the frame's RGB image");
-  VH_HIP(hipMemcpy2DAsync(v->stage_depth, row, f->depth, pitch, row, (size_t)v->cfg.height, hipMemcpyHostToDevice,
-                          v->stream));
-  VH_HIP(hipMemcpyAsync(v->stage_pose, f->c2w, 16 * sizeof(float), hipMemcpyHostToDevice, v->stream));
-  if (v->colors)
-    VH_HIP(hipMemcpyAsync(v->stage_rgb, f->rgb, (size_t)v->cfg.width * v->cfg.height * 3, hipMemcpyHostToDevice,
-                          v->stream));
+  const size_t rows = (size_t)v->cfg.height, frame_px = (size_t)v->cfg.width * rows;
+  const size_t stage_bytes = kPoseBytes + frame_px * (v->colors ? 7 : 4);
+  const HostImage depth = host_image(f->depth, row, pitch, rows, &v->stage_host, stage_bytes, kPoseBytes);
+  if (depth.gathered) {  // the pose goes with it
+    std::memcpy(v->stage_host, f->c2w, kPoseBytes);
+    VH_HIP(hipMemcpyAsync(v->stage_pose, v->stage_host, kPoseBytes + row * rows, hipMemcpyHostToDevice, v->stream));
+  } else {
+    VH_HIP(copy_image(v->stage_depth, depth, f->depth, row, pitch, rows, v->stream));
+    VH_HIP(hipMemcpyAsync(v->stage_pose, f->c2w, kPoseBytes, hipMemcpyHostToDevice, v->stream));
+  }
+  if (v->colors) {
+    const size_t line = (size_t)v->cfg.width * 3;
+    const HostImage rgb = host_image(f->rgb, line, line, rows, &v->stage_host, stage_bytes, kPoseBytes + frame_px * 4);
+    VH_HIP(hipMemcpyAsync(v->stage_rgb, rgb.from ? rgb.from : f->rgb, line * rows, hipMemcpyHostToDevice, v->stream));
+  }
   const int which = f->depth_format == VH_DEPTH_U16 ? 0 : 1;
   // the staged uint16 graph bakes the depth scale; re-capture when it changes
   if (which == 0 && f->depth_scale != v->graph_scale) {
@@ -1196,7 +1271,10 @@ int vh_integrate(vh_volume* v, const vh_frame* f) {
     v->graph_scale = f->depth_scale;
   }
   rc = launch_frame(v, which, f->depth_scale);
-  if (rc) return rc;
+  if (rc) {
+    (void)hipStreamSynchronize(v->stream);  // the copies above are done before the buffers are used again
+    return rc;
+  }
   return sync_and_check(v);
 }
 
@@ -1247,13 +1325,17 @@ int vh_integrate_async(vh_volume* v, const vh_frame* f) {
   }
   std::memcpy(v->ring_pose_host + 16 * slot, f->c2w, 16 * sizeof(float));
   char* dst = static_cast<char*>(v->ring_depth) + (size_t)slot * v->cfg.width * v->cfg.height * elem;
-  VH_HIP(hipMemcpy2DAsync(dst, row, f->depth, pitch, row, (size_t)v->cfg.height, hipMemcpyHostToDevice,
-                          v->copy_stream));
+  const size_t rows = (size_t)v->cfg.height, slot_bytes = frame_px * (v->colors ? 7 : 4);
+  const HostImage depth = host_image(f->depth, row, pitch, rows, &v->ring_host, R * slot_bytes, slot * slot_bytes);
+  VH_HIP(copy_image(dst, depth, f->depth, row, pitch, rows, v->copy_stream));
   VH_HIP(hipMemcpyAsync(v->ring_pose + 16 * slot, v->ring_pose_host + 16 * slot, 16 * sizeof(float),
                         hipMemcpyHostToDevice, v->copy_stream));
-  if (v->colors)
-    VH_HIP(hipMemcpyAsync(v->ring_rgb + (size_t)slot * frame_px * 3, f->rgb, frame_px * 3, hipMemcpyHostToDevice,
-                          v->copy_stream));
+  if (v->colors) {
+    const size_t line = (size_t)v->cfg.width * 3;
+    const HostImage rgb = host_image(f->rgb, line, line, rows, &v->ring_host, R * slot_bytes, slot * slot_bytes + frame_px * 4);
+    VH_HIP(hipMemcpyAsync(v->ring_rgb + (size_t)slot * frame_px * 3, rgb.from ? rgb.from : f->rgb, line * rows,
+                          hipMemcpyHostToDevice, v->copy_stream));
+  }
   VH_HIP(hipEventRecord(v->ring_copied[slot], v->copy_stream));
   VH_HIP(hipStreamWaitEvent(v->stream, v->ring_copied[slot], 0));
   if ((rc = launch_frame(v, which, f->depth_scale))) return rc;
