@@ -64,3 +64,28 @@ def test_host_images(vh, oracle, W, H, fmt, pad, shift, locked):
         assert vol.stats()["frames"] == n
         (assert_same_colour_volume if color else assert_same_volume)(oracle, vol, ref)
         vol.close()
+
+
+@pytest.mark.parametrize("locked", [False, True])
+def test_images_on_both_sides_of_the_direct_copy(vh, oracle, locked):
+    """700 x 600: uint16 is read in the frame's own stream, float32 (1.68 MB) copied on the other one; the
+    queue takes runs of both, so that slots change hands both ways."""
+    import torch
+
+    W, H = 700, 600
+    w = workload(W, H, 0)
+    rng = np.random.default_rng(3)
+    kinds = [0, 1, 1, 0, 0, 1, 1, 1, 1, 1, 1, 0, 0, 0, 0, 0, 1]
+    base = (1000 + 0.5 * np.arange(W) + 0.3 * np.arange(H)[:, None]).astype(np.uint16)
+    mm = [(base + rng.integers(0, 30, (H, W)).astype(np.uint16)) for _ in kinds]
+    vol, ref, keep = vh.Volume(vh.config_from_workload(w)), oracle.Oracle(w), []
+    T = np.eye(4, dtype=np.float32)
+    for k, d in zip(kinds, mm):
+        ref.integrate(d, T)
+        a = torch.from_numpy(d.astype(np.float32) * np.float32(0.001) if k else d.view(np.int16))
+        keep.append(a.pin_memory() if locked else a)
+        vol.integrate_async(keep[-1], T)
+    vol.sync()
+    assert vol.stats()["frames"] == len(kinds)
+    assert_same_volume(oracle, vol, ref)
+    vol.close()

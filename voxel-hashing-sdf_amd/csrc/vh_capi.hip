@@ -13,11 +13,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <map>
 #include <mutex>
 #include <new>
 #include <string>
-#include <tuple>
 #include <unordered_map>
 #include <unordered_set>
 #include <vector>
@@ -111,11 +109,10 @@ struct vh_volume {
   uint32_t* touched = nullptr;
   uint32_t stripe_cap = 0;
   FrameCtl* ctl = nullptr;
-  // staged host input (one frame, both formats) and its pose
+  // staged host input (one frame, both formats)
   void* stage_depth = nullptr;
-  float* stage_pose = nullptr;   // 16, directly before stage_depth (one allocation)
   // page-locked copies of callers' pageable images (host_image), allocated when the first one comes:
-  // vh_integrate's pose, depth and colours; per ring slot the depth and colours
+  // vh_integrate's depth and colours; the same per ring slot
   char* stage_host = nullptr;
   char* ring_host = nullptr;
   uint8_t* stage_rgb = nullptr;  // colour volumes: W*H*3
@@ -142,19 +139,16 @@ struct vh_volume {
   void* ring_depth = nullptr;       // kRing frames of W*H elements
   int32_t ring_format = -1;         // depth format of the queued frames (slot stride W*H*element)
   uint8_t* ring_rgb = nullptr;      // colour volumes: kRing frames of W*H*3 bytes
-  float* ring_pose = nullptr;       // kRing x 16 (device)
-  float* ring_pose_host = nullptr;  // kRing x 16 (page-locked)
   hipEvent_t ring_copied[kRing] = {}, ring_done[kRing] = {};
+  bool ring_held[kRing] = {};       // the slot's copy is waited for by the host before its next (ring_copied)
+  bool ring_marked[kRing] = {};     // ring_done covers the frame that read the slot last
   uint64_t ring_next = 0;           // frames queued since create/reset (= device cursor 2)
-  // graphs by (kind, frames integrated, frames allocated): kinds [0] staged u16, [1] staged
-  // f32, [2] bound sequence step (integrate batch b + allocate batch b+1), [3] tracked
-  // sequence, [4] bound sequence first allocation, [5] bound sequence last integration,
-  // [6] ring u16, [7] ring f32
-  static constexpr int kGraphs = 8;
-  std::map<std::tuple<int, int, int>, hipGraphExec_t> graphs;
+  // kinds of frame steps: [0] staged u16, [1] staged f32, [2] bound sequence step (integrate batch b +
+  // allocate batch b+1), [3] tracked sequence, [4] bound sequence first allocation, [5] bound
+  // sequence last integration, [6] ring u16, [7] ring f32
+  hipGraphExec_t track_graph = nullptr;  // kind 3, of the bound sequence
   int batch = kMaxBatch;  // frames per launch on bound sequences
-  float ring_scale = -1.0f;  // depth scale baked into the ring uint16 graph
-  // profiling: 1 = eager launches with events around each kernel, 2 = the captured graphs with
+  // profiling: 1 = eager launches with events around each kernel, 2 = the usual launches with
   // events around each fused batch launch
   int profiling = 0;
   std::vector<hipEvent_t> ev_pool;
@@ -205,7 +199,6 @@ struct vh_volume {
   double* gn_stats = nullptr;
   GnState* gn_state = nullptr;
   float* bw_pose = nullptr;
-  float graph_scale = -1.0f;  // depth scale baked into the staged uint16 graph
   std::mutex mu;
 };
 
@@ -222,15 +215,14 @@ size_t voxel_bytes(int storage) { return storage == VH_STORAGE_F32 ? 8 : 4; }
 // of 4, so that a row starts at a 16-byte boundary.
 int image_pitch(const vh_config& c) { return (c.width + 3) & ~3; }
 
-FrameArgs frame_args(vh_volume* v, int which) {
+// host: the frame of a host kind (0, 1, 6, 7), whose pose and depth scale come with the launch.
+FrameArgs frame_args(vh_volume* v, int which, const vh_frame* host = nullptr) {
   FrameArgs a{};
   const vh_config& c = v->cfg;
   if (which == 6 || which == 7) {
     a.depth = v->ring_depth;
-    a.poses = v->ring_pose;
     a.n_seq = vh_volume::kRing;
     a.cursor_id = 2;
-    a.depth_scale = which == 6 ? v->ring_scale : 1.0f;
     a.rgb = v->ring_rgb;
   } else if (which >= 2) {
     a.depth = v->seq_depth;
@@ -241,11 +233,13 @@ FrameArgs frame_args(vh_volume* v, int which) {
     a.rgb = v->seq_rgb;
   } else {
     a.depth = v->stage_depth;
-    a.poses = v->stage_pose;
     a.n_seq = 1;
     a.cursor_id = 0;
-    a.depth_scale = 1.0f;  // the caller sets the uint16 scale of a staged frame
     a.rgb = v->stage_rgb;
+  }
+  if (host) {
+    for (int k = 0; k < 12; ++k) a.pose[k] = host->c2w[k];
+    a.depth_scale = host->depth_format == VH_DEPTH_U16 ? host->depth_scale : 1.0f;
   }
   a.W = c.width;
   a.H = c.height;
@@ -372,11 +366,10 @@ int frame_u16(vh_volume* v, int which) {
 // batches of up to `batch` frames: kind 4 (allocate the first batch, ka frames), kind 2 per
 // further batch (integrate the previous batch, ki frames, and allocate this one, ka frames,
 // in one launch) and kind 5 (integrate the last batch, ki frames).
-int enqueue_frame_kernels(vh_volume* v, int which, float staged_scale, int ki, int ka) {
+int enqueue_frame_kernels(vh_volume* v, int which, const vh_frame* host, int ki, int ka) {
   const int fa = which == 4 || which == 5 ? 2 : which;
-  FrameArgs a = frame_args(v, fa);
+  const FrameArgs a = frame_args(v, fa, host);
   const int u16 = frame_u16(v, fa);
-  if (fa < 2 || fa >= 6) a.depth_scale = u16 ? staged_scale : 1.0f;
   const bool carve = v->cfg.carve != 0;
   if (which == 2) {
     VH_HIP(launch_integrate_alloc(a, v->cfg.storage, u16, fused_grid(), ki, ka, v->stream));
@@ -407,16 +400,38 @@ hipEvent_t take_event(vh_volume* v) {
   return e;
 }
 
-// One launch of kind `which` (ki frames integrated, ka allocated; single frames: 1, 1). In
+// A frame of the tracked sequence, captured once per binding.
+int launch_tracked(vh_volume* v) {
+  hipGraphExec_t& g = v->track_graph;
+  if (!g) {
+    hipGraph_t graph = nullptr;
+    VH_HIP(hipStreamBeginCapture(v->stream, hipStreamCaptureModeThreadLocal));
+    int rc = enqueue_frame_kernels(v, 3, nullptr, 1, 1);
+    hipError_t e = hipStreamEndCapture(v->stream, &graph);
+    if (rc != VH_OK) {
+      if (graph) (void)hipGraphDestroy(graph);
+      return rc;
+    }
+    VH_HIP(e);
+    e = hipGraphInstantiate(&g, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    VH_HIP(e);
+  }
+  VH_HIP(hipGraphLaunch(g, v->stream));
+  return VH_OK;
+}
+
+// One step of kind `which` (ki frames integrated, ka allocated; single frames: 1, 1). A tracked
+// frame's nine kernels replay as a graph; the other kinds are one to three kernels, launched as they
+// are (launching a graph of two takes 28 us of host time, two kernels 8). In
 // profiling mode a batch of k = max(ki, ka) frames runs eagerly as (tracking,) allocation of k
 // frames and integration of k frames, with events around each.
-int launch_frame(vh_volume* v, int which, float staged_scale, int ki = 1, int ka = 1) {
+int launch_frame(vh_volume* v, int which, const vh_frame* host, int ki = 1, int ka = 1) {
   if (v->profiling == 1) {
     hipEvent_t e[5] = {take_event(v), take_event(v), take_event(v), take_event(v), take_event(v)};
     if (!e[0] || !e[1] || !e[2] || !e[3] || !e[4]) return fail(VH_ERR_DEVICE, "hipEventCreate failed");
-    FrameArgs a = frame_args(v, which);
+    const FrameArgs a = frame_args(v, which, host);
     const int u16 = frame_u16(v, which);
-    if (which < 2 || which >= 6) a.depth_scale = u16 ? staged_scale : 1.0f;
     const int k = std::max(ki, ka);
     VH_HIP(hipEventRecord(e[0], v->stream));
     if (which == 3) {
@@ -434,44 +449,24 @@ int launch_frame(vh_volume* v, int which, float staged_scale, int ki = 1, int ka
     v->ev_frames.push_back(k);
     return VH_OK;
   }
-  hipGraphExec_t& g = v->graphs[std::make_tuple(which, ki, ka)];
-  if (!g) {
-    hipGraph_t graph = nullptr;
-    VH_HIP(hipStreamBeginCapture(v->stream, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue_frame_kernels(v, which, staged_scale, ki, ka);
-    hipError_t e = hipStreamEndCapture(v->stream, &graph);
-    if (rc != VH_OK) {
-      if (graph) (void)hipGraphDestroy(graph);
-      return rc;
-    }
-    VH_HIP(e);
-    e = hipGraphInstantiate(&g, graph, nullptr, nullptr, 0);
-    (void)hipGraphDestroy(graph);
-    VH_HIP(e);
-  }
+  if (which == 3) return launch_tracked(v);
   if (v->profiling == 2 && which == 2) {
     hipEvent_t e0 = take_event(v), e1 = take_event(v);
     if (!e0 || !e1) return fail(VH_ERR_DEVICE, "hipEventCreate failed");
     VH_HIP(hipEventRecord(e0, v->stream));
-    VH_HIP(hipGraphLaunch(g, v->stream));
+    int rc = enqueue_frame_kernels(v, which, host, ki, ka);
+    if (rc) return rc;
     VH_HIP(hipEventRecord(e1, v->stream));
     v->ev_fused.push_back(e0);
     v->ev_fused.push_back(e1);
     return VH_OK;
   }
-  VH_HIP(hipGraphLaunch(g, v->stream));
-  return VH_OK;
+  return enqueue_frame_kernels(v, which, host, ki, ka);
 }
 
-void drop_graphs(vh_volume* v, int which_mask) {
-  for (auto it = v->graphs.begin(); it != v->graphs.end();) {
-    if ((which_mask >> std::get<0>(it->first)) & 1) {
-      if (it->second) (void)hipGraphExecDestroy(it->second);
-      it = v->graphs.erase(it);
-    } else {
-      ++it;
-    }
-  }
+void drop_graph(vh_volume* v) {
+  if (v->track_graph) (void)hipGraphExecDestroy(v->track_graph);
+  v->track_graph = nullptr;
 }
 
 int collect_profile(vh_volume* v) {
@@ -506,7 +501,7 @@ int collect_profile(vh_volume* v) {
 // the copy go through a staging buffer): n <= kPinWords words from dev into out.
 constexpr int kPinWords = 16;
 int read_words(vh_volume* v, const uint32_t* dev, uint32_t* out, int n) {
-  VH_HIP(hipMemcpyAsync(v->pin, dev, (size_t)n * 4, hipMemcpyDeviceToHost, v->stream));
+  VH_HIP(launch_words_out(v->pin, dev, n, v->stream));
   VH_HIP(hipStreamSynchronize(v->stream));
   for (int i = 0; i < n; ++i) out[i] = v->pin[i];
   return VH_OK;
@@ -596,14 +591,13 @@ void free_volume(vh_volume* v) {
   if (!v) return;
   (void)hipSetDevice(v->device);
   if (v->stream) (void)hipStreamSynchronize(v->stream);
-  drop_graphs(v, (1 << vh_volume::kGraphs) - 1);
+  drop_graph(v);
   if (v->copy_stream) (void)hipStreamSynchronize(v->copy_stream);
   for (hipEvent_t e : v->ev_pool) (void)hipEventDestroy(e);
   for (int k = 0; k < vh_volume::kRing; ++k) {
     if (v->ring_copied[k]) (void)hipEventDestroy(v->ring_copied[k]);
     if (v->ring_done[k]) (void)hipEventDestroy(v->ring_done[k]);
   }
-  if (v->ring_pose_host) (void)hipHostFree(v->ring_pose_host);
   if (v->stage_host) (void)hipHostFree(v->stage_host);
   if (v->ring_host) (void)hipHostFree(v->ring_host);
   if (v->pin) (void)hipHostFree(v->pin);
@@ -611,9 +605,9 @@ void free_volume(vh_volume* v) {
   for (hipEvent_t e : v->ev_pending) (void)hipEventDestroy(e);
   free_index_buffers(v);
   void* ptrs[] = {v->keys, v->vals, v->marks, v->block_keys, v->block_info, v->tilemax, v->dm, v->voxels, v->touched, v->ctl,
-                  v->stage_pose, v->mc_tris, v->mc_cubes, v->mc_counts, v->mc_chunks, v->mc_total, v->mc_nbrs,
+                  v->stage_depth, v->mc_tris, v->mc_cubes, v->mc_counts, v->mc_chunks, v->mc_total, v->mc_nbrs,
                   v->gn_partials, v->gn_pose, v->gn_stats, v->bw_pose, v->gn_state, v->trk_pts,
-                  v->ring_depth, v->ring_pose, v->colors, v->stage_rgb, v->ring_rgb, v->mc_rgb, v->rgba,
+                  v->ring_depth, v->colors, v->stage_rgb, v->ring_rgb, v->mc_rgb, v->rgba,
                   v->st_idx, v->st_keys, v->d_slab_w, v->d_slab_c};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -725,8 +719,8 @@ int index_count(vh_volume* v, McArgs& a, int64_t* n_faces, int64_t* n_vertices) 
   uint32_t tot[2] = {0u, 0u};
   if (a.n_blocks) {
     VH_HIP(launch_mesh_index_count(a, v->cfg.storage, v->stream));
-    VH_HIP(hipMemcpyAsync(&v->pin[0], v->mc_total, 4, hipMemcpyDeviceToHost, v->stream));
-    VH_HIP(hipMemcpyAsync(&v->pin[1], v->ix_vtotal, 4, hipMemcpyDeviceToHost, v->stream));
+    VH_HIP(launch_words_out(&v->pin[0], v->mc_total, 1, v->stream));
+    VH_HIP(launch_words_out(&v->pin[1], v->ix_vtotal, 1, v->stream));
   }
   VH_HIP(hipStreamSynchronize(v->stream));
   if (a.n_blocks) {
@@ -1069,8 +1063,6 @@ int scratch_for_device(int device, double** out) {
   return VH_OK;
 }
 
-constexpr size_t kPoseBytes = 16 * sizeof(float);
-
 // Where a caller's image lies: page-locked memory is copied from where it is; pageable memory is
 // first copied, rows together, into page-locked memory of the volume; anything else the runtime knows
 // (device or managed memory) is left to its own 2D copy. The runtime's 2D copy goes row by row from
@@ -1106,25 +1098,37 @@ void copy_rows(char* dst, const void* src, size_t row, size_t pitch, size_t rows
   for (size_t r = 0; r < rows; ++r) std::memcpy(dst + r * row, s + r * pitch, row);
 }
 
-// An image on its way to the device: from `from`, or from the caller's rows where that is null.
-struct HostImage {
-  const void* from = nullptr;  // contiguous page-locked bytes
-  bool gathered = false;       // they are the volume's own
-};
-HostImage host_image(const void* src, size_t row, size_t pitch, size_t rows, char** buf, size_t bytes, size_t offset) {
+// The image as contiguous page-locked bytes: the caller's own, or `offset` into the volume's *buf, of `bytes`
+// bytes; null: to be copied from the caller's rows as the runtime does.
+const void* host_image(const void* src, size_t row, size_t pitch, size_t rows, char** buf, size_t bytes, size_t offset) {
   const HostMemory m = memory_of(src);
-  if (m == HostMemory::kOther) return {};
+  if (m == HostMemory::kOther) return nullptr;
   if (m == HostMemory::kLocked) {
-    if (pitch == row) return {src, false};
-    if (((row | pitch | reinterpret_cast<uintptr_t>(src)) & 3) == 0) return {};
+    if (pitch == row) return src;
+    if (((row | pitch | reinterpret_cast<uintptr_t>(src)) & 3) == 0) return nullptr;
   }
   char* b = locked_buffer(buf, bytes);
-  if (!b) return {};
-  copy_rows(b + offset, src, row, pitch, rows);
-  return {b + offset, true};
+  if (b) copy_rows(b + offset, src, row, pitch, rows);
+  return b ? b + offset : nullptr;
 }
-hipError_t copy_image(void* dst, const HostImage& h, const void* src, size_t row, size_t pitch, size_t rows, hipStream_t st) {
-  if (h.from) return hipMemcpyAsync(dst, h.from, row * rows, hipMemcpyHostToDevice, st);
+
+// Images of a frame up to here are read by a kernel in the frame's own stream (k_copy_in), larger ones by
+// the copy engine on the copy stream, where the copy overlaps the kernels of the frame before. The
+// overlap costs the host and the streams' waits 64 us a frame (640 x 480 uint16, queued), the bus moves
+// 1.6 MB in 36 us, and a frame's kernels take 25; the small frame takes 46 us in one stream.
+constexpr size_t kDirectBytes = 1600 * 1024;
+
+// An image to the device: `from`, its contiguous page-locked bytes (read by a kernel if direct), or where that
+// is null the caller's rows.
+hipError_t copy_image(void* dst, const void* from, const void* src, size_t row, size_t pitch, size_t rows, bool direct,
+                      hipStream_t st) {
+  if (from && direct) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, from) == hipSuccess && a.devicePointer) return launch_copy_in(dst, a.devicePointer, row * rows, st);
+    (void)hipGetLastError();
+  }
+  if (from) return hipMemcpyAsync(dst, from, row * rows, hipMemcpyHostToDevice, st);
+  if (pitch == row && memory_of(src) != HostMemory::kOther) return hipMemcpyAsync(dst, src, row * rows, hipMemcpyHostToDevice, st);
   return hipMemcpy2DAsync(dst, row, src, pitch, row, rows, hipMemcpyHostToDevice, st);
 }
 
@@ -1195,14 +1199,13 @@ int vh_create(const vh_config* cfg, vh_volume** out) {
       (rc = dev_alloc(&v->voxels, pool * kB3 * voxel_bytes(cfg->storage))) ||
       (rc = dev_alloc(&v->touched, (size_t)2 * kStripes * v->stripe_cap * 4)) ||
       (rc = dev_alloc(&v->ctl, sizeof(FrameCtl))) ||
-      (rc = dev_alloc(&v->stage_pose, kPoseBytes + frame_px * 4)) ||
+      (rc = dev_alloc(&v->stage_depth, frame_px * 4)) ||
       (cfg->color && ((rc = dev_alloc(&v->colors, pool * kB3 * 4)) || (rc = dev_alloc(&v->stage_rgb, frame_px * 3)) ||
                       (rc = dev_alloc(&v->rgba, 2 * kMaxBatch * image_px * 4))))) {
     std::string msg = g_last_error;
     free_volume(v);
     return fail(rc, msg);
   }
-  v->stage_depth = reinterpret_cast<char*>(v->stage_pose) + kPoseBytes;
   hipError_t e = hipMemsetAsync(v->marks, 0, 2 * v->n_slots * 4, v->stream);
   if (e == hipSuccess) e = hipMemsetAsync(v->ctl, 0, sizeof(FrameCtl), v->stream);
   if (e != hipSuccess) {
@@ -1250,27 +1253,17 @@ int vh_integrate(vh_volume* v, const vh_frame* f) {
   if (pitch < row) return fail(VH_ERR_INVALID_ARG, "pitch smaller than a row");
   if (v->colors && !f->rgb) return fail(VH_ERR_INVALID_ARG, "a colour volume needs the frame's RGB image");
   const size_t rows = (size_t)v->cfg.height, frame_px = (size_t)v->cfg.width * rows;
-  const size_t stage_bytes = kPoseBytes + frame_px * (v->colors ? 7 : 4);
-  const HostImage depth = host_image(f->depth, row, pitch, rows, &v->stage_host, stage_bytes, kPoseBytes);
-  if (depth.gathered) {  // the pose goes with it
-    std::memcpy(v->stage_host, f->c2w, kPoseBytes);
-    VH_HIP(hipMemcpyAsync(v->stage_pose, v->stage_host, kPoseBytes + row * rows, hipMemcpyHostToDevice, v->stream));
-  } else {
-    VH_HIP(copy_image(v->stage_depth, depth, f->depth, row, pitch, rows, v->stream));
-    VH_HIP(hipMemcpyAsync(v->stage_pose, f->c2w, kPoseBytes, hipMemcpyHostToDevice, v->stream));
-  }
+  const size_t stage_bytes = frame_px * (v->colors ? 7 : 4);
+  const void* depth = host_image(f->depth, row, pitch, rows, &v->stage_host, stage_bytes, 0);
+  const bool direct = rows * (row + (v->colors ? 3 * (size_t)v->cfg.width : 0)) <= kDirectBytes;
+  VH_HIP(copy_image(v->stage_depth, depth, f->depth, row, pitch, rows, direct, v->stream));
   if (v->colors) {
     const size_t line = (size_t)v->cfg.width * 3;
-    const HostImage rgb = host_image(f->rgb, line, line, rows, &v->stage_host, stage_bytes, kPoseBytes + frame_px * 4);
-    VH_HIP(hipMemcpyAsync(v->stage_rgb, rgb.from ? rgb.from : f->rgb, line * rows, hipMemcpyHostToDevice, v->stream));
+    const void* rgb = host_image(f->rgb, line, line, rows, &v->stage_host, stage_bytes, frame_px * 4);
+    VH_HIP(copy_image(v->stage_rgb, rgb, f->rgb, line, line, rows, direct, v->stream));
   }
   const int which = f->depth_format == VH_DEPTH_U16 ? 0 : 1;
-  // the staged uint16 graph bakes the depth scale; re-capture when it changes
-  if (which == 0 && f->depth_scale != v->graph_scale) {
-    drop_graphs(v, 1);
-    v->graph_scale = f->depth_scale;
-  }
-  rc = launch_frame(v, which, f->depth_scale);
+  rc = launch_frame(v, which, f);
   if (rc) {
     (void)hipStreamSynchronize(v->stream);  // the copies above are done before the buffers are used again
     return rc;
@@ -1298,10 +1291,8 @@ int vh_integrate_async(vh_volume* v, const vh_frame* f) {
   const size_t frame_px = (size_t)v->cfg.width * v->cfg.height;
   if (!v->copy_stream) {
     if ((rc = dev_alloc(&v->ring_depth, (size_t)R * frame_px * 4)) ||
-        (rc = dev_alloc(&v->ring_pose, (size_t)R * 16 * sizeof(float))) ||
         (v->colors && (rc = dev_alloc(&v->ring_rgb, (size_t)R * frame_px * 3))))
       return rc;
-    VH_HIP(hipHostMalloc((void**)&v->ring_pose_host, (size_t)R * 16 * sizeof(float), hipHostMallocDefault));
     for (int k = 0; k < R; ++k) {
       VH_HIP(hipEventCreateWithFlags(&v->ring_copied[k], hipEventDisableTiming));
       VH_HIP(hipEventCreateWithFlags(&v->ring_done[k], hipEventDisableTiming));
@@ -1309,37 +1300,38 @@ int vh_integrate_async(vh_volume* v, const vh_frame* f) {
     VH_HIP(hipStreamCreateWithFlags(&v->copy_stream, hipStreamNonBlocking));
   }
   const int which = f->depth_format == VH_DEPTH_U16 ? 6 : 7;
-  if (which == 6 && f->depth_scale != v->ring_scale) {  // the ring uint16 graph bakes the scale
-    VH_HIP(hipStreamSynchronize(v->stream));
-    drop_graphs(v, 1 << 6);
-    v->ring_scale = f->depth_scale;
-  }
   // The slots are laid out with the element size of the frames in flight: before a frame of
   // the other format is copied, the queued frames finish (their slots would overlap).
   if (v->ring_format >= 0 && v->ring_format != f->depth_format) VH_HIP(hipStreamSynchronize(v->stream));
   v->ring_format = f->depth_format;
   const int slot = (int)(v->ring_next % R);
-  if (v->ring_next >= (uint64_t)R) {
-    VH_HIP(hipStreamWaitEvent(v->copy_stream, v->ring_done[slot], 0));  // the frame that read the slot
-    VH_HIP(hipEventSynchronize(v->ring_copied[slot]));                    // the pose staging is free
-  }
-  std::memcpy(v->ring_pose_host + 16 * slot, f->c2w, 16 * sizeof(float));
-  char* dst = static_cast<char*>(v->ring_depth) + (size_t)slot * v->cfg.width * v->cfg.height * elem;
   const size_t rows = (size_t)v->cfg.height, slot_bytes = frame_px * (v->colors ? 7 : 4);
-  const HostImage depth = host_image(f->depth, row, pitch, rows, &v->ring_host, R * slot_bytes, slot * slot_bytes);
-  VH_HIP(copy_image(dst, depth, f->depth, row, pitch, rows, v->copy_stream));
-  VH_HIP(hipMemcpyAsync(v->ring_pose + 16 * slot, v->ring_pose_host + 16 * slot, 16 * sizeof(float),
-                        hipMemcpyHostToDevice, v->copy_stream));
-  if (v->colors) {
-    const size_t line = (size_t)v->cfg.width * 3;
-    const HostImage rgb = host_image(f->rgb, line, line, rows, &v->ring_host, R * slot_bytes, slot * slot_bytes + frame_px * 4);
-    VH_HIP(hipMemcpyAsync(v->ring_rgb + (size_t)slot * frame_px * 3, rgb.from ? rgb.from : f->rgb, line * rows,
-                          hipMemcpyHostToDevice, v->copy_stream));
+  const size_t line = (size_t)v->cfg.width * 3;
+  const bool direct = rows * (row + (v->colors ? line : 0)) <= kDirectBytes;
+  const hipStream_t copies = direct ? v->stream : v->copy_stream;
+  if (v->ring_held[slot]) VH_HIP(hipEventSynchronize(v->ring_copied[slot]));
+  if (!direct) {  // the copy waits for the frame that read the slot
+    if (!v->ring_marked[slot]) VH_HIP(hipEventRecord(v->ring_done[slot], v->stream));
+    VH_HIP(hipStreamWaitEvent(v->copy_stream, v->ring_done[slot], 0));
   }
-  VH_HIP(hipEventRecord(v->ring_copied[slot], v->copy_stream));
-  VH_HIP(hipStreamWaitEvent(v->stream, v->ring_copied[slot], 0));
-  if ((rc = launch_frame(v, which, f->depth_scale))) return rc;
-  VH_HIP(hipEventRecord(v->ring_done[slot], v->stream));
+  char* dst = static_cast<char*>(v->ring_depth) + (size_t)slot * v->cfg.width * v->cfg.height * elem;
+  const void* depth = host_image(f->depth, row, pitch, rows, &v->ring_host, R * slot_bytes, slot * slot_bytes);
+  VH_HIP(copy_image(dst, depth, f->depth, row, pitch, rows, direct, copies));
+  const void* rgb = nullptr;
+  if (v->colors) {
+    rgb = host_image(f->rgb, line, line, rows, &v->ring_host, R * slot_bytes, slot * slot_bytes + frame_px * 4);
+    VH_HIP(copy_image(v->ring_rgb + (size_t)slot * frame_px * 3, rgb, f->rgb, line, line, rows, direct, copies));
+  }
+  // the volume's own page-locked bytes are written again only after the copy; a caller's are the caller's
+  v->ring_held[slot] = !direct || (depth && depth != f->depth) || (rgb && rgb != f->rgb);
+  if (v->ring_held[slot]) VH_HIP(hipEventRecord(v->ring_copied[slot], copies));
+  if (!direct) VH_HIP(hipStreamWaitEvent(v->stream, v->ring_copied[slot], 0));
+  v->ring_marked[slot] = false;
+  if ((rc = launch_frame(v, which, f))) return rc;
+  if (!direct) {
+    VH_HIP(hipEventRecord(v->ring_done[slot], v->stream));
+    v->ring_marked[slot] = true;
+  }
   ++v->ring_next;
   return VH_OK;
 }
@@ -1360,8 +1352,8 @@ int vh_bind_sequence(vh_volume* v, const void* d_depth, int32_t fmt, float scale
   v->seq_format = fmt;
   v->seq_scale = scale;
   v->track = false;
-  // the captured graphs hold the sequence pointers
-  if (!same || v->seq_rgb) drop_graphs(v, 4 | 8 | 16 | 32);
+  // the tracked frame's graph holds the sequence pointers
+  if (!same || v->seq_rgb) drop_graph(v);
   v->seq_rgb = nullptr;
   const uint32_t zero = 0;
   VH_HIP(hipMemcpyAsync(&v->ctl->cursor[1], &zero, sizeof zero, hipMemcpyHostToDevice, v->stream));
@@ -1397,7 +1389,7 @@ int vh_bind_tracking(vh_volume* v, const void* d_depth, int32_t fmt, float scale
     if (v->trk_pts) (void)hipFree(v->trk_pts);
     v->trk_pts = nullptr;
     v->trk_pts_cap = 0;
-    drop_graphs(v, 8);
+    drop_graph(v);
     if ((rc = dev_alloc(&v->trk_pts, npts * 3 * sizeof(float)))) return rc;
     v->trk_pts_cap = npts;
   }
@@ -1425,7 +1417,7 @@ int vh_bind_tracking(vh_volume* v, const void* d_depth, int32_t fmt, float scale
   v->trk_sigma_t = tc->prior_sigma_t;
   v->trk_sigma_r = tc->prior_sigma_rot;
   v->trk_points = tc->depth_points;
-  if (!same || v->seq_rgb) drop_graphs(v, 4 | 8 | 16 | 32);
+  if (!same || v->seq_rgb) drop_graph(v);
   v->seq_rgb = nullptr;
   const uint32_t zero = 0;
   VH_HIP(hipMemcpyAsync(&v->ctl->cursor[1], &zero, sizeof zero, hipMemcpyHostToDevice, v->stream));
@@ -1442,7 +1434,7 @@ int vh_bind_sequence_rgb(vh_volume* v, const uint8_t* d_rgb) {
   if (rc) return rc;
   if (v->seq_rgb != d_rgb) {
     VH_HIP(hipStreamSynchronize(v->stream));
-    drop_graphs(v, 4 | 8 | 16 | 32);
+    drop_graph(v);
     v->seq_rgb = d_rgb;
   }
   return VH_OK;
@@ -1459,7 +1451,7 @@ int vh_integrate_next(vh_volume* v, int32_t n) {
   if (v->track) {
     // per frame: tracking, allocation, integration (each pose depends on the volume so far)
     for (int k = 0; k < n; ++k) {
-      rc = launch_frame(v, 3, v->seq_scale);
+      rc = launch_frame(v, 3, nullptr);
       if (rc) return rc;
     }
     return VH_OK;
@@ -1468,20 +1460,20 @@ int vh_integrate_next(vh_volume* v, int32_t n) {
   const int K = v->batch;
   if (v->profiling == 1) {
     for (int f = 0; f < n; f += K)
-      if ((rc = launch_frame(v, 2, v->seq_scale, std::min(K, n - f), std::min(K, n - f)))) return rc;
+      if ((rc = launch_frame(v, 2, nullptr, std::min(K, n - f), std::min(K, n - f)))) return rc;
     return VH_OK;
   }
   // allocation of batch b+1 overlaps the integration of batch b; nothing stays allocated
   // but unintegrated when the call returns
   if (n == 0) return VH_OK;
   int prev = std::min(K, n);
-  if ((rc = launch_frame(v, 4, v->seq_scale, 0, prev))) return rc;
+  if ((rc = launch_frame(v, 4, nullptr, 0, prev))) return rc;
   for (int f = prev; f < n; f += K) {
     const int cur = std::min(K, n - f);
-    if ((rc = launch_frame(v, 2, v->seq_scale, prev, cur))) return rc;
+    if ((rc = launch_frame(v, 2, nullptr, prev, cur))) return rc;
     prev = cur;
   }
-  return launch_frame(v, 5, v->seq_scale, prev, 0);
+  return launch_frame(v, 5, nullptr, prev, 0);
 }
 
 int vh_sync(vh_volume* v) {

@@ -96,9 +96,11 @@ struct HashView {
 };
 
 struct FrameArgs {
-  // input frames: frame f of the input is depth + f*W*H elements, pose poses + 16 f
+  // input frames: frame f of the input is depth + f*W*H elements, pose poses + 16 f; a host
+  // frame's pose comes with the launch (poses null): no copy of it, 64 bytes, in front of the kernels
   const void* depth;
   const float* poses;
+  float pose[12];
   uint32_t n_seq;
   int32_t cursor_id;
   float depth_scale;
@@ -383,6 +385,8 @@ hipError_t launch_stream_rehash(const StreamArgs& a, hipStream_t st);
 // and their words; keys already resident are merged into the resident block (placed[] says
 // which).
 hipError_t launch_stream_insert(const StreamArgs& a, int storage, hipStream_t st);
+hipError_t launch_copy_in(void* dst, const void* src, size_t bytes, hipStream_t st);
+hipError_t launch_words_out(uint32_t* dst, const uint32_t* src, int n, hipStream_t st);
 hipError_t launch_query(const QueryArgs& q, int storage, const float* pts, int64_t n, float* sdf,
                         uint8_t* valid, hipStream_t st);
 hipError_t launch_backward(const QueryArgs& q, int storage, const float* pts, int64_t n,

@@ -76,6 +76,23 @@ __device__ __forceinline__ float depth_at(const void* base, float scale, int pix
   return reinterpret_cast<const float*>(base)[(uint32_t)pix];
 }
 
+// ============================================================================ host images
+// A small image from page-locked host memory, read over the bus by the lanes themselves. Through the
+// copy engine on a second stream a queued frame cost the host 64 us, most of it for the copy's and the
+// kernels' waits for each other; in the kernels' own stream it costs its time on the bus (640 x
+// 480 uint16: 15 us) and a launch. System-scope loads: the host writes this memory between frames.
+template <class T>
+__global__ __launch_bounds__(256) void k_copy_in(T* dst, const T* src, size_t n) {
+  for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += gridDim.x * (size_t)256)
+    dst[i] = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// n <= 64 device words into page-locked host memory, where the copy engine and its hand-over take longer.
+__global__ __launch_bounds__(64) void k_words_out(uint32_t* dst, const uint32_t* src, int n) {
+  const int k = threadIdx.x;
+  if (k < n) __hip_atomic_store(dst + k, src[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ============================================================================ allocation
 // Workgroup = a tile of 64 x 16 pixels (16 x 16 in a single frame's launch), 256 lanes, each lane
 // one pixel in each of the tile's 16 x 16 bands, so a workgroup reads and writes whole cache lines
@@ -359,10 +376,14 @@ __device__ void alloc_tile(const FrameArgs& a, uint32_t tile, uint32_t frame, ui
   const int u0 = tx * (16 * kBands) + ((wave & 1) << 3) + (lane & 7);
   const int v = ty * 16 + ((wave >> 1) << 3) + (lane >> 3);
   const uint32_t stripe = tile & (kStripes - 1);
-  const float* Tp = a.poses + 16 * (size_t)fs;
   float T[12];
+  if (kBands > 1 || a.poses) {  // a host frame is a launch of its own
 #pragma unroll
-  for (int k = 0; k < 12; ++k) T[k] = Tp[k];
+    for (int k = 0; k < 12; ++k) T[k] = a.poses[16 * (size_t)fs + k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < 12; ++k) T[k] = a.pose[k];
+  }
   const size_t elem = kU16 ? 2 : 4;
   const void* base = reinterpret_cast<const char*>(a.depth) + (size_t)fs * a.W * a.H * elem;
 
@@ -956,6 +977,12 @@ constexpr int kIntegrateWaves = 4;  // independent workers per workgroup
 // waves (128 VGPRs: at 96 about 50 values spill into the frame loop, 13 % slower).
 #define VH_INTEGRATE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(kColor ? 4 : 6)))
 
+// Entry q of the pose of the batch's frame j (kBatch: of a bound sequence).
+template <bool kBatch>
+__device__ __forceinline__ float pose_entry(const FrameArgs& a, uint32_t cur, uint32_t j, uint32_t q) {
+  return kBatch || a.poses ? a.poses[16 * (size_t)input_slot(cur, j, a.n_seq) + q] : a.pose[q];
+}
+
 // The k poses of a batch (inputs cur .. cur+k-1) into LDS, read by every block of the
 // workgroup's workers (a global load per block and frame would put a memory round trip in
 // front of each frame's projections). All 256 lanes call it.
@@ -963,7 +990,7 @@ __device__ __forceinline__ void stage_poses(const FrameArgs& a, uint32_t cur, ui
   const uint32_t t = threadIdx.x;
   if (t < 12u * k) {
     const uint32_t j = t / 12u, q = t - 12u * j;
-    s_pose[j][q] = a.poses[16 * (size_t)input_slot(cur, j, a.n_seq) + q];
+    s_pose[j][q] = pose_entry<false>(a, cur, j, q);
   }
   __syncthreads();
 }
@@ -1036,7 +1063,7 @@ __device__ __forceinline__ void integrate_group(const FrameArgs& a, uint32_t gro
   float pose = 0.0f;
   if (t < 12u * k) {
     const uint32_t j = t / 12u, q = t - 12u * j;
-    pose = a.poses[16 * (size_t)input_slot(cur, j, a.n_seq) + q];
+    pose = pose_entry<kBatch>(a, cur, j, q);
   }
   const uint32_t my_len = min(list_count_of(a.ctl, parity)[lane * kLine], a.stripe_cap);
   const bool tab = rcp_table_covers(a, a.ctl, k);
@@ -3280,6 +3307,28 @@ static int query_grid(int64_t n) {
   if (g > 4096) g = 4096;
   if (g < 1) g = 1;
   return (int)g;
+}
+
+template <class T>
+static void copy_in(void* dst, const void* src, size_t bytes, hipStream_t st) {
+  const size_t n = bytes / sizeof(T);
+  const int g = (int)(n < 1024 * 256 ? (n + 255) / 256 : 1024);
+  hipLaunchKernelGGL(k_copy_in<T>, dim3(g), dim3(256), 0, st, static_cast<T*>(dst), static_cast<const T*>(src), n);
+}
+// In the widest units that both ends and the length are multiples of.
+hipError_t launch_copy_in(void* dst, const void* src, size_t bytes, hipStream_t st) {
+  if (bytes == 0) return hipSuccess;
+  const size_t m = reinterpret_cast<size_t>(dst) | reinterpret_cast<size_t>(src) | bytes;
+  if (m % 8 == 0) copy_in<uint64_t>(dst, src, bytes, st);
+  else if (m % 4 == 0) copy_in<uint32_t>(dst, src, bytes, st);
+  else if (m % 2 == 0) copy_in<uint16_t>(dst, src, bytes, st);
+  else copy_in<uint8_t>(dst, src, bytes, st);
+  return hipGetLastError();
+}
+
+hipError_t launch_words_out(uint32_t* dst, const uint32_t* src, int n, hipStream_t st) {
+  hipLaunchKernelGGL(k_words_out, dim3(1), dim3(64), 0, st, dst, src, n);
+  return hipGetLastError();
 }
 
 hipError_t launch_query(const QueryArgs& q, int storage, const float* pts, int64_t n, float* sdf, uint8_t* valid,
