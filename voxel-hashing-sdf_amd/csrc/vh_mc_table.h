@@ -15,7 +15,7 @@ namespace vh {
 #if defined(__HIPCC__)
 __device__ __constant__
 #endif
-static const uint64_t kTriTable[256] = {
+static constexpr uint64_t kTriTable[256] = {
     0x0fffffffffffffffull, 0x1ffffffffffff380ull, 0x1ffffffffffff910ull, 0x2fffffffff189381ull,
     0x1ffffffffffffa21ull, 0x2fffffffffa21380ull, 0x2fffffffff920a29ull, 0x3ffffff89a8a2382ull,
     0x1ffffffffffff2b3ull, 0x2fffffffff0b82b0ull, 0x2fffffffffb32091ull, 0x3ffffffb89b912b1ull,
