@@ -3,8 +3,8 @@
 
 Workload (default room_medium_5mm): 500 synthetic 640x480 uint16 depth frames of an
 8x6x3 m room with 12 primitives, 5 mm voxels, 2 cm truncation, 2^21 buckets, 1.5M-block
-pool, FP32 voxels; per frame one captured HIP graph launch integrates frame f and allocates
-frame f+1 (the first allocation and the last integration of a call run alone); marching
+pool, FP32 voxels; one launch per batch of up to 8 frames integrates it and allocates
+the next batch (the first allocation and the last integration of a call run alone); marching
 cubes runs every 100 frames (5 extractions per pass, the last one final). The integration
 kernel's time for the roofline comes from a separate pass in profiling mode, where
 allocation and integration run as their own launches with HIP events around each.
@@ -263,7 +263,7 @@ def main():
                     help="short run for hardware-counter passes: one FP32 integration pass over the "
                          "sequence plus a 1 GiB device copy that calibrates FETCH_SIZE/WRITE_SIZE")
     ap.add_argument("--counters-fused", action="store_true",
-                    help="with --counters: the captured-graph batches (fused integration + allocation launches) "
+                    help="with --counters: the usual batches (fused integration + allocation launches) "
                          "instead of the profiling mode's separate launches")
     ap.add_argument("--counters-mc", action="store_true",
                     help="with --counters: one marching-cubes extraction after the integration pass")
@@ -304,7 +304,7 @@ def main():
         dst.copy_(src)
         torch.cuda.synchronize()
         vol = vh.Volume(vh.config_from_workload(w))
-        # allocation and integration as separate launches per batch, or the fused graph batches
+        # allocation and integration as separate launches per batch, or the fused batches
         vol.set_profiling(2 if args.counters_fused else True)
         run_pass(vol, vh, (d_depth, d_pose), nf, 0, d_xyz, cap, final_mc=args.counters_mc)
         st = vol.stats()
@@ -396,7 +396,7 @@ def main():
         pst = vol.stats()
         vol.set_profiling(False)
         fst = None
-        if name == "f32":  # the fused batch launches of the captured graphs, HIP events around each
+        if name == "f32":  # the fused batch launches, HIP events around each
             vol.set_profiling(2)
             run_pass(vol, vh, (d_depth, d_pose), nf, 0, d_xyz, cap, final_mc=False, **cr)
             fst = vol.stats()
@@ -461,7 +461,7 @@ def main():
 
     # the fused launch (integration of batch b + allocation of batch b+1): algorithmic bytes =
     # the integration's (as above) + the allocation's, one depth image per frame plus 16 B per
-    # touched block (hash probe and list entry); time from HIP events around each graph launch
+    # touched block (hash probe and list entry); time from HIP events around each launch
     roofline_fused = None
     fz = r.get("fused")
     if fz and fz["fused_launches"]:
@@ -486,7 +486,7 @@ def main():
         roofline_fused = dict(bound="hbm", achieved=round(a_f, 1), peak=HBM_PEAK_GBS, unit="GB/s",
                               frac=round(a_f / HBM_PEAK_GBS, 4), traffic=f_traffic, traffic_source=f_src, valu=f_valu,
                               kernel="k_integrate_alloc<F32,u16>", avg_launch_us=round(1e6 * t_f, 2),
-                              timing="HIP events around each captured-graph batch launch on the volume's stream",
+                              timing="HIP events around each batch launch on the volume's stream",
                               bytes_per_launch=int(fused_bytes), launches=fz["fused_launches"])
     out = {"metric": METRIC, "value": round(r["fps"], 2), "unit": "frames/s", "n_gpus": 1, "steps": args.steps,
            "warmup": args.warmup, "ms_per_step": round(r["ms_per_step"], 3), "higher_is_better": True,
@@ -495,7 +495,7 @@ def main():
                       "voxel_m": w["vox_size"], "trunc_m": w["trunc"], "log2_buckets": w["log2_buckets"],
                       "pool_blocks": w["pool_blocks"], "block": 8, "mc_every": mc_every,
                       "depth": "uint16 mm, device-resident",
-                      "per_launch": f"one captured-graph launch per batch of {w.get('seq_batch', 8)} frames: integration of batch b "
+                      "per_launch": f"one launch per batch of {w.get('seq_batch', 8)} frames: integration of batch b "
                                     "(each block read and written once, updated by each of its frames in "
                                     "order) and allocation of batch b+1"},
            "integrate_only_fps": round(r["fps_integrate"], 2), "mc_blocks": r["blocks"],

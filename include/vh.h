@@ -133,9 +133,8 @@ typedef struct vh_stats {
   int64_t carved_total;       /* carving volumes: block-frame updates added by carving (a frame
                                  observes a block that its truncation bands did not cross) */
   double carve_ms;            /* profiling mode: summed carve-pass time */
-  double fused_ms;            /* profiling mode 2: summed time of the fused batch launches (one
-                                 captured graph: integration of a batch and allocation of the
-                                 next), HIP events around each on the volume's stream */
+  double fused_ms;            /* profiling mode 2: summed time of the fused batch launches
+                                 (integration of a batch and allocation of the next), HIP events around each on the volume's stream */
   int64_t fused_launches;     /* profiling mode 2: fused batch launches timed */
 } vh_stats;
 
@@ -201,11 +200,12 @@ int vh_abi_version(void);
  * one). Host buffers are copied before return; the call is synchronous. */
 int vh_integrate(vh_volume* vol, const vh_frame* frame);
 /* Asynchronous variant of vh_integrate (no reference counterpart; processFrame blocks,
- * src/tsdf.cu:1495-1497): the depth (and RGB) is copied on a second stream into one of 4
- * device slots while earlier frames integrate, and the frame's allocation and integration
- * wait for the copy. The call returns after queuing; the buffers must stay unchanged until vh_sync
- * (page-locked memory, e.g. from hipHostMalloc, gives an asynchronous copy; pageable memory
- * is staged by the runtime before the call returns). Overflows are reported by vh_sync. */
+ * src/tsdf.cu:1495-1497): the depth (and RGB) goes into one of 4 device slots, read by a kernel
+ * on the volume's stream (images of up to 1.6 MB a frame) or copied on a second stream while
+ * earlier frames integrate, and the frame's allocation and integration follow it. The call
+ * returns after queuing; the buffers must stay unchanged until vh_sync (page-locked memory, e.g.
+ * from hipHostMalloc, is read where it lies; pageable memory is first copied into page-locked
+ * memory of the volume, before the call returns). Overflows are reported by vh_sync. */
 int vh_integrate_async(vh_volume* vol, const vh_frame* frame);
 
 /* Device-resident input: binds n_frames depth images (tightly packed, device memory,
@@ -233,13 +233,13 @@ int vh_bind_sequence_rgb(vh_volume* vol, const uint8_t* d_rgb);
  * No reference counterpart (the reference takes poses as given, PointCloudGenerator.cpp:93-128). */
 int vh_bind_tracking(vh_volume* vol, const void* d_depth, int32_t depth_format, float depth_scale,
                      int32_t n_frames, const vh_track_config* track);
-/* Enqueues the next n frames of the bound sequence on the volume's stream (one captured
- * HIP graph launch per frame unless profiling is on). Asynchronous; see vh_sync. */
+/* Enqueues the next n frames of the bound sequence on the volume's stream (a launch per batch;
+ * a tracked frame is a captured HIP graph unless profiling is on). Asynchronous; see vh_sync. */
 int vh_integrate_next(vh_volume* vol, int32_t n);
 /* Waits for queued work and reports any pool/hash/range overflow raised by it. */
 int vh_sync(vh_volume* vol);
 /* Profiling mode 1: frames launch eagerly with HIP events around each kernel; the summed
- * kernel times appear in vh_stats. Mode 2: bound sequences run their captured graphs as
+ * kernel times appear in vh_stats. Mode 2: bound sequences run as
  * without profiling, with HIP events around each fused batch launch (vh_stats.fused_ms).
  * 0: off. Switching clears the sums. */
 int vh_set_profiling(vh_volume* vol, int32_t on);

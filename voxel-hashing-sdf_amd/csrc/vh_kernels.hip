@@ -1806,9 +1806,10 @@ __global__ __launch_bounds__(256) void k_mc_neighbours(McArgs a) {
   a.nbrs[i] = nb;
 }
 
-// Bound by the voxels' bytes: 144,600 blocks (FP32, 592 MB and the neighbours' faces, 732 MB fetched)
-// take 202 us, 3.6 TB/s; asking mc_crossed first and leaving out the values and the near-zero
-// bits took a third of the instructions out and left the time as it was.
+// Bound by the lines it fetches: 144,600 blocks (FP32) take 202 us and fetch about 1.4 GB for 592 MB of
+// own voxels, since the +z face and the edges touch a line per value. Asking mc_crossed first and
+// leaving out the values and the near-zero bits took a third of the instructions out and left the
+// time as it was.
 template <int kStorage>
 __global__ __launch_bounds__(64 * kMcWaves) void k_mc_count(McArgs a) {
   __shared__ McShared SS[kMcWaves];
@@ -2781,7 +2782,8 @@ __device__ __forceinline__ void gn_add(const GnArgs& a, const double* pose, cons
 //   sample, 1,536 points at a time, into LDS, and 8 of them add those up in order; a sampling wave
 //   doesn't hold the 31 FP64 sums (62 registers), so twice as many lookups are in flight
 //   as with both in one loop.
-// Workgroups take neighbouring points by XCD (xcd_chunk): 300,000 points fetched 48 MB, now 19.
+// Workgroups take neighbouring points by XCD (xcd_chunk): 300,000 points made 0.70e6 read requests beyond
+// the L2, now 0.29e6.
 // Measured, per evaluation: 19,200 points (F16) 12.4 -> 8.9 us, 300,000 (FP32) 35.0 -> 23.3 us;
 // 3.5 and 3.3 us of that by the step's shorter chain (gn_step) and the prior's own wave.
 struct GnStepOut {

@@ -414,8 +414,8 @@ class Volume:
             self._pending = []
 
     def set_profiling(self, on):
-        """False/0: off; True/1: eager launches with events around each kernel; 2: the captured
-        graphs with events around each fused batch launch (stats fused_ms, fused_launches)."""
+        """False/0: off; True/1: eager launches with events around each kernel; 2: the usual
+        launches with events around each fused batch launch (stats fused_ms, fused_launches)."""
         _check(_lib.vh_set_profiling(self._h, 2 if on == 2 else (1 if on else 0)))
 
     def stats(self) -> dict:
