@@ -304,7 +304,7 @@ struct GnState {
 // per-evaluation stats: n_valid, rms, |delta|, lambda, accepted, accepted pose (12)
 constexpr int kGnStats = 17;
 
-// Starting pose (row-major 3x4) and damping of a refinement (k_gn_start).
+// Starting pose (row-major 3x4) and damping of a refinement.
 struct GnStart {
   double pose[12];
   double lambda;
@@ -340,7 +340,8 @@ struct GnArgs {
   float mu;           // truncation (metres): residual scale of the noise model
   const float* pts;   // camera-frame points (a non-finite coordinate marks a point to skip)
   int64_t n;
-  const double* pose; // without a previous evaluation: the pose to evaluate (12 doubles, 3x4)
+  GnStart start;      // without a previous evaluation: the pose to evaluate, and the damping
+  GnState* st_start;  // and the state they begin (written by workgroup 0)
   double* partials;   // grid * kGnAcc
   int grid;           // partial sums of this evaluation
   // the previous evaluation, stepped from at the start of the launch (prev_grid = 0: none)
@@ -386,7 +387,8 @@ hipError_t launch_stream_rehash(const StreamArgs& a, hipStream_t st);
 // which).
 hipError_t launch_stream_insert(const StreamArgs& a, int storage, hipStream_t st);
 hipError_t launch_copy_in(void* dst, const void* src, size_t bytes, hipStream_t st);
-hipError_t launch_words_out(uint32_t* dst, const uint32_t* src, int n, hipStream_t st);
+// na words of a, then nb of b, into page-locked host memory.
+hipError_t launch_words_out(uint32_t* dst, const void* a, int na, const void* b, int nb, hipStream_t st);
 hipError_t launch_query(const QueryArgs& q, int storage, const float* pts, int64_t n, float* sdf,
                         uint8_t* valid, hipStream_t st);
 hipError_t launch_backward(const QueryArgs& q, int storage, const float* pts, int64_t n,
@@ -400,7 +402,6 @@ hipError_t launch_gn_solve(const double* partials, int grid, const GnState* st_i
 hipError_t launch_track_solve(const double* partials, int grid, const GnState* st_in, GnState* st_out, double* cand,
                               const TrackArgs& t, hipStream_t st);
 // cand = s.pose, solver state cleared with damping s.lambda.
-hipError_t launch_gn_start(const GnStart& s, GnState* state, double* cand, hipStream_t st);
 // Gauss-Newton state reset + prior pose of the current frame, and the depth back-projection,
 // in one launch.
 // Accepted pose (and the frame's solver stats) to the per-frame outputs.

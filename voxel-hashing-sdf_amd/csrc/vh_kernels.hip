@@ -87,10 +87,10 @@ __global__ __launch_bounds__(256) void k_copy_in(T* dst, const T* src, size_t n)
     dst[i] = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// n <= 64 device words into page-locked host memory, where the copy engine and its hand-over take longer.
-__global__ __launch_bounds__(64) void k_words_out(uint32_t* dst, const uint32_t* src, int n) {
-  const int k = threadIdx.x;
-  if (k < n) __hip_atomic_store(dst + k, src[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+// Device words into page-locked host memory, where the copy engine and its hand-over take longer.
+__global__ __launch_bounds__(256) void k_words_out(uint32_t* dst, const uint32_t* a, int na, const uint32_t* b, int nb) {
+  for (int k = threadIdx.x; k < na + nb; k += 256)
+    __hip_atomic_store(dst + k, k < na ? a[k] : b[k - na], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ============================================================================ allocation
@@ -2771,7 +2771,7 @@ __device__ __forceinline__ void gn_add(const GnArgs& a, const double* pose, cons
 // Levenberg-Marquardt step itself (gn_solve_wg over the previous partials: the same sums in
 // the same order, so every workgroup gets the same candidate; workgroup 0 stores the state,
 // the candidate and the stats row), which saves a launch per evaluation and needs no ordering
-// between workgroups; otherwise the candidate is a.pose.
+// between workgroups; otherwise the candidate is a.start.pose.
 //
 // Partial sum b of the a.grid is over the points b 256 + t (t < 256), and every a.grid 256th
 // after them, added in order per t. What bounds an evaluation is latency: of the step's serial FP64
@@ -2797,6 +2797,19 @@ __device__ __forceinline__ GnStepOut gn_step_out(const GnArgs& a) {
 template <int kThreads>
 __device__ __forceinline__ void gn_solve_wg(const double* partials, int grid, const GnState* st_in, const GnStepOut& out,
                                             double* s_cand, int final_step);
+// Start of a refinement: the first evaluation's pose comes with its launch, and workgroup 0 clears the solver
+// state to it and the initial damping (all words of the state: 69).
+__device__ __forceinline__ void gn_start(const GnArgs& a, double* s_pose) {
+  constexpr int kWords = (int)(sizeof(GnState) / sizeof(double)), kCand = (int)(offsetof(GnState, cand) / sizeof(double)),
+                kLambda = (int)(offsetof(GnState, lambda) / sizeof(double));
+  const int t = threadIdx.x;
+  if (t < 12) s_pose[t] = a.start.pose[t];
+  if (blockIdx.x == 0 && t < kWords) {
+    double v = t == kLambda ? a.start.lambda : 0.0;
+    if (t >= kCand && t < kCand + 12) v = a.start.pose[t - kCand];
+    reinterpret_cast<double*>(a.st_start)[t] = v;
+  }
+}
 template <int kThreads>
 __device__ __forceinline__ void gn_pose(const GnArgs& a, uint32_t fs, double* s_pose) {
   if (a.prev_grid > 0) {
@@ -2804,7 +2817,7 @@ __device__ __forceinline__ void gn_pose(const GnArgs& a, uint32_t fs, double* s_
     return;
   }
   if (a.track) track_start(a.t, fs, s_pose);
-  else if (threadIdx.x < 12) s_pose[threadIdx.x] = a.pose[threadIdx.x];
+  else gn_start(a, s_pose);
   __syncthreads();
 }
 
@@ -3190,21 +3203,6 @@ __global__ __launch_bounds__(kThreads) void k_track_solve(const double* partials
   if (k < 16) t.out[16 * (size_t)fs + k] = k < 12 ? (float)s_cand[k] : (k == 15 ? 1.0f : 0.0f);
 }
 
-// Start of a refinement: the candidate is the starting pose and the solver state is cleared
-// with the initial damping. The pose comes in by value (kernel argument), so starting a
-// refinement needs no host-to-device copy.
-__global__ __launch_bounds__(64) void k_gn_start(GnStart s, GnState* st, double* cand) {
-  const int k = threadIdx.x;
-  if (k == 0) {
-    GnState z{};
-    z.lambda = s.lambda;
-#pragma unroll
-    for (int q = 0; q < 12; ++q) z.cand[q] = s.pose[q];
-    *st = z;
-  }
-  if (k < 12) cand[k] = s.pose[k];
-}
-
 }  // namespace
 
 // ============================================================================ launchers
@@ -3382,8 +3380,9 @@ hipError_t launch_copy_in(void* dst, const void* src, size_t bytes, hipStream_t 
   return hipGetLastError();
 }
 
-hipError_t launch_words_out(uint32_t* dst, const uint32_t* src, int n, hipStream_t st) {
-  hipLaunchKernelGGL(k_words_out, dim3(1), dim3(64), 0, st, dst, src, n);
+hipError_t launch_words_out(uint32_t* dst, const void* a, int na, const void* b, int nb, hipStream_t st) {
+  hipLaunchKernelGGL(k_words_out, dim3(1), dim3(256), 0, st, dst, static_cast<const uint32_t*>(a), na,
+                     static_cast<const uint32_t*>(b), nb);
   return hipGetLastError();
 }
 
@@ -3433,11 +3432,6 @@ hipError_t launch_track_solve(const double* partials, int grid, const GnState* s
                               const TrackArgs& t, hipStream_t st) {
   if (grid <= 128) hipLaunchKernelGGL(k_track_solve<kGnThreads>, dim3(1), dim3(kGnThreads), 0, st, partials, grid, st_in, st_out, cand, t);
   else hipLaunchKernelGGL(k_track_solve<kGnWideThreads>, dim3(1), dim3(kGnWideThreads), 0, st, partials, grid, st_in, st_out, cand, t);
-  return hipGetLastError();
-}
-
-hipError_t launch_gn_start(const GnStart& s, GnState* state, double* cand, hipStream_t st) {
-  hipLaunchKernelGGL(k_gn_start, dim3(1), dim3(64), 0, st, s, state, cand);
   return hipGetLastError();
 }
 
