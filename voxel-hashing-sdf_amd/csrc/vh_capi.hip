@@ -1,11 +1,10 @@
 // vh_capi.hip - extern "C" entry points of libvh (see include/vh.h).
 //
 // One volume owns one HIP stream (default priority) and all of its device memory. The
-// per-frame pipeline (k_alloc -> k_integrate, preceded for tracked sequences by the
-// back-projection and the Gauss-Newton iterations) is captured once into a HIP graph per
-// input kind (host-staged frames, bound device sequence, tracked sequence); its kernels read
-// the frame index and counters from device memory, so a launch needs no host-side parameter
-// updates.
+// per-frame pipeline (k_alloc -> k_integrate) is launched as it is for host frames and batches
+// of a bound sequence; a tracked frame (the Gauss-Newton evaluations in front) is captured once
+// into a HIP graph. The kernels read the frame index and counters from device memory, so a
+// replay needs no host-side parameter updates.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

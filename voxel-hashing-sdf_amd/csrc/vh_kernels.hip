@@ -1,6 +1,6 @@
 // vh_kernels.hip - gfx950 kernels of libvh.
 //
-// Per batch of k consecutive frames (one captured graph per launch): k_alloc (one lane per
+// Per batch of k consecutive frames: k_alloc (one lane per
 // pixel of each frame: truncation-band DDA, hash insert, per-frame marks, compaction of the
 // batch's block list) -> k_integrate (one wave per listed block, grid-stride: the block's
 // voxels are read once, updated by each frame that touched it, written once; the last
@@ -1528,7 +1528,7 @@ __device__ __forceinline__ void mc_stage(const McArgs& a, uint32_t b, uint32_t n
 // triangles iff its 8 corners are observed and its case is not 0 or 255 (bit c set iff
 // corner c < 0, reference corner order); its case goes to S.cases. Returns the lane's table
 // triangle count. near: bit x set iff cube x of the column has triangles and a corner with
-// |value| < tiny (the kTiny bits of mc_stage; see mc_count_exact).
+// |value| < tiny (the kTiny bits of mc_put_columns; see mc_count_exact).
 __device__ __forceinline__ uint32_t mc_classify(McShared& S, uint32_t& near) {
   const int lane = mc_lane(), i = (lane >> 3) * 9 + (lane & 7);
   const uint64_t w0 = S.col[i], w1 = S.col[i + 1], w2 = S.col[i + 9], w3 = S.col[i + 10];
@@ -2775,7 +2775,7 @@ __device__ __forceinline__ void gn_add(const GnArgs& a, const double* pose, cons
 //
 // Partial sum b of the a.grid is over the points b 256 + t (t < 256), and every a.grid 256th
 // after them, added in order per t. What bounds an evaluation is latency: of the step's serial FP64
-// chain and of the points' lookups. Two launch shapes (gn_shape):
+// chain and of the points' lookups. Two launch shapes (launch_gn_accum):
 // - k_gn_accum, while each point has a lane of its own: a workgroup of 256 per partial sum, one point
 //   to a lane, loaded before the step; a fifth wave takes the motion prior's part of the step.
 // - k_gn_accum_wide above: 16 waves, two partial sums a workgroup, a workgroup per CU. All waves
