@@ -1123,7 +1123,10 @@ hipError_t copy_image(void* dst, const void* from, const void* src, size_t row, 
                       hipStream_t st) {
   if (from && direct) {
     hipPointerAttribute_t a{};
-    if (hipPointerGetAttributes(&a, from) == hipSuccess && a.devicePointer) return launch_copy_in(dst, a.devicePointer, row * rows, st);
+    int device = -1;
+    if (hipPointerGetAttributes(&a, from) == hipSuccess && hipGetDevice(&device) == hipSuccess && a.devicePointer &&
+        a.device == device)  // mapped for this GPU
+      return launch_copy_in(dst, a.devicePointer, row * rows, st);
     (void)hipGetLastError();
   }
   if (from) return hipMemcpyAsync(dst, from, row * rows, hipMemcpyHostToDevice, st);
