@@ -129,3 +129,39 @@ def test_solver_counts(vh, oracle, n):
     want, _ = lm_reference(ref, kept, T0, 2, w["trunc"])
     assert np.abs(T - want).max() < 1e-6
     vol.close()
+
+
+# 80 x 60 and 640 x 480 points of a tracked frame: one point per lane, and several; uint16 and float depth
+@pytest.mark.parametrize("W,H,stride,fmt", [(320, 240, 4, 0), (320, 240, 1, 0), (640, 480, 1, 0), (640, 480, 1, 1)])
+def test_tracked_frame_equals_refinement(vh, oracle, W, H, stride, fmt):
+    """A tracked frame without a motion prior runs the refinement's arithmetic on its own back-projected
+    points: its pose is the refinement's, rounded to FP32, bit for bit."""
+    import torch
+
+    s = W / 320
+    w = dict(workload(), width=W, height=H, fx=260.0 * s, fy=262.0 * s, cx=159.3 * s, cy=119.6 * s)
+    v, u = np.mgrid[0:H, 0:W]
+    d = (1100 + (2 * u + 1.5 * v) / s + 180 * ((u // 40 + v // 30) % 2)).astype(np.uint16)
+    d[(u // 16 + v // 12) % 11 == 0] = 0
+    metres = d.astype(np.float32) * np.float32(0.001)
+    a, b = (vh.Volume(vh.config_from_workload(w)) for _ in range(2))
+    for vol in (a, b):
+        vol.integrate(d, look_down_z(0.0, 0.0, 0.0))
+    prior = look_down_z(0.002, -0.001, 0.003)
+    dd = torch.from_numpy(metres if fmt else d.view(np.int16)).cuda()[None].contiguous()
+    pr, out = torch.from_numpy(prior).cuda()[None].contiguous(), torch.zeros(1, 4, 4, device="cuda")
+    torch.cuda.synchronize()
+    a.bind_tracking(dd, vh.DEPTH_F32 if fmt else vh.DEPTH_U16, 1.0 if fmt else 0.001, 1, pr, out, None, gn_iters=4,
+                    point_stride=stride)
+    a.integrate_next(1)
+    a.sync()
+    z = metres[::stride, ::stride]
+    uu, vv = (c[::stride, ::stride].astype(np.float32) for c in (u, v))
+    x = ((uu - np.float32(w["cx"])) * z) / np.float32(w["fx"])
+    y = ((vv - np.float32(w["cy"])) * z) / np.float32(w["fy"])
+    pts = np.stack([x, y, z], -1).reshape(-1, 3)
+    pts[z.reshape(-1) == 0] = np.nan
+    T, _ = b.gn_refine(pts, prior, 4)
+    assert np.array_equal(out.cpu().numpy()[0].view(np.uint32), T.astype(np.float32).view(np.uint32))
+    a.close()
+    b.close()
