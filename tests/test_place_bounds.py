@@ -1,0 +1,70 @@
+"""A block with a corner at the camera: the integration leaves out the checks per voxel only where the
+corners' pixels bound the voxels' (near_depth, csrc/vh_math.h). On the host (tests/host_checks/place_bounds.cpp):
+no voxel outside its block's rectangle, and some without the bound. On the GPU: cameras of a wide field
+of view on and by lattice points inside the map, identical to the oracle (no tolerance)."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from conftest import ROOT
+from test_gpu_integration import assert_same_volume
+
+
+def test_corners_bound_the_voxels(tmp_path):
+    src = os.path.join(ROOT, "tests", "host_checks", "place_bounds.cpp")
+    exe = str(tmp_path / "place_bounds")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-I", os.path.join(ROOT, "voxel-hashing-sdf_amd", "csrc"),
+                    "-I", os.path.join(ROOT, "include"), "-o", exe, src], check=True, timeout=120)
+    inside, near, out = map(int, subprocess.run([exe], capture_output=True, text=True, timeout=120, check=True).stdout.split())
+    assert inside > 20_000 and near > 1_000 and out == 0
+    assert int(subprocess.run([exe, "without"], capture_output=True, text=True, timeout=120, check=True).stdout.split()[2]) > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("storage,color", [(0, 0), (1, 0), (2, 1)])
+@pytest.mark.parametrize("away", [0.0, 1e-9, 3e-7, 1e-5, 2e-3])
+def test_camera_on_a_lattice_point(vh, oracle, storage, color, away):
+    import torch
+
+    from test_gpu_color import assert_same_colour_volume
+
+    W, H, vox = 64, 48, 0.03125
+    print(f"{away} m behind lattice points, storage {storage}, colour {color}", flush=True)
+    w = dict(width=W, height=H, fx=5.0, fy=6.0, cx=31.3, cy=23.9, min_depth=0.05, max_depth=6.0, vox_size=vox, trunc=4 * vox,
+             log2_buckets=15, pool_blocks=1 << 16, storage=storage, weight_cap=255 if storage else 0, color=color, carve=1)
+    rng = np.random.default_rng(5)
+    n = 24
+    mm = rng.integers(400, 900, (n, H, W), dtype=np.uint16)
+    rgb = rng.integers(0, 256, (n, H, W, 3), dtype=np.uint8)
+    T = np.tile(np.eye(4, dtype=np.float32), (n, 1, 1))
+    for k in range(1, n):  # into the blocks that the first frame made
+        at = 8 * rng.integers(-2, 3, 3) + 7 * rng.integers(0, 2, 3)
+        if k % 3 == 0:
+            R = np.eye(3)[rng.permutation(3)] * rng.choice([-1.0, 1.0], 3)[:, None]
+            R[:, 0] *= np.linalg.det(R)
+        else:
+            R = np.linalg.qr(rng.normal(0, 1, (3, 3)))[0]
+            R[:, 0] *= np.linalg.det(R)
+        T[k, :3, :3] = R
+        T[k, :3, 3] = at * vox - away * R[:, 2]
+    ref = oracle.Oracle(w, color=bool(color))
+    for k in range(n):
+        ref.integrate(mm[k], T[k], rgb=rgb[k] if color else None)
+    same = assert_same_colour_volume if color else assert_same_volume
+    batch = vh.Volume(vh.config_from_workload(w))
+    d_depth, d_pose, d_rgb = torch.from_numpy(mm.view(np.int16)).cuda(), torch.from_numpy(T).cuda(), torch.from_numpy(rgb).cuda()
+    torch.cuda.synchronize()
+    batch.bind_sequence(d_depth, vh.DEPTH_U16, 0.001, d_pose, n)
+    if color:
+        batch.bind_sequence_rgb(d_rgb)
+    batch.integrate_next(n)
+    batch.sync()
+    same(oracle, batch, ref)
+    batch.close()
+    single = vh.Volume(vh.config_from_workload(w))
+    for k in range(n):
+        single.integrate(mm[k], T[k], rgb=rgb[k] if color else None)
+    same(oracle, single, ref)
+    single.close()

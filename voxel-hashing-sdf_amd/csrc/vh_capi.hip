@@ -249,6 +249,7 @@ FrameArgs frame_args(vh_volume* v, int which, const vh_frame* host = nullptr) {
   a.vox = c.vox_size;
   a.bsz = c.vox_size * (float)kB;
   a.band = band_scale(a.K, a.bsz);
+  a.near = near_image(c.width, c.height);
   a.mu = c.trunc;
   a.inv_mu = 1.0f / c.trunc;
   a.cap = c.weight_cap > 0 ? (float)c.weight_cap : INFINITY;

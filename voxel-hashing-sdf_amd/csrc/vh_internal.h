@@ -109,6 +109,7 @@ struct FrameArgs {
   int32_t pitch;   // row pitch of dm and rgba in pixels: W rounded up to a multiple of 4
   Intr K;
   BandScale band;  // reciprocals for the band setup
+  float near;      // near_image
   float max_depth, min_depth, vox, bsz, mu, inv_mu;
   float cap;  // weight cap, +inf when uncapped
   // tables

@@ -525,12 +525,13 @@ __device__ __forceinline__ int32_t oct_max(int32_t x) {
 // offset), so one pass over the lanes places the block in every frame of the batch (a pass per
 // frame spent about 75 vector instructions on wave-uniform values in each). The block's lattice
 // box is the convex hull of its corners. For depths > 0 the perspective image of a convex
-// combination is a convex combination of the images, and a voxel's own projection differs from
-// the exact one, as the corners' do, by far less than 1/2 pixel. So if every corner has z in
-// [2^-60, 2^60], every voxel's z lies in [2^-64, 2^64], and with umin, umax the least and
-// largest u = X/z of the corners a voxel's pixel round(u) lies in [round(umin - 1/2),
-// round(umax + 1/2)] (for errors below 1/2 these roundings cannot cross the voxel's); likewise
-// v. That rectangle, its left edge moved down to a multiple of 4 pixels, is the block's window.
+// combination is a convex combination of the images, and where every corner's z is at least
+// near_depth, a voxel's own projection and the corners' each differ from the exact ones by less
+// than 1/8 pixel. So if every corner also has z in [2^-60, 2^60], every voxel's z lies in
+// [2^-64, 2^64], and with umin, umax the least and largest u = X/z of the corners a voxel's
+// pixel round(u) lies in [round(umin - 1/2), round(umax + 1/2)] (for errors below 1/2 these
+// roundings cannot cross the voxel's); likewise v. A corner nearer than that (640 x 480, a block 1 m
+// from the camera: 1 cm) leaves the block to the checks per voxel. That rectangle, its left edge moved down to a multiple of 4 pixels, is the block's window.
 // kPlaceEdge unless the rectangle lies inside the image; then kPlaceWindow when it fits kWin at
 // a pitch of at most 64 pixels, else kPlaceInside. The bounds are the bits of (u -+ 1/2) + M as
 // signed integers: for positive sums below 2^24 they are M's plus the rounded bound, larger
@@ -539,11 +540,11 @@ struct Placement {
   uint32_t first, bias;  // DepthWindow's
   uint32_t desc;         // placement | shift << 2 | cols << 5 | rows << 12
 };
-__device__ __forceinline__ Placement block_place(const FrameArgs& a, const float hb[3], const float off[3]) {
+__device__ __forceinline__ Placement block_place(const FrameArgs& a, const float hb[3], const float off[3], float steps) {
   const float z = hb[2] + off[2];
   const float iz = __builtin_amdgcn_rcpf(z);  // within 1 ulp: the bounds leave 1/2 pixel
   const float u = (hb[0] + off[0]) * iz, v = (hb[1] + off[1]) * iz;
-  const uint64_t zin = __builtin_amdgcn_ballot_w64((z >= 0x1p-60f) & (z <= 0x1p60f));
+  const uint64_t zin = __builtin_amdgcn_ballot_w64((z >= near_depth(steps, hb, a.near)) & (z >= 0x1p-60f) & (z <= 0x1p60f));
   const int32_t lu = oct_min((int32_t)__float_as_uint((u - 0.5f) + kPixMagic));
   const int32_t hu = oct_max((int32_t)__float_as_uint((u + 0.5f) + kPixMagic));
   const int32_t lv = oct_min((int32_t)__float_as_uint((v - 0.5f) + kPixMagic));
@@ -744,7 +745,8 @@ __device__ __forceinline__ void frame_update(const FrameArgs& a, uint32_t place,
 }
 
 // Per frame of a batch, staged in LDS by stage_frames: the pose (row-major 3x4) and the
-// frame's homogeneous voxel steps (block_frame_h), each padded to 16 bytes.
+// frame's homogeneous voxel steps (block_frame_h), each padded to 16 bytes; ax[3] holds their
+// near_steps.
 struct __align__(16) FrameLds {
   float T[12];
   float ax[4], ay[4], az[4];
@@ -784,6 +786,7 @@ __device__ void integrate_worker(const FrameArgs& a, uint32_t worker, uint32_t w
     for (int r = 0; r < 3; ++r)
       corner[r] = __builtin_fmaf(c0, s_frm[jl].ax[r], __builtin_fmaf(c1, s_frm[jl].ay[r], c2 * s_frm[jl].az[r]));
   }
+
 
   // Lane j fetches the list entry, slot value, key and mark of this worker's j-th block
   // (clearing the mark for the next batch of this parity) and parks them in LDS, so the
@@ -851,7 +854,7 @@ __device__ void integrate_worker(const FrameArgs& a, uint32_t worker, uint32_t w
           for (int q = 0; q < 12; ++q) T[q] = s_frm[jl].T[q];
           block_origin_cam(T, a.vox, bx, by, bz, cb);
           to_pixel_h(a.K, cb, hb);
-          pl = block_place(a, hb, corner);
+          pl = block_place(a, hb, corner, s_frm[jl].ax[3]);
         }
 #pragma unroll
         for (int q = 0; q < 8; ++q) vx.load(q, old[q]);
@@ -1021,6 +1024,7 @@ __device__ __forceinline__ void stage_frames(const FrameArgs& a, float pose, uin
         s_frm[j].ax[r] = h.ax[r];
         s_frm[j].ay[r] = h.ay[r];
         s_frm[j].az[r] = h.az[r];
+        if (r == 0) s_frm[j].ax[3] = near_steps(h, a.near);
       }
       s_col[j].off[lane][r] = __builtin_fmaf((float)(lane >> 3), h.ay[r], (float)(lane & 7u) * h.az[r]);
     }

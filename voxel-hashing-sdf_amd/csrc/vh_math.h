@@ -133,6 +133,24 @@ VH_HD void block_frame_h(const float* T, float vox, const Intr& K, BlockFrame& f
 // The column (j, i) of a block whose origin is at cb (homogeneous) lies at cb + fma(j, b, i c) with
 // the frame's homogeneous steps b, c along y and z; voxel k of it at fma(k, a, column).
 
+// Least depth z of a block's 8 corners from which the corners' pixels bound the voxels': a corner is
+// formed as o + fma(c0, a, fma(c1, b, c2 c)) from the homogeneous block origin o, a voxel as fma(k, a,
+// o + fma(j, b, i c)), four roundings each. With m[r] = |o[r]| + 7 (|a[r]| + |b[r]| + |c[r]|) either lies
+// within e[r] = 2^-22 m[r] of the exact point, and its pixel within (e[0] + W e[2]) / z (columns;
+// rows likewise) of the exact one where z is large against e[2]. Depths of at least
+// 16 (e[0] + e[1] + (W + H) e[2]) keep each of the two below 1/8 pixel, and every voxel's z above 3/4 of the
+// least corner's. near_image: the image's part of it, near_steps: the frame's, near_depth: with a block's
+// origin (NaN fails any comparison with it).
+VH_HD float near_image(int W, int H) { return 0x1p-18f * (float)(W + H); }
+VH_HD float near_steps(const BlockFrame& f, float image) {
+  float m[3];
+  for (int r = 0; r < 3; ++r) m[r] = 7.0f * (fabsf(f.ax[r]) + fabsf(f.ay[r]) + fabsf(f.az[r]));
+  return fmaf(image, m[2], 0x1p-18f * (m[0] + m[1]));
+}
+VH_HD float near_depth(float steps, const float o[3], float image) {
+  return fmaf(image, fabsf(o[2]), fmaf(0x1p-18f, fabsf(o[0]) + fabsf(o[1]), steps));
+}
+
 // Observation of the voxel at homogeneous point (X, Y, z) (reference IntegrateHashKernel skip
 // rules, src/tsdf.cu:706-738), in two steps so that a caller can issue all depth fetches of a
 // block before using any of them:
