@@ -1067,16 +1067,26 @@ int scratch_for_device(int device, double** out) {
 // first copied, rows together, into page-locked memory of the volume; anything else the runtime knows
 // (device or managed memory) is left to its own 2D copy. The runtime's 2D copy goes row by row from
 // pageable memory, and from page-locked memory where rows aren't whole words: a 640 x 480 frame of
-// uint16 took 4.5 ms (and 20 to 97 ms at odd widths), through page-locked memory 0.1.
+// uint16 took 4.5 ms (and 20 to 97 ms at odd widths), through page-locked memory 0.1. Page-locked is
+// an image that lies whole in one allocation, mapped for the GPU: one that runs past its allocation's end
+// (ordinary memory may follow it) is read by the host.
 enum class HostMemory { kLocked, kPageable, kOther };
-HostMemory memory_of(const void* p) {
+HostMemory memory_of(const void* p, size_t bytes) {
   hipPointerAttribute_t a{};
   if (hipPointerGetAttributes(&a, p) != hipSuccess) {
     (void)hipGetLastError();  // an address the runtime doesn't know
     return HostMemory::kPageable;
   }
   if (a.type == hipMemoryTypeUnregistered) return HostMemory::kPageable;
-  return a.type == hipMemoryTypeHost ? HostMemory::kLocked : HostMemory::kOther;
+  if (a.type != hipMemoryTypeHost) return HostMemory::kOther;
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (!a.devicePointer || hipMemGetAddressRange(&base, &size, a.devicePointer) != hipSuccess) {
+    (void)hipGetLastError();
+    return HostMemory::kPageable;
+  }
+  const size_t before = (size_t)(static_cast<char*>(a.devicePointer) - static_cast<char*>(base));
+  return before <= size && bytes <= size - before ? HostMemory::kLocked : HostMemory::kPageable;
 }
 
 // *buf: `bytes` of page-locked memory, allocated once; null if there is none left (the caller then copies as
@@ -1101,7 +1111,7 @@ void copy_rows(char* dst, const void* src, size_t row, size_t pitch, size_t rows
 // The image as contiguous page-locked bytes: the caller's own, or `offset` into the volume's *buf, of `bytes`
 // bytes; null: to be copied from the caller's rows as the runtime does.
 const void* host_image(const void* src, size_t row, size_t pitch, size_t rows, char** buf, size_t bytes, size_t offset) {
-  const HostMemory m = memory_of(src);
+  const HostMemory m = memory_of(src, pitch * (rows - 1) + row);
   if (m == HostMemory::kOther) return nullptr;
   if (m == HostMemory::kLocked) {
     if (pitch == row) return src;
@@ -1131,7 +1141,7 @@ hipError_t copy_image(void* dst, const void* from, const void* src, size_t row, 
     (void)hipGetLastError();
   }
   if (from) return hipMemcpyAsync(dst, from, row * rows, hipMemcpyHostToDevice, st);
-  if (pitch == row && memory_of(src) != HostMemory::kOther) return hipMemcpyAsync(dst, src, row * rows, hipMemcpyHostToDevice, st);
+  if (pitch == row && memory_of(src, row * rows) != HostMemory::kOther) return hipMemcpyAsync(dst, src, row * rows, hipMemcpyHostToDevice, st);
   return hipMemcpy2DAsync(dst, row, src, pitch, row, rows, hipMemcpyHostToDevice, st);
 }
 
