@@ -1122,11 +1122,17 @@ const void* host_image(const void* src, size_t row, size_t pitch, size_t rows, c
   return b ? b + offset : nullptr;
 }
 
-// Images of a frame up to here are read by a kernel in the frame's own stream (k_copy_in), larger ones by
-// the copy engine on the copy stream, where the copy overlaps the kernels of the frame before. The
-// overlap costs the host and the streams' waits 64 us a frame (640 x 480 uint16, queued), the bus moves
-// 1.6 MB in 36 us, and a frame's kernels take 25; the small frame takes 46 us in one stream.
+// Images of a frame up to here are read by a kernel in the frame's own stream (k_copy_in), larger ones
+// copied by the runtime: for a frame that the call waits for in that stream too, for a queued frame on the
+// copy stream, where the copy overlaps the kernels of the frame before. Queued, the overlap costs waits
+// between the streams, the kernel its time on the bus: a frame into a room at 5 mm (binary16; us by the copy
+// stream / by the kernel) 150 KB 36 / 31, 600 KB 37 / 40, 938 KB 40 / 48, 1.2 MB 41 / 52, 1.5 MB 49 / 65.
+// With three volumes in use, whose six streams share four hardware queues, 600 KB 43 to 62 / 41, 938 KB 50 to 70 /
+// 48, 1.2 MB 44 to 63 / 52: so the kernel up to 1 MB, where it is also no slower than the copy
+// stream with a graph of the frame's kernels was (48). Waited for, the kernel is the faster at every size (640 x 480 float
+// 62 us, 64 by a copy; 1280 x 960 137 and 141); 1.6 MB leaves the bus to the copy engine above.
 constexpr size_t kDirectBytes = 1600 * 1024;
+constexpr size_t kDirectQueuedBytes = 1024 * 1024;
 
 // An image to the device: `from`, its contiguous page-locked bytes (read by a kernel if direct), or where that
 // is null the caller's rows.
@@ -1140,6 +1146,10 @@ hipError_t copy_image(void* dst, const void* from, const void* src, size_t row, 
       return launch_copy_in(dst, a.devicePointer, row * rows, st);
     (void)hipGetLastError();
   }
+  // in whole words the runtime's 2D copy: its plain copy takes up to half as long again at some sizes of
+  // 0.8 to 6 MB (queued frames, 1.9 MB: 79 us against 54)
+  if (from && ((row | reinterpret_cast<uintptr_t>(from) | reinterpret_cast<uintptr_t>(dst)) & 3) == 0)
+    return hipMemcpy2DAsync(dst, row, from, row, row, rows, hipMemcpyHostToDevice, st);
   if (from) return hipMemcpyAsync(dst, from, row * rows, hipMemcpyHostToDevice, st);
   if (pitch == row && memory_of(src, row * rows) != HostMemory::kOther) return hipMemcpyAsync(dst, src, row * rows, hipMemcpyHostToDevice, st);
   return hipMemcpy2DAsync(dst, row, src, pitch, row, rows, hipMemcpyHostToDevice, st);
@@ -1318,9 +1328,9 @@ int vh_integrate_async(vh_volume* v, const vh_frame* f) {
   if (v->ring_format >= 0 && v->ring_format != f->depth_format) VH_HIP(hipStreamSynchronize(v->stream));
   v->ring_format = f->depth_format;
   const int slot = (int)(v->ring_next % R);
-  const size_t rows = (size_t)v->cfg.height, slot_bytes = frame_px * (v->colors ? 7 : 4);
+  const size_t rows = (size_t)v->cfg.height, slot_bytes = (frame_px * (v->colors ? 7 : 4) + 7) & ~(size_t)7;
   const size_t line = (size_t)v->cfg.width * 3;
-  const bool direct = rows * (row + (v->colors ? line : 0)) <= kDirectBytes;
+  const bool direct = rows * (row + (v->colors ? line : 0)) <= kDirectQueuedBytes;
   const hipStream_t copies = direct ? v->stream : v->copy_stream;
   if (v->ring_held[slot]) VH_HIP(hipEventSynchronize(v->ring_copied[slot]));
   if (!direct) {  // the copy waits for the frame that read the slot
