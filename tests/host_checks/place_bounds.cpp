@@ -3,8 +3,9 @@
 // degrees to nearly 180, images from 1 x 1 to 16384 x 16384 and the corners' reciprocals off by up to
 // 1 ulp, the block's rectangle is formed as the kernel forms it (block_place); wherever that puts it inside
 // the image, every voxel's z has to lie in the range of the kernel's reciprocal and its pixel in the rectangle.
-// Prints "blocks inside, of them with a corner below a millimetre, voxels outside"; with an argument the
-// bound on the corners' depth is left out.
+// Prints "blocks inside, of them with a corner below a millimetre, voxels outside"; with the argument "without" the
+// bound on the corners' depth is left out, with "columns" the corners are the ends of the voxels' columns, summed as voxels
+// are, as for a single frame (block_place_one).
 #include <cinttypes>
 #include <cmath>
 #include <cstdio>
@@ -21,7 +22,8 @@ static int32_t bits(float x) {
   return b;
 }
 
-int main(int argc, char**) {
+int main(int argc, char** argv) {
+  const bool without = argc > 1 && !std::strcmp(argv[1], "without"), columns = argc > 1 && !std::strcmp(argv[1], "columns");
   std::mt19937_64 rng(7);
   std::uniform_real_distribution<double> uni(0.0, 1.0);
   int64_t inside = 0, near = 0, out = 0;
@@ -68,7 +70,7 @@ int main(int argc, char**) {
     float cb[3], hb[3];
     block_origin_cam(T, vox, b[0], b[1], b[2], cb);
     to_pixel_h(K, cb, hb);
-    const float need = argc > 1 ? 0.0f : near_depth(near_steps(h, near_image(W, H)), hb, near_image(W, H));
+    const float need = without ? 0.0f : near_depth(near_steps(h, near_image(W, H)), hb, near_image(W, H));
     bool zin = true;
     int32_t lu = INT32_MAX, hu = INT32_MIN, lv = INT32_MAX, hv = INT32_MIN;
     float zmin = INFINITY;
@@ -76,11 +78,16 @@ int main(int argc, char**) {
       const float c0 = (c & 1) ? 7.0f : 0.0f, c1 = (c & 2) ? 7.0f : 0.0f, c2 = (c & 4) ? 7.0f : 0.0f;
       float off[3];
       for (int r = 0; r < 3; ++r) off[r] = std::fma(c0, h.ax[r], std::fma(c1, h.ay[r], c2 * h.az[r]));
-      const float z = hb[2] + off[2];
+      float P[3];
+      for (int r = 0; r < 3; ++r) {
+        const float col = hb[r] + std::fma(c1, h.ay[r], c2 * h.az[r]);
+        P[r] = !columns ? hb[r] + off[r] : c0 > 0.0f ? std::fma(c0, h.ax[r], col) : col;
+      }
+      const float z = P[2];
       float iz = 1.0f / z;
       const int ulp = (int)(rng() % 3);
       if (ulp) iz = std::nextafter(iz, ulp == 1 ? INFINITY : -INFINITY);
-      const float u = (hb[0] + off[0]) * iz, v = (hb[1] + off[1]) * iz;
+      const float u = P[0] * iz, v = P[1] * iz;
       zin = zin && z >= need && z >= 0x1p-60f && z <= 0x1p60f;
       zmin = std::fmin(zmin, z);
       lu = std::min(lu, bits((u - 0.5f) + kPixMagic));

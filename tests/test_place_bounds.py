@@ -17,8 +17,9 @@ def test_corners_bound_the_voxels(tmp_path):
     exe = str(tmp_path / "place_bounds")
     subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-I", os.path.join(ROOT, "voxel-hashing-sdf_amd", "csrc"),
                     "-I", os.path.join(ROOT, "include"), "-o", exe, src], check=True, timeout=120)
-    inside, near, out = map(int, subprocess.run([exe], capture_output=True, text=True, timeout=120, check=True).stdout.split())
-    assert inside > 20_000 and near > 1_000 and out == 0
+    for corners in ([], ["columns"]):
+        inside, near, out = map(int, subprocess.run([exe] + corners, capture_output=True, text=True, timeout=120, check=True).stdout.split())
+        assert inside > 20_000 and near > 1_000 and out == 0
     assert int(subprocess.run([exe, "without"], capture_output=True, text=True, timeout=120, check=True).stdout.split()[2]) > 0
 
 

@@ -256,10 +256,14 @@ __device__ __forceinline__ bool set_insert(AllocLds<kBands>& L, unsigned long lo
 // x of another lane of the row of 16 (DPP control kCtrl).
 template <int kCtrl>
 __device__ __forceinline__ int32_t dpp(int32_t x) { return __builtin_amdgcn_mov_dpp(x, kCtrl, 0xf, 0xf, false); }
-// Windows of a wave's pixels in a single frame's launch; the lanes left then walk. A frame of
-// 47,000 blocks at 4 mm, far and noisy: 16.6 us with no limit, 15.3 with 2; one of 15,000 at 5 mm:
-// 9.8 and 10.7. A batch's launch, with four bands per workgroup, is 1 to 3 % slower with a limit.
-constexpr int kMaxWindows = 3;
+// Windows of a wave's pixels in a single frame's launch; the lanes left then walk. Near surfaces are done
+// with one or two windows, far and noisy ones would need many of few lanes each, where a walk is
+// the faster. Launch times in us with at most 0 / 1 / 2 / 3 / any number of windows: a small room at 1 cm 9.5 / 8.2 / 8.3 /
+// 8.3 / 8.3, a room at 5 mm 9.4 / 10.0 / 9.9 / 9.7 / 9.6, at 4 mm 9.3 / 10.3 / 10.5 / 10.3 / 9.9, a floor at 4 mm 9.8 / 11.4 /
+// 12.6 / 13.5 / 15.3, tracked 14.4 / 14.8 / 15.1 / 15.7 / 17.2; and a frame of the small room with its
+// integration, one by one, 19.1 with 0, 19.4 with 1, 18.6 with 2 or 3. A batch's launch, with four bands per workgroup, is 1 to 3 %
+// slower with a limit.
+constexpr int kMaxWindows = 2;
 
 // OR of x over the wave's lanes (in every lane's result; DPP within rows of 16, then the rows').
 __device__ __forceinline__ uint32_t wave_or(uint32_t x) {
@@ -577,6 +581,53 @@ __device__ __forceinline__ Placement block_place(const FrameArgs& a, const float
   return p;
 }
 
+// Smallest and largest of x over lanes 0, 7, 56 and 63: the half-row mirror pairs lane 0 with 7 and 56
+// with 63, then two reads.
+__device__ __forceinline__ int32_t ends_min(int32_t x) {
+  x = min(x, dpp<0x141>(x));
+  return min(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 56));
+}
+__device__ __forceinline__ int32_t ends_max(int32_t x) {
+  x = max(x, dpp<0x141>(x));
+  return max(__builtin_amdgcn_readlane(x, 0), __builtin_amdgcn_readlane(x, 56));
+}
+
+// block_place for the launch of a single frame: the lane's column of voxels runs from cl to cl + 7 ax,
+// and the columns of lanes 0, 7, 56 and 63 end at the block's 8 corners. hb: the homogeneous block origin.
+// By lane groups, as in block_place, a single frame's block is placed eight times over and read back with
+// readlane. Per frame, by lane groups / in this form: 640 x 480 into a far floor at 4 mm, binary16 43.1 / 42.0 us,
+// FP32 32.4 / 31.9; into a room at 5 mm, binary16 23.7 / 22.7; at 4 mm, F16R 37.1 / 34.7.
+__device__ __forceinline__ int block_place_one(const FrameArgs& a, const float ax[3], const float cl[3], const float hb[3],
+                                               float steps, DepthWindow& w) {
+  const float near = near_depth(steps, hb, a.near);
+  bool zin = true;
+  float u[2], v[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {
+    const float z = e ? __builtin_fmaf(7.0f, ax[2], cl[2]) : cl[2];
+    const float iz = recip_rn(z);
+    u[e] = (e ? __builtin_fmaf(7.0f, ax[0], cl[0]) : cl[0]) * iz;
+    v[e] = (e ? __builtin_fmaf(7.0f, ax[1], cl[1]) : cl[1]) * iz;
+    zin = zin & (z >= near) & (z >= 0x1p-60f) & (z <= 0x1p60f);
+  }
+  const int32_t lu = ends_min((int32_t)__float_as_uint((fminf(u[0], u[1]) - 0.5f) + kPixMagic));
+  const int32_t hu = ends_max((int32_t)__float_as_uint((fmaxf(u[0], u[1]) + 0.5f) + kPixMagic));
+  const int32_t lv = ends_min((int32_t)__float_as_uint((fminf(v[0], v[1]) - 0.5f) + kPixMagic));
+  const int32_t hv = ends_max((int32_t)__float_as_uint((fmaxf(v[0], v[1]) + 0.5f) + kPixMagic));
+  const int32_t mb = (int32_t)kPixMagicBits, la = lu & ~3;
+  const uint32_t cols = (uint32_t)(hu - la) + 1u, rows = (uint32_t)(hv - lv) + 1u;
+  const uint32_t shift = 32u - (uint32_t)__builtin_clz(min(cols - 1u, 63u) | 3u);
+  w.first = 4u * (((uint32_t)lv - kPixMagicBits) * (uint32_t)a.pitch + ((uint32_t)la - kPixMagicBits));
+  w.shift = shift;
+  w.rows = rows;
+  w.cols = cols;
+  w.bias = ((uint32_t)lv << (shift + 2u)) + ((uint32_t)la << 2);
+  const bool inside = __builtin_amdgcn_ballot_w64(!zin) == 0 && lu >= mb && hu <= mb + a.W - 1 && lv >= mb &&
+                      hv <= mb + a.H - 1;
+  const bool fits = cols <= 64u && rows <= (kWin >> shift);
+  return inside ? (fits ? kPlaceWindow : kPlaceInside) : kPlaceEdge;
+}
+
 // LDS addresses as integers: the byte address of an LDS location, and a read from one.
 typedef __attribute__((address_space(3))) float LdsFloat;
 __device__ __forceinline__ uint32_t lds_address(const float* p) { return (uint32_t)(size_t)(const LdsFloat*)p; }
@@ -771,7 +822,8 @@ struct __align__(16) ColumnLds {
 // my_off, n: lane s holds the exclusive offset of the list's stripe s; the list's length. s_frm,
 // s_col: the batch's k frames; rcp_tab: RN(1/w) for w < kRcpTab with 0 at w = 0 (read when
 // kTab); s_win: the LDS byte address of the wave's depth window (kWin pixels). kBatch: a launch of
-// several frames (k > 1).
+// several frames (k > 1), whose blocks are placed in all of them at once (block_place); a single
+// frame's are placed by block_place_one, with no s_col.
 template <int kStorage, bool kColor, bool kTab, bool kBatch>
 __device__ void integrate_worker(const FrameArgs& a, uint32_t worker, uint32_t workers, uint32_t my_off, uint32_t n,
                                  uint32_t f0, uint32_t k, uint32_t parity, unsigned long long* s_val,
@@ -787,17 +839,16 @@ __device__ void integrate_worker(const FrameArgs& a, uint32_t worker, uint32_t w
   const size_t frame_px = (size_t)a.pitch * a.H;
   const uint32_t t_cap = a.cap < (float)kRcpTab ? 4u * (uint32_t)a.cap : ~0u;
 
-  // lanes 8 j .. 8 j + 7: the 8 corners of a block in frame j of the batch (a single frame: all
-  // groups the same), as homogeneous offsets from its origin
+  // lanes 8 j .. 8 j + 7: the 8 corners of a block in frame j of the batch, as homogeneous
+  // offsets from its origin
   const uint32_t jl = kBatch ? min((uint32_t)lane >> 3, k - 1u) : 0u;
   float corner[3];
-  {
+  if constexpr (kBatch) {
     const float c0 = (lane & 1) ? 7.0f : 0.0f, c1 = (lane & 2) ? 7.0f : 0.0f, c2 = (lane & 4) ? 7.0f : 0.0f;
 #pragma unroll
     for (int r = 0; r < 3; ++r)
       corner[r] = __builtin_fmaf(c0, s_frm[jl].ax[r], __builtin_fmaf(c1, s_frm[jl].ay[r], c2 * s_frm[jl].az[r]));
   }
-
 
   // Lane j fetches the list entry, slot value, key and mark of this worker's j-th block
   // (clearing the mark for the next batch of this parity) and parks them in LDS, so the
@@ -855,24 +906,50 @@ __device__ void integrate_worker(const FrameArgs& a, uint32_t worker, uint32_t w
 #pragma unroll
           for (int q = 0; q < 8; ++q) cold[q] = fresh ? 0u : cp[lane + 64 * q];
         }
-        // the block's placement in every frame of the batch, while its voxels are on their way
-        // (lane group j holds frame j's; the frame loop takes it with readlane)
+        // the block's origin (kBatch: its placement too, lane group j holding frame j's for the frame loop to
+        // take with readlane), while its voxels are on their way
         float hb[3];
-        Placement pl;
         {
           float T[12], cb[3];
 #pragma unroll
           for (int q = 0; q < 12; ++q) T[q] = s_frm[jl].T[q];
           block_origin_cam(T, a.vox, bx, by, bz, cb);
           to_pixel_h(a.K, cb, hb);
-          pl = block_place(a, hb, corner, s_frm[jl].ax[3]);
         }
+        Placement pl{};
+        if constexpr (kBatch) pl = block_place(a, hb, corner, s_frm[jl].ax[3]);
 #pragma unroll
         for (int q = 0; q < 8; ++q) vx.load(q, old[q]);
         uint32_t upd = 0u;  // colour volumes: bit q set when voxel q was observed in the batch
-        for (uint32_t m = mark; m != 0u; m &= m - 1u) {
+        if constexpr (!kBatch) {
+          if (mark) {
+            const FrameLds& F = s_frm[0];
+            float ax[3], cl[3];
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+              ax[r] = F.ax[r];
+              cl[r] = hb[r] + __builtin_fmaf((float)(lane >> 3), F.ay[r], (float)(lane & 7) * F.az[r]);
+            }
+            const size_t fo = (size_t)parity * kMaxBatch * frame_px;
+            const uint32_t* rgba = kColor ? a.rgba + fo : nullptr;
+            const float* dmf = a.dm + fo;
+            DepthWindow win;
+            const int place = block_place_one(a, ax, cl, hb, F.ax[3], win);
+            // the update once per placement: its variants' registers don't join before another frame's
+            if (place == kPlaceWindow) {
+              stage_window(a, dmf, win, s_win);
+              frame_update<kStorage, kColor, kTab, kReg>(a, kPlaceWindow, ax, cl, dmf, rgba, win.shift, s_win - win.bias, t_cap, vx,
+                                                         cold, upd, rcp_tab);
+            } else if (place == kPlaceInside) {
+              frame_update<kStorage, kColor, kTab, kReg>(a, kPlaceInside, ax, cl, dmf, rgba, 0u, 0u, t_cap, vx, cold, upd, rcp_tab);
+            } else {
+              frame_update<kStorage, kColor, kTab, kReg>(a, kPlaceEdge, ax, cl, dmf, rgba, 0u, 0u, t_cap, vx, cold, upd, rcp_tab);
+            }
+          }
+        }
+        for (uint32_t m = kBatch ? mark : 0u; m != 0u; m &= m - 1u) {
           const uint32_t jf = (uint32_t)__builtin_ctz(m);
-          const int src = kBatch ? 8 * (int)jf : 0;
+          const int src = 8 * (int)jf;
           float ax[3], cl[3];
 #pragma unroll
           for (int r = 0; r < 3; ++r) {
@@ -987,9 +1064,11 @@ constexpr int kIntegrateWaves = 4;  // independent workers per workgroup
 // Register budget of the integration kernels: depth only, 6 waves per SIMD (80 VGPRs, at most one
 // value spills; 500 frames of a room at 5 mm in batches of 8, FP32: 6.22 ms at 5 waves, 5.94 at 6,
 // with the fused launch's 4,096 workers; before the values and weights of a block stayed in
-// registers in the form the update takes them, 6 waves spilled into the frame loop); colour, 4
+// registers in the form the update takes them, 6 waves spilled into the frame loop); a single frame's
+// launch 5, all its workers at once (FP32 needs 84 VGPRs; at 6 waves four values spill: a room at
+// 4 mm 33.0 us, at 5 waves 31.9); colour, 4
 // waves (128 VGPRs: at 96 about 50 values spill into the frame loop, 13 % slower).
-#define VH_INTEGRATE_OCCUPANCY __attribute__((amdgpu_waves_per_eu(kColor ? 4 : 6)))
+#define VH_INTEGRATE_OCCUPANCY(kBatch) __attribute__((amdgpu_waves_per_eu(kColor ? 4 : kBatch ? 6 : 5)))
 
 // Entry q of the pose of the batch's frame j (kBatch: of a bound sequence).
 template <bool kBatch>
@@ -1011,7 +1090,9 @@ __device__ __forceinline__ void stage_poses(const FrameArgs& a, uint32_t cur, ui
 // The poses, homogeneous steps and column offsets of a batch's frames into LDS, and the
 // reciprocal table. pose: the t-th of the batch's 12 k pose entries in lane t. All 256 lanes call
 // it. Each wave forms the steps of the frames whose columns it fills (the same values in every
-// lane), so that one barrier separates the poses from everything made of them.
+// lane), so that one barrier separates the poses from everything made of them. A single frame (not
+// kBatch) has no columns.
+template <bool kBatch>
 __device__ __forceinline__ void stage_frames(const FrameArgs& a, float pose, uint32_t k, FrameLds* s_frm,
                                              ColumnLds* s_col, float* rcp_tab, bool tab) {
   const uint32_t t = threadIdx.x;
@@ -1037,7 +1118,7 @@ __device__ __forceinline__ void stage_frames(const FrameArgs& a, float pose, uin
         s_frm[j].az[r] = h.az[r];
         if (r == 0) s_frm[j].ax[3] = near_steps(h, a.near);
       }
-      s_col[j].off[lane][r] = __builtin_fmaf((float)(lane >> 3), h.ay[r], (float)(lane & 7u) * h.az[r]);
+      if constexpr (kBatch) s_col[j].off[lane][r] = __builtin_fmaf((float)(lane >> 3), h.ay[r], (float)(lane & 7u) * h.az[r]);
     }
   }
   __syncthreads();
@@ -1051,27 +1132,25 @@ __device__ __forceinline__ bool rcp_table_covers(const FrameArgs& a, const Frame
 }
 
 // The integration's LDS: per wave the staged list entries, slot values, keys and marks and
-// the depth window; per workgroup the batch's frames and the reciprocal table. kFrames: 1 or
-// kMaxBatch (27 KB, 5 workgroups per CU).
-template <int kFrames>
+// the depth window; per workgroup the batch's frames and the reciprocal table (kBatch: 26,368 bytes, 6
+// workgroups per CU, as many as its registers allow; a single frame: 17,504).
+template <bool kBatch>
 struct IntegrateLds {
   float rcp[kRcpTab];
-  FrameLds frm[kFrames];
-  ColumnLds col[kFrames];
+  FrameLds frm[kBatch ? kMaxBatch : 1];
+  ColumnLds col[kBatch ? kMaxBatch : 0];
   float win[kIntegrateWaves][kWin];
   unsigned long long val[kIntegrateWaves][64], key[kIntegrateWaves][64];
   uint32_t mark[kIntegrateWaves][64];
 };
-template <bool kBatch>
-using IntegrateLdsOf = IntegrateLds<kBatch ? kMaxBatch : 1>;
-static_assert(offsetof(IntegrateLds<1>, win) % 16 == 0 && offsetof(IntegrateLds<kMaxBatch>, win) % 16 == 0,
+static_assert(offsetof(IntegrateLds<false>, win) % 16 == 0 && offsetof(IntegrateLds<true>, win) % 16 == 0,
               "stage_window writes 16 bytes per lane");
 
 // The workgroup's share of the batch of k frames (first frame f0, list parity, first input
 // cur). All 256 lanes call it.
 template <int kStorage, bool kColor, bool kBatch>
 __device__ __forceinline__ void integrate_group(const FrameArgs& a, uint32_t group, uint32_t groups, uint32_t f0,
-                                                uint32_t k, uint32_t parity, uint32_t cur, IntegrateLdsOf<kBatch>& L) {
+                                                uint32_t k, uint32_t parity, uint32_t cur, IntegrateLds<kBatch>& L) {
   const uint32_t t = threadIdx.x, lane = t & 63u;
   const int wave = t >> 6;
   // the pose entries and the list's lengths, in flight together
@@ -1092,7 +1171,7 @@ __device__ __forceinline__ void integrate_group(const FrameArgs& a, uint32_t gro
   const uint32_t my_off = incl - my_len, n = read_lane_u32(incl, 63);
   const uint32_t worker = group * kIntegrateWaves + wave, workers = groups * kIntegrateWaves;
   if (group * kIntegrateWaves >= n) return;  // a short list: no block for this workgroup
-  stage_frames(a, pose, k, L.frm, L.col, L.rcp, tab);
+  stage_frames<kBatch>(a, pose, k, L.frm, L.col, L.rcp, tab);
   const uint32_t win = uniform(lds_address(L.win[wave]));
   if (tab)
     integrate_worker<kStorage, kColor, true, kBatch>(a, worker, workers, my_off, n, f0, k, parity, L.val[wave],
@@ -1104,8 +1183,8 @@ __device__ __forceinline__ void integrate_group(const FrameArgs& a, uint32_t gro
 
 // Integration of the batch of k frames that the last allocation launch prepared (kBatch: k > 1).
 template <int kStorage, bool kColor, bool kBatch>
-__global__ __launch_bounds__(64 * kIntegrateWaves) VH_INTEGRATE_OCCUPANCY void k_integrate(FrameArgs a, uint32_t k) {
-  __shared__ IntegrateLdsOf<kBatch> L;
+__global__ __launch_bounds__(64 * kIntegrateWaves) VH_INTEGRATE_OCCUPANCY(kBatch) void k_integrate(FrameArgs a, uint32_t k) {
+  __shared__ IntegrateLds<kBatch> L;
   const FrameCtl* ctl = a.ctl;
   // control values are uniform: keep them (and what derives from them) in scalar registers
   const uint32_t f0 = uniform(ctl->frame_id), parity = uniform(ctl->batch_id) & 1u,
@@ -1121,13 +1200,13 @@ __global__ __launch_bounds__(64 * kIntegrateWaves) VH_INTEGRATE_OCCUPANCY void k
 // b, so the frame id, cursor and batch id the allocation workgroups read at their start
 // cannot advance under them.
 template <int kStorage, bool kU16, bool kColor>
-__global__ __launch_bounds__(64 * kIntegrateWaves) VH_INTEGRATE_OCCUPANCY void k_integrate_alloc(FrameArgs a, uint32_t int_groups,
+__global__ __launch_bounds__(64 * kIntegrateWaves) VH_INTEGRATE_OCCUPANCY(true) void k_integrate_alloc(FrameArgs a, uint32_t int_groups,
                                                                          uint32_t alloc_groups, uint32_t tiles,
                                                                          uint32_t k_int) {
   // a workgroup either allocates or integrates: the two share the LDS
   __shared__ union {
     AllocLds<kAllocBands> alloc;
-    IntegrateLdsOf<true> integ;
+    IntegrateLds<true> integ;
   } L;
   const uint32_t b = blockIdx.x;
   const bool alloc = b >= int_groups;
