@@ -1,6 +1,6 @@
 """Allocation against the oracle over the forms its tile pass takes: bands of a fraction of a block to
-several blocks (one key, closed form, walk in the window, walk block by block), tile keys relative
-to the camera and packed ones (small voxels, scaled poses), poses at and far from the origin and
+several blocks (one key, closed form, walk in the window, walk block by block), keys of small and
+large block coordinates (small voxels, scaled poses), poses at and far from the origin and
 on block faces, single frames and batches, images of partial tiles. Bar: per-frame touched counts,
 allocated sets and voxels identical (no tolerance)."""
 import numpy as np
@@ -73,7 +73,7 @@ def test_band_lengths(vh, oracle, trunc_voxels, size):
     (0.02, (0.0, 0.0, 0.0), 1.0),          # the camera on a block corner
     (0.02, (0.16 * 7, -0.16 * 3, 0.0), 1.0),  # and on others
     (0.02, (2000.0, -1500.0, 900.0), 1.0),  # coarse coordinates
-    (0.0011, (0.2, 0.1, -0.3), 1.0),       # bands beyond the near keys' reach
+    (0.0011, (0.2, 0.1, -0.3), 1.0),       # block coordinates in the hundreds
     (0.02, (0.3, 0.2, 0.1), 3.0),          # rows longer than a rotation's
 ])
 def test_keys_and_poses(vh, oracle, vox, shift, scale):

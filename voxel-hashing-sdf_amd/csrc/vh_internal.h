@@ -404,9 +404,5 @@ hipError_t launch_gn_solve(const double* partials, int grid, const GnState* st_i
                            double* stats_row, hipStream_t st);
 hipError_t launch_track_solve(const double* partials, int grid, const GnState* st_in, GnState* st_out, double* cand,
                               const TrackArgs& t, hipStream_t st);
-// cand = s.pose, solver state cleared with damping s.lambda.
-// Gauss-Newton state reset + prior pose of the current frame, and the depth back-projection,
-// in one launch.
-// Accepted pose (and the frame's solver stats) to the per-frame outputs.
 
 }  // namespace vh

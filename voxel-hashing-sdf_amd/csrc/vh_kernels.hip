@@ -2375,9 +2375,12 @@ __global__ __launch_bounds__(256) void k_st_place(StreamArgs a) {
 }
 
 // ============================================================================ queries
-// q = a / b, correctly rounded, from y = RN(1 / b): q0 = RN(a y) is within an ulp, a - q0 b is exact
-// under FMA, and RN(q0 + (a - q0 b) y) is the quotient (Markstein): 3
-// operations instead of the division's 11.
+// a / b from y = RN(1 / b): q0 = RN(a y) is within 1.5 ulp, and RN(q0 + (a - q0 b) y), Markstein's
+// correction, takes 3 operations instead of the division's 11. Correctly rounded where b has 24
+// significant bits, as the voxel size has: a - q0 b then has 25 and is exact under FMA, the corrected sum is
+// off by 1.5 ulp 2^-53 at most, and a / b is no midpoint of two doubles nor within 2^-25 ulp of one. For a divisor of 53 bits (gn_step's
+// pivots) a - q0 b may round, and only a quotient within some 2^-50 ulp of a midpoint can come out as its neighbour. No
+// subnormal quotients.
 __device__ __forceinline__ double quotient(double a, double b, double y) {
   const double q0 = a * y;
   return __builtin_fma(__builtin_fma(-q0, b, a), y, q0);
@@ -3334,8 +3337,6 @@ static void with_storage(int storage, F f) {
     default: f(std::integral_constant<int, VH_STORAGE_F32>()); break;
   }
 }
-
-// Calls f(std::integral_constant<bool, u16>(), std::integral_constant<bool, colour>()).
 
 hipError_t launch_integrate(const FrameArgs& a, int storage, int grid, int k, hipStream_t st) {
   with_storage(storage, [&](auto S) {
