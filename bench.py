@@ -525,7 +525,7 @@ def main():
     if "pcie" in results:
         out["host_input_fps"] = {"value": round(results.pop("pcie"), 2), "unit": "frames/s",
                                  "note": "the same 500 frames from page-locked host memory: vh_integrate_async per frame "
-                                         "(uint16 depth copied over PCIe into a 4-slot device ring on a second stream, "
+                                         "(uint16 depth read over PCIe by a kernel into one of 4 device slots, "
                                          "then allocation + integration), no marching cubes"}
     if "gn" in results:
         out["gn"] = results.pop("gn")

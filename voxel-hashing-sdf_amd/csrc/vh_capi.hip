@@ -1124,15 +1124,16 @@ const void* host_image(const void* src, size_t row, size_t pitch, size_t rows, c
 
 // Images of a frame up to here are read by a kernel in the frame's own stream (k_copy_in), larger ones
 // copied by the runtime: for a frame that the call waits for in that stream too, for a queued frame on the
-// copy stream, where the copy overlaps the kernels of the frame before. Queued, the overlap costs waits
-// between the streams, the kernel its time on the bus: a frame into a room at 5 mm (binary16; us by the copy
-// stream / by the kernel) 150 KB 36 / 31, 600 KB 37 / 40, 938 KB 40 / 48, 1.2 MB 41 / 52, 1.5 MB 49 / 65.
-// With three volumes in use, whose six streams share four hardware queues, 600 KB 43 to 62 / 41, 938 KB 50 to 70 /
-// 48, 1.2 MB 44 to 63 / 52: so the kernel up to 1 MB, where it is also no slower than the copy
-// stream with a graph of the frame's kernels was (48). Waited for, the kernel is the faster at every size (640 x 480 float
-// 62 us, 64 by a copy; 1280 x 960 137 and 141); 1.6 MB leaves the bus to the copy engine above.
+// copy stream, where the copy overlaps the kernels of the frame before. Queued, the kernel costs its time on the bus
+// (57 GB/s). The overlap costs waits between the streams: little while the host is the slower side, some 35 us a frame once
+// the kernels are and each wait really waits. A frame of 1.2 MB into a room at 6 mm, FP32: 44 us by the copy stream
+// and 56 by the kernel in a view of few blocks, 79 and 64 in one of many; 32 of them on three volumes in turn
+// 2,530 and 1,950; binary16 42 and 51. 1.5 MB (1024 x 768 uint16): 53 and 71, 60 and 78. So the kernel up to 1.25 MB; with a graph of
+// a frame's kernels behind each copy on the copy stream, as before, those frames took 54 and 82, 57, 60 and 66. Waited for, the
+// kernel is the faster at every size (640 x 480 float 62 us, 64 by a copy; 1280 x 960 137 and 141); 1.6 MB leaves the bus to
+// the copy engine above.
 constexpr size_t kDirectBytes = 1600 * 1024;
-constexpr size_t kDirectQueuedBytes = 1024 * 1024;
+constexpr size_t kDirectQueuedBytes = 1280 * 1024;
 
 // An image to the device: `from`, its contiguous page-locked bytes (read by a kernel if direct), or where that
 // is null the caller's rows.

@@ -115,7 +115,7 @@ __global__ __launch_bounds__(256) void k_words_out(uint32_t* dst, const uint32_t
 // frame's bit clear count the block for that frame.
 // What bounds it: vector issue (about 270 instructions per wave and band) with the latency of the
 // set and of phase 2's four dependent round trips between. 8 frames of 640 x 480 launched alone:
-// 5 mm 43.3 -> 31.5 us, 1 cm 38.2 -> 28.0 us against a walk per lane with a compare-and-swap per key
+// 5 mm 42.6 -> 32.3 us, 1 cm 37.9 -> 28.1 us against a walk per lane with a compare-and-swap per key
 // (a launch without the bands takes 7.7 us, without the set 22.6).
 constexpr int kSetSlots = 1024;  // LDS key set (8 KB)
 // 16 x 16 bands per tile of a batched launch. One workgroup per four bands pays the LDS clear,
