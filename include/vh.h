@@ -201,8 +201,9 @@ int vh_abi_version(void);
 int vh_integrate(vh_volume* vol, const vh_frame* frame);
 /* Asynchronous variant of vh_integrate (no reference counterpart; processFrame blocks,
  * src/tsdf.cu:1495-1497): the depth (and RGB) goes into one of 4 device slots, read by a kernel
- * on the volume's stream (images of up to 1.25 MB a frame) or copied on a second stream while
- * earlier frames integrate, and the frame's allocation and integration follow it. The call
+ * on the volume's stream (images of up to 640 KB a frame, pageable ones up to 1.6 MB) or copied
+ * on a second stream while earlier frames integrate, and the frame's allocation and integration
+ * follow it. The call
  * returns after queuing; the buffers must stay unchanged until vh_sync (page-locked memory, e.g.
  * from hipHostMalloc, is read where it lies; pageable memory is first copied into page-locked
  * memory of the volume, before the call returns). Overflows are reported by vh_sync. */

@@ -1125,15 +1125,17 @@ const void* host_image(const void* src, size_t row, size_t pitch, size_t rows, c
 // Images of a frame up to here are read by a kernel in the frame's own stream (k_copy_in), larger ones
 // copied by the runtime: for a frame that the call waits for in that stream too, for a queued frame on the
 // copy stream, where the copy overlaps the kernels of the frame before. Queued, the kernel costs its time on the bus
-// (57 GB/s). The overlap costs waits between the streams: little while the host is the slower side, some 35 us a frame once
-// the kernels are and each wait really waits. A frame of 1.2 MB into a room at 6 mm, FP32: 44 us by the copy stream
-// and 56 by the kernel in a view of few blocks, 79 and 64 in one of many; 32 of them on three volumes in turn
-// 2,530 and 1,950; binary16 42 and 51. 1.5 MB (1024 x 768 uint16): 53 and 71, 60 and 78. So the kernel up to 1.25 MB; with a graph of
-// a frame's kernels behind each copy on the copy stream, as before, those frames took 54 and 82, 57, 60 and 66. Waited for, the
+// (57 GB/s) in front of the frame's own, the copy stream two waits between streams. By the kernel / by the copy stream (and with
+// a graph of the frame's kernels behind each copy, as before), us a frame into a small room at 1 cm, a room at 6 mm, a floor at
+// 5 mm, FP32: 640 x 480 float (1.2 MB) 43 / 42 (47), 61 / 49 (56), 77 / 64 (71); 511 x 383 float (783 KB) 37 / 33 (46), 55 / 47 (53),
+// 68 / 60 (65); 640 x 480 uint16 (614 KB) 32 / 34 (46), 50 / 48 (55), three volumes in turn 20 / 29 and 31 / 32; 320 x 240 float
+// (307 KB) 24 / 33 (46), 42 / 45 (51). So the kernel up to 640 KB. A pageable image is copied by the host first, which is then the
+// slower side, and a copy costs it more than a launch: 640 x 480 float 65 / 73, 848 x 480 float (1.6 MB) 70 / 83, so up to the
+// limit of frames that are waited for (511 x 383 float 58 / 55; thousands before). Waited for, the
 // kernel is the faster at every size (640 x 480 float 62 us, 64 by a copy; 1280 x 960 137 and 141); 1.6 MB leaves the bus to
 // the copy engine above.
 constexpr size_t kDirectBytes = 1600 * 1024;
-constexpr size_t kDirectQueuedBytes = 1280 * 1024;
+constexpr size_t kDirectQueuedBytes = 640 * 1024;
 
 // An image to the device: `from`, its contiguous page-locked bytes (read by a kernel if direct), or where that
 // is null the caller's rows.
@@ -1331,21 +1333,21 @@ int vh_integrate_async(vh_volume* v, const vh_frame* f) {
   const int slot = (int)(v->ring_next % R);
   const size_t rows = (size_t)v->cfg.height, slot_bytes = (frame_px * (v->colors ? 7 : 4) + 7) & ~(size_t)7;
   const size_t line = (size_t)v->cfg.width * 3;
-  const bool direct = rows * (row + (v->colors ? line : 0)) <= kDirectQueuedBytes;
-  const hipStream_t copies = direct ? v->stream : v->copy_stream;
   if (v->ring_held[slot]) VH_HIP(hipEventSynchronize(v->ring_copied[slot]));
+  const void* depth = host_image(f->depth, row, pitch, rows, &v->ring_host, R * slot_bytes, slot * slot_bytes);
+  const void* rgb = nullptr;
+  if (v->colors) rgb = host_image(f->rgb, line, line, rows, &v->ring_host, R * slot_bytes, slot * slot_bytes + frame_px * 4);
+  const size_t limit = depth && depth != f->depth ? kDirectBytes : kDirectQueuedBytes;
+  const bool direct = rows * (row + (v->colors ? line : 0)) <= limit;
+  const hipStream_t copies = direct ? v->stream : v->copy_stream;
   if (!direct) {  // the copy waits for the frame that read the slot
     if (!v->ring_marked[slot]) VH_HIP(hipEventRecord(v->ring_done[slot], v->stream));
     VH_HIP(hipStreamWaitEvent(v->copy_stream, v->ring_done[slot], 0));
   }
   char* dst = static_cast<char*>(v->ring_depth) + (size_t)slot * v->cfg.width * v->cfg.height * elem;
-  const void* depth = host_image(f->depth, row, pitch, rows, &v->ring_host, R * slot_bytes, slot * slot_bytes);
   VH_HIP(copy_image(dst, depth, f->depth, row, pitch, rows, direct, copies));
-  const void* rgb = nullptr;
-  if (v->colors) {
-    rgb = host_image(f->rgb, line, line, rows, &v->ring_host, R * slot_bytes, slot * slot_bytes + frame_px * 4);
+  if (v->colors)
     VH_HIP(copy_image(v->ring_rgb + (size_t)slot * frame_px * 3, rgb, f->rgb, line, line, rows, direct, copies));
-  }
   // the volume's own page-locked bytes are written again only after the copy; a caller's are the caller's
   v->ring_held[slot] = !direct || (depth && depth != f->depth) || (rgb && rgb != f->rgb);
   if (v->ring_held[slot]) VH_HIP(hipEventRecord(v->ring_copied[slot], copies));
