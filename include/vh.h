@@ -394,7 +394,9 @@ int vh_gn_refine_device_noalloc(vh_volume* vol, const float* d_pts, int64_t n, d
 /* Pool layout for callers that wrap the voxel memory (e.g. as a tensor): device pointer of
  * the voxel pool (pool_blocks*512 voxels; FP32: float2 {tsdf, weight}; FP16: uint32
  * {binary16 tsdf | uint16 weight << 16}; F16R: uint32 {binary16 tsdf | uint8 weight << 16 |
- * int8 residual << 24}) and of the block keys (pool_blocks packed keys). */
+ * int8 residual << 24}) and of the block keys (pool_blocks packed keys). Weights are counts of
+ * frames: a caller that writes voxels keeps them whole numbers, at most the frames integrated
+ * and the weight cap. */
 int vh_pool_view(vh_volume* vol, void** d_voxels, void** d_block_keys, int64_t* n_blocks);
 
 #ifdef __cplusplus
